@@ -122,6 +122,9 @@ struct FftPlans {
 };
 constexpr int kFftCache = 6;  // plan sets a context keeps (least recently used replaced)
 
+struct LinePlan;
+constexpr int kLineCache = 8;  // line lengths a context keeps tables for (least recently used replaced)
+
 }  // namespace pp
 
 struct pp_ctx {
@@ -142,7 +145,8 @@ struct pp_ctx {
     unsigned long long fft_clock = 0;
     // scratch
     pp::DevBuf d_field_a, d_field_b, d_k0, d_k1, d_k2, d_mask, d_misc, d_peaks, d_scan, d_cub;
-    pp::DevBuf d_in[8], d_pk, d_res, d_prof, d_queue, d_walk;
+    pp::DevBuf d_in[8], d_pk, d_res, d_prof, d_queue, d_walk, d_spec;
+    pp::LinePlan *line_cache = nullptr;  // [kLineCache]
     // persistent-form tunables (pp_autotune_shell): small-peak threshold in
     // finalised shells (several peaks per wave), shells per LDS chunk of the
     // wave gather, the shell count above which a peak's Float64 post runs on
@@ -166,5 +170,6 @@ int fft_prepare(pp_ctx *ctx, int n);                       // makes the n^3 out-
 int fft_plans(pp_ctx *ctx, int n, int kind, FftPlans **out);  // a cached set, without changing the current one
 void persist_release(pp_ctx *ctx);    // pp_persist.hip: drops the context's gather tables
 int noalloc_scratch_init(int device);  // pp_filter.hip: device address of the static scratch
+void line_release(pp_ctx *ctx);       // drops the line transforms' tables
 int ensure_device(pp_ctx *ctx);
 }  // namespace pp

@@ -6,6 +6,7 @@
 #include <cstring>
 
 #include "pp_common.h"
+#include "pp_fft.h"
 
 namespace pp {
 
@@ -142,6 +143,118 @@ int fft_plans(pp_ctx *ctx, int n, int kind, FftPlans **out)
     return PP_OK;
 }
 
+// ------------------------------------------------------- line transforms
+bool line_supported(int n)
+{
+    if (n < kLineMin || n > kLineMax) return false;
+    for (int p : {2, 3, 5, 7})
+        while (n % p == 0) n /= p;
+    return n == 1;
+}
+
+int line_plan(pp_ctx *ctx, int n, LineFft *out)
+{
+    PP_ARG(line_supported(n), "line length %d has no line transform", n);
+    if (!ctx->line_cache) ctx->line_cache = new LinePlan[kLineCache];
+    LinePlan *hit = nullptr, *victim = &ctx->line_cache[0];
+    for (int q = 0; q < kLineCache; q++) {
+        LinePlan &L = ctx->line_cache[q];
+        if (L.f.n == n) hit = &L;
+        if (L.last_use < victim->last_use) victim = &L;
+    }
+    if (!hit) {
+        // the streams may still run transforms with the tables being replaced
+        if (victim->f.n) {
+            PP_HIP(hipStreamSynchronize(ctx->stream));
+            PP_HIP(hipStreamSynchronize(ctx->side));
+        }
+        victim->f = LineFft{};
+        victim->last_use = 0;
+        LineFft f{};
+        f.n = n;
+        int rest = n, e2 = 0;
+        while (rest % 2 == 0) { rest /= 2; e2++; }
+        // powers of two as few stages as radix 8 and 4 give (8 8 2 -> 8 4 4)
+        std::vector<int> rad;
+        while (e2 > 0) {
+            const int take = e2 == 4 || e2 == 2 ? 2 : e2 >= 3 ? 3 : 1;
+            rad.push_back(1 << take);
+            e2 -= take;
+        }
+        for (int p : {3, 5, 7})
+            while (rest % p == 0) { rest /= p; rad.push_back(p); f.five |= p > 3; }
+        PP_ARG(rad.size() <= 8, "line length %d takes %zu stages", n, rad.size());
+        std::vector<float2> t;
+        auto root = [&](double num, double den) {  // exp(-i pi num / den)
+            const double a = M_PI * num / den;
+            t.push_back(make_float2((float)cos(a), (float)-sin(a)));
+        };
+        for (int k = 0; k < n; k++) root(k, n);
+        int ns = 1;
+        for (size_t q = 0; q < rad.size(); q++) {
+            const int R = rad[q];
+            f.rad[q] = R;
+            f.ns[q] = ns;
+            f.nr[q] = n / R;
+            f.lin[q] = f.nr[q] % 8 == 0 && (ns % 8 == 0 || (ns == 1 && 8 % R == 0));
+            f.magic[q] = (1u << 22) / (unsigned)ns + 1;
+            while (t.size() % 2) t.push_back(float2{});  // 16-byte aligned tables
+            f.two[q] = (int)t.size() - n;
+            if (q > 0)
+                for (int k = 0; k < ns; k++)
+                    for (int r = 0; r < R; r++) root(2.0 * k * r, (double)ns * R);
+            ns *= R;
+        }
+        f.nst = (int)rad.size();
+        PP_CHECK(victim->buf.grow(t.size() * sizeof(float2)));
+        PP_HIP(hipMemcpy(victim->buf.ptr, t.data(), t.size() * sizeof(float2), hipMemcpyHostToDevice));
+        f.half = victim->buf.as<float2>();
+        f.tw = f.half + n;
+        victim->f = f;
+        hit = victim;
+    }
+    hit->last_use = ++ctx->fft_clock;
+    *out = hit->f;
+    return PP_OK;
+}
+
+void line_release(pp_ctx *ctx)
+{
+    if (!ctx->line_cache) return;
+    for (int q = 0; q < kLineCache; q++) ctx->line_cache[q].buf.release();
+    delete[] ctx->line_cache;
+    ctx->line_cache = nullptr;
+}
+
+LineShape col_shape(LineFft &P, int max_block)
+{
+    // 16 columns (128-byte pieces of a row) where their threads fit the
+    // workgroup and the tile fits 64 KB, else 8
+    LineShape s{};
+    for (s.logl = 4; s.logl >= 3; s.logl--) {
+        const int step = 64 >> s.logl;  // whole wavefronts
+        P.tj = ((P.n + kLineEpt - 1) / kLineEpt + step - 1) / step * step;
+        s.nl = 1 << s.logl;
+        s.block = P.tj << s.logl;
+        s.lds = sizeof(float2) * ((size_t)P.n << s.logl);
+        if ((s.block <= max_block && s.lds <= 65536) || s.logl == 3) break;
+    }
+    return s;
+}
+
+LineShape row_shape(LineFft &P)
+{
+    // one wavefront where it holds whole lines (its barriers cost nothing),
+    // else the fewest lines that fill whole wavefronts
+    LineShape s{};
+    P.tj = ((P.n + kLineEpt - 1) / kLineEpt + 15) / 16 * 16;
+    s.nl = 1;
+    while (s.nl * P.tj % 64) s.nl++;
+    s.block = s.nl * P.tj;
+    s.lds = sizeof(float2) * (size_t)s.nl * row_pitch(P.n);
+    return s;
+}
+
 int fft_prepare(pp_ctx *ctx, int n)
 {
     FftPlans *F = nullptr;
@@ -223,6 +336,8 @@ int pp_ctx_destroy(pp_ctx *ctx)
                       &ctx->shells.d_akk, &ctx->shells.d_wrow, &ctx->shells.d_wtab,
                       &ctx->shells.d_shell_ge};
     for (DevBuf *b : bufs) b->release();
+    ctx->d_spec.release();
+    line_release(ctx);
     persist_release(ctx);
     for (auto &b : ctx->d_in) b.release();
     for (auto &e : ctx->ev)
@@ -289,7 +404,7 @@ int pp_ctx_release_scratch(pp_ctx *ctx)
     PP_HIP(hipStreamSynchronize(ctx->side));
     DevBuf *bufs[] = {&ctx->d_field_a, &ctx->d_field_b, &ctx->d_k0, &ctx->d_k1, &ctx->d_k2, &ctx->d_mask,
                       &ctx->d_misc, &ctx->d_peaks, &ctx->d_scan, &ctx->d_cub, &ctx->d_pk, &ctx->d_res,
-                      &ctx->d_prof, &ctx->d_queue, &ctx->d_walk};
+                      &ctx->d_prof, &ctx->d_queue, &ctx->d_walk, &ctx->d_spec};
     for (DevBuf *b : bufs) b->release();
     for (auto &b : ctx->d_in) b.release();
     return PP_OK;

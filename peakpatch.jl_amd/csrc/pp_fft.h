@@ -1,0 +1,363 @@
+// pp_fft.h -- single-precision line transforms in LDS, the building block of
+// the field kernels' three-dimensional transforms.
+//
+// A 3-D real transform here is three kinds of pass over a half spectrum
+// S[kz][ky][kx] (kx fastest): rows along x, columns along y, columns along z.
+// Every pass brings whole lines into LDS, transforms them there and lets the
+// kernel around it do its own arithmetic on the way in and out, so transfer
+// functions, several outputs of one input, the noise draw or a product of
+// fields in real space cost no pass over memory of their own.  Each pass is
+// bound by HBM: a line element is read and written once.
+//
+// * Columns: a workgroup takes 2^logl consecutive kx (a run of whole 64- or
+//   128-byte pieces in every row) of one (ky or kz) plane.  In LDS the line
+//   index is the fastest one, so the accesses of every stage are conflict
+//   free whatever the radix.
+// * Rows: two real rows travel as the real and imaginary part of one complex
+//   line; the half spectra of both are separated (or joined) on the fly.
+// * A line is transformed by Stockham stages of radix 8, 4, 2, 3, 5 and 7 (the
+//   radices are chosen at run time, so one kernel serves every length up to
+//   kLineMax with no larger prime factor).  A stage reads its inputs into
+//   registers, then writes them back in place, so one buffer is enough.
+//   Twiddles come from a table rounded from Float64, laid out as the
+//   butterflies read them.  Vector instructions are the second bound beside
+//   HBM (a radix-8 stage takes 14 per element, a pass has room for about a
+//   hundred), so addresses advance by scalar strides and the kernels' own
+//   factors are Float32 wherever their error stays below the transform's.
+#pragma once
+
+#include "pp_common.h"
+
+namespace pp {
+
+constexpr int kLineEpt = 8;    // line elements a thread holds
+constexpr int kLineMax = 1024; // longest line
+constexpr int kLineMin = 16;
+constexpr int kRowBins = 5;    // bins of a half spectrum a thread handles, >= (n / 2 + 1) / tj
+
+// One length's stages, passed to kernels by value.
+struct LineFft {
+    int n, nst;
+    int tj;                  // threads per line, >= n / kLineEpt
+    int five;                // a stage of radix 5 or 7
+    int rad[8], ns[8], nr[8], lin[8];  // radix, sub-length, butterflies; rows: constant strides
+    unsigned magic[8];       // floor(2^22 / ns) + 1: j / ns = j magic >> 22 for j < 2048
+    int two[8];              // a stage's twiddles exp(-2 pi i k r / (ns R)) at tw[two + k R + r]
+    const float2 *tw;
+    const float2 *half;      // exp(-pi i k / n), k < n
+};
+
+struct LinePlan {
+    LineFft f{};
+    unsigned long long last_use = 0;
+    DevBuf buf;
+};
+
+bool line_supported(int n);                              // pp_context.hip
+int line_plan(pp_ctx *ctx, int n, LineFft *out);         // a cached plan (the tables stay on the device)
+
+// A half spectrum's layout: rows of pitch complex values, planes of plane.
+struct SpecGeo {
+    int n, nk;
+    int pitch;
+    long long plane;
+};
+
+inline SpecGeo spec_geo(int n, int rows)
+{
+    SpecGeo g;
+    g.n = n;
+    g.nk = n / 2 + 1;
+    g.pitch = (g.nk + 15) / 16 * 16;  // whole tiles of columns: the kernels carry the padding along
+    // three 128-byte lines on top keep the planes off a common power of two
+    g.plane = (long long)g.pitch * rows + 48;
+    return g;
+}
+
+__device__ __forceinline__ float2 fmul(float2 a, float2 b)
+{
+    return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+}
+__device__ __forceinline__ float2 fmulc(float2 a, float2 b)  // a conj(b)
+{
+    return make_float2(a.x * b.x + a.y * b.y, a.y * b.x - a.x * b.y);
+}
+__device__ __forceinline__ float2 fadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
+__device__ __forceinline__ float2 fsub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
+// times -i (forward) or +i (inverse)
+template <int SIGN> __device__ __forceinline__ float2 rot(float2 a)
+{
+    return SIGN < 0 ? make_float2(a.y, -a.x) : make_float2(-a.y, a.x);
+}
+
+template <int R, int SIGN> __device__ __forceinline__ void butterfly(float2 *v)
+{
+    if constexpr (R == 2) {
+        const float2 a = v[0], b = v[1];
+        v[0] = fadd(a, b);
+        v[1] = fsub(a, b);
+    } else if constexpr (R == 4) {
+        const float2 a = fadd(v[0], v[2]), b = fsub(v[0], v[2]), c = fadd(v[1], v[3]), d = rot<SIGN>(fsub(v[1], v[3]));
+        v[0] = fadd(a, c);
+        v[1] = fadd(b, d);
+        v[2] = fsub(a, c);
+        v[3] = fsub(b, d);
+    } else if constexpr (R == 8) {
+        constexpr float h = 0.70710678118654752f;
+        float2 e[4] = {v[0], v[2], v[4], v[6]}, o[4] = {v[1], v[3], v[5], v[7]};
+        butterfly<4, SIGN>(e);
+        butterfly<4, SIGN>(o);
+        // odd half times exp(SIGN 2 pi i r / 8)
+        const float2 r1 = rot<SIGN>(o[1]), r3 = rot<SIGN>(o[3]);
+        o[1] = make_float2((o[1].x + r1.x) * h, (o[1].y + r1.y) * h);
+        o[2] = rot<SIGN>(o[2]);
+        o[3] = make_float2((r3.x - o[3].x) * h, (r3.y - o[3].y) * h);
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            v[r] = fadd(e[r], o[r]);
+            v[r + 4] = fsub(e[r], o[r]);
+        }
+    } else {
+        // odd prime: the sums and differences of conjugate inputs
+        constexpr float C3[1] = {-0.5f}, S3[1] = {0.86602540378443865f};
+        constexpr float C5[2] = {0.30901699437494742f, -0.80901699437494742f},
+                        S5[2] = {0.95105651629515357f, 0.58778525229247313f};
+        constexpr float C7[3] = {0.62348980185873353f, -0.22252093395631440f, -0.90096886790241913f},
+                        S7[3] = {0.78183148246802981f, 0.97492791218182361f, 0.43388373911755812f};
+        const float *C = R == 3 ? C3 : R == 5 ? C5 : C7, *S = R == 3 ? S3 : R == 5 ? S5 : S7;
+        constexpr int H = R / 2;
+        float2 p[H], m[H], x0 = v[0], sum = v[0];
+#pragma unroll
+        for (int q = 0; q < H; q++) {
+            p[q] = fadd(v[q + 1], v[R - 1 - q]);
+            m[q] = fsub(v[q + 1], v[R - 1 - q]);
+            sum = fadd(sum, p[q]);
+        }
+        v[0] = sum;
+#pragma unroll
+        for (int k = 1; k <= H; k++) {
+            float2 a = x0, b = make_float2(0.f, 0.f);
+#pragma unroll
+            for (int q = 0; q < H; q++) {
+                const int t = (k * (q + 1)) % R, u = t <= H ? t : R - t;
+                const float c = C[u - 1], s = t <= H ? S[u - 1] : -S[u - 1];
+                a.x += c * p[q].x;
+                a.y += c * p[q].y;
+                b.x += s * m[q].x;
+                b.y += s * m[q].y;
+            }
+            b = rot<SIGN>(b);
+            v[k] = fadd(a, b);
+            v[R - k] = fsub(a, b);
+        }
+    }
+}
+
+// LDS addresses of this thread's line, in bytes.  Columns: element e of
+// 2^logl interleaved lines.  Rows: one float2 of padding every eight, so the
+// strided writes of the first stages spread over the banks; a stage whose
+// strides are whole eights (or whose outputs fill one eight) still advances
+// by a constant.
+struct ColAddr {
+    char *s;
+    int logl;
+    static constexpr bool kAlwaysLinear = true;
+    __device__ __forceinline__ ColAddr(float2 *lds, int l, int logl) : s((char *)(lds + l)), logl(logl + 3) {}
+    __device__ __forceinline__ int off(int e) const { return e << logl; }
+    __device__ __forceinline__ int step(int e) const { return e << logl; }
+    __device__ __forceinline__ float2 &at(int o) const { return *(float2 *)(s + o); }
+    __device__ __forceinline__ float2 &operator()(int e) const { return at(off(e)); }
+};
+struct RowAddr {
+    char *s;
+    static constexpr bool kAlwaysLinear = false;
+    __device__ __forceinline__ explicit RowAddr(float2 *line) : s((char *)line) {}
+    __device__ __forceinline__ int off(int e) const { return (e + (e >> 3)) << 3; }
+    __device__ __forceinline__ int step(int e) const { return (e + (e >> 3)) << 3; }
+    __device__ __forceinline__ float2 &at(int o) const { return *(float2 *)(s + o); }
+    __device__ __forceinline__ float2 &operator()(int e) const { return at(off(e)); }
+};
+__host__ __device__ constexpr int row_pitch(int n) { return n + n / 8 + 1; }
+
+template <int R, int SIGN, bool FIRST, bool LIN, class A>
+__device__ __forceinline__ void line_stage(const A &at, const LineFft &P, int st, int jj)
+{
+    constexpr int B = (kLineEpt + R - 1) / R;
+    const int nr = P.nr[st], ns = P.ns[st];
+    // opaque, here and below, so that the addresses of every radix are not
+    // formed ahead of the stage loop and held in registers (128 instead of 64)
+    asm volatile("" : "+v"(jj));
+    // the odd radices' twiddles are loaded where they are used: two or three
+    // butterflies of them beside their values would cost half the occupancy
+    constexpr bool kAhead = !FIRST && (R & (R - 1)) == 0;
+    float2 v[B][R], w[kAhead ? B : 1][R];
+    int o[B];
+    const float2 *t[B];
+    int rd = at.step(nr), wr = at.step(ns);
+    asm volatile("" : "+s"(rd), "+s"(wr));
+#pragma unroll
+    for (int b = 0; b < B; b++) {
+        const int j = jj + b * P.tj;
+        if (j < nr) {
+            const int a = at.off(j);
+#pragma unroll
+            for (int r = 0; r < R; r++) v[b][r] = LIN ? at.at(a + r * rd) : at(j + r * nr);
+            // the twiddles travel while the line's reads finish
+            if constexpr (FIRST) {
+                o[b] = j * R;
+            } else {
+                const int h = (int)(__umul24((unsigned)j, P.magic[st]) >> 22) * ns, k = j - h;
+                o[b] = h * R + k;
+                t[b] = P.tw + (unsigned)(P.two[st] + k * R);
+                if constexpr (kAhead) {
+#pragma unroll
+                    for (int r = 1; r < R; r++) w[b][r] = t[b][r];
+                }
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < B; b++) {
+        const int j = jj + b * P.tj;
+        if (j < nr) {
+            if constexpr (!FIRST) {
+#pragma unroll
+                for (int r = 1; r < R; r++) {
+                    const float2 u = kAhead ? w[kAhead ? b : 0][r] : t[b][r];
+                    v[b][r] = SIGN < 0 ? fmul(v[b][r], u) : fmulc(v[b][r], u);
+                }
+            }
+            butterfly<R, SIGN>(v[b]);
+            const int a = at.off(o[b]);
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                if (LIN) at.at(a + r * wr) = v[b][r];
+                else at(o[b] + r * ns) = v[b][r];
+            }
+        }
+    }
+    __syncthreads();
+}
+
+template <int R, int SIGN, bool FIRST, class A>
+__device__ __forceinline__ void line_stage_any(const A &at, const LineFft &P, int st, int jj)
+{
+    if (A::kAlwaysLinear || P.lin[st]) line_stage<R, SIGN, FIRST, true>(at, P, st, jj);
+    else line_stage<R, SIGN, FIRST, false>(at, P, st, jj);
+}
+
+// FIVE: the lengths with factors 5 or 7.  Their butterflies need more
+// registers, which the other lengths' kernels are spared (64 instead of 79 in
+// the y-inverse, a quarter more wavefronts).
+template <int SIGN, bool FIRST, bool FIVE, class A>
+__device__ __forceinline__ void line_radix(const A &at, const LineFft &P, int st, int jj)
+{
+    const int R = P.rad[st];
+    if (R == 8) line_stage_any<8, SIGN, FIRST>(at, P, st, jj);
+    else if (R == 4) line_stage_any<4, SIGN, FIRST>(at, P, st, jj);
+    else if (R == 2) line_stage_any<2, SIGN, FIRST>(at, P, st, jj);
+    else if (!FIVE || R == 3) line_stage_any<3, SIGN, FIRST>(at, P, st, jj);
+    else if (R == 5) line_stage_any<5, SIGN, FIRST>(at, P, st, jj);
+    else line_stage_any<7, SIGN, FIRST>(at, P, st, jj);
+}
+
+// Transforms every line of the workgroup in place (no scaling); all threads
+// call it, and the line's elements are in LDS and visible.
+template <int SIGN, bool FIVE, class A> __device__ __forceinline__ void line_fft(const A &at, const LineFft &P, int jj)
+{
+    line_radix<SIGN, true, FIVE>(at, P, 0, jj);
+    for (int st = 1; st < P.nst; st++) line_radix<SIGN, false, FIVE>(at, P, st, jj);
+}
+
+// kernel<FIVE> by the length's factors
+#define PP_LINE_LAUNCH(P, kernel, grid, block, lds, stream, ...)                                          \
+    do {                                                                                                  \
+        if ((P).five) hipLaunchKernelGGL(kernel<true>, grid, block, lds, stream, __VA_ARGS__);            \
+        else hipLaunchKernelGGL(kernel<false>, grid, block, lds, stream, __VA_ARGS__);                    \
+        PP_HIP(hipGetLastError());                                                                        \
+    } while (0)
+
+// A line in global memory: element e at p + e step bytes, p and the step as
+// the kernel's thread sees them.  Line32 addresses within one plane by 32 bits
+// from a base that the whole workgroup shares.
+struct Line64 {
+    char *p;
+    long long step;
+    __device__ __forceinline__ float2 *at(int e) const { return (float2 *)(p + e * step); }
+};
+struct Line32 {
+    char *p;
+    unsigned off, step;
+    __device__ __forceinline__ float2 *at(int e) const { return (float2 *)(p + (off + (unsigned)e * step)); }
+};
+
+// The eight elements e = jj + q tj of a thread from and to global memory
+// (elements past the end: the last one, dropped by line_put and line_store).
+// All loads are issued before the first is used.
+template <class G> __device__ __forceinline__ void line_load(const LineFft &P, int jj, float2 x[kLineEpt], const G &g)
+{
+#pragma unroll
+    for (int q = 0; q < kLineEpt; q++) x[q] = *g.at(min(jj + q * P.tj, P.n - 1));
+}
+template <class A>
+__device__ __forceinline__ void line_put(const A &at, const LineFft &P, int jj, const float2 x[kLineEpt])
+{
+#pragma unroll
+    for (int q = 0; q < kLineEpt; q++) {
+        const int e = jj + q * P.tj;
+        if (e < P.n) at(e) = x[q];
+    }
+}
+template <class A>
+__device__ __forceinline__ void line_get(const A &at, const LineFft &P, int jj, float2 x[kLineEpt])
+{
+#pragma unroll
+    for (int q = 0; q < kLineEpt; q++) x[q] = at(min(jj + q * P.tj, P.n - 1));
+}
+template <class A, class G>
+__device__ __forceinline__ void line_store(const A &at, const LineFft &P, int jj, const G &g)
+{
+    float2 x[kLineEpt];
+    line_get(at, P, jj, x);
+#pragma unroll
+    for (int q = 0; q < kLineEpt; q++) {
+        const int e = jj + q * P.tj;
+        if (e < P.n) *g.at(e) = x[q];
+    }
+}
+
+// ------------------------------------------------------------- row joins
+// Half spectra a, b of two real rows at bin k (0 < k < n / 2, or the bins of
+// the DC and Nyquist with real values) as the complex line of both.
+template <class A> __device__ __forceinline__ void join_rows(const A &at, int n, int k, float2 a, float2 b)
+{
+    const int kc = k == 0 ? 0 : n - k;
+    if (kc == k) {  // DC and, for even n, Nyquist: real
+        at(k) = make_float2(a.x, b.x);
+    } else {
+        at(k) = make_float2(a.x - b.y, a.y + b.x);
+        at(kc) = make_float2(a.x + b.y, b.x - a.y);
+    }
+}
+
+// bins k of both rows from the transformed complex line; kc: the line's bin
+// that pairs with k
+__device__ __forceinline__ void split_rows(float2 z, float2 zc, float2 &a, float2 &b)
+{
+    a = make_float2(0.5f * (z.x + zc.x), 0.5f * (z.y - zc.y));
+    b = make_float2(0.5f * (z.y + zc.y), 0.5f * (zc.x - z.x));
+}
+
+// ---------------------------------------------------------------- host side
+// Workgroup shapes.  Columns: 2^logl lines of one plane, tj threads each.
+// Rows: nl lines (row pairs), tj threads each.
+struct LineShape {
+    int logl, nl, block;
+    size_t lds;
+    int tiles(int nk) const { return (nk + (1 << logl) - 1) >> logl; }
+};
+LineShape col_shape(LineFft &P, int max_block);  // sets P.tj
+LineShape row_shape(LineFft &P);
+
+}  // namespace pp

@@ -1,0 +1,110 @@
+// pp_fields.h -- the passes of a periodic grid's transforms with line
+// transforms (pp_fft.h), shared by the tile fields of run_tile
+// (pp_fields.hip) and of run_multitile_split (pp_split.hip).
+#pragma once
+
+#include "pp_fft.h"
+
+namespace pp {
+
+// Transfer of one output of the z pass, times scale: X; X k^2 (with k and the
+// product as _compute_laplacian forms them, or from the integer wave
+// numbers); X / k^2, kz X / k^2, kz^2 X / k^2 (0 at k = 0).  |k|^2 is mult^2
+// times an integer, exact in Float32, so these factors carry one or two
+// Float32 roundings, and the amplitude comes from a table over that integer.  The
+// factors of kx and ky that a displacement or potential takes besides are
+// constant along z and follow in the y and x passes, so three z-inverses
+// serve the nine spectra of both orders.
+enum ZKind { Z_X = 0, Z_K2F, Z_K2, Z_INV, Z_INV_Z, Z_INV_ZZ };
+
+struct ZArgs {
+    const float2 *in;
+    int nout;
+    struct Out {
+        float2 *p;
+        int kind, nyq;  // nyq: the Nyquist planes are zeroed
+    } out[7];
+    float mult, scale;  // k of an index
+    float inv, k2;      // scale / mult^2, scale mult^2
+    const float *amp;   // amplitude by integer |k|^2, or null
+    float dkf;
+    void set(double m, double sc)
+    {
+        mult = (float)m;
+        scale = (float)sc;
+        inv = (float)(sc / (m * m));
+        k2 = (float)(sc * (m * m));
+    }
+    void add(float2 *p, int kind, int nyq) { out[nout++] = Out{p, kind, nyq}; }
+};
+
+struct YArgs {
+    int narr;
+    struct Arr {
+        const float2 *in;
+        float2 *out[3];  // times 1, ky, ky^2; null: not wanted
+    } arr[7];
+    float mult;
+    void add(const float2 *in, float2 *o0, float2 *o1, float2 *o2) { arr[narr++] = Arr{in, {o0, o1, o2}}; }
+};
+
+struct XArgs {
+    int nop;
+    struct Op {
+        const float2 *in;
+        float *out;
+        int pow;    // power of kx
+        bool imag;  // the factor is i f kx^pow, else f kx^pow
+        float f;
+    } op[5];
+    float mult;
+    void add(const float2 *in, float *out, int pow, bool imag, float f) { op[nop++] = Op{in, out, pow, imag, f}; }
+};
+
+struct SrcArgs {
+    const float2 *in[6];  // potentials 11 22 33 12 13 23
+    int pow[6];
+    const float *delta;
+    float2 *out;
+    float mult;
+};
+
+// The rows of a P(k) table (device, npk log k then npk log P) and, for rows
+// evenly spaced in log k, {first log k, 1 / spacing}, else {.., 0}.
+struct PkLog {
+    const double *lk, *lp, *even;
+    int np;
+};
+inline size_t pk_log_doubles(int npk) { return 4 * (size_t)npk + 2; }
+// Copies the table into buf (pk_log_doubles values) and takes the logarithms
+// there (on the host they took as long as a 128^3 tile's kernels).
+int pk_log_device(pp_ctx *ctx, const pp_pk_table *pk, double *buf, PkLog *out);
+
+// sqrt(P(k) dk^3 n^3) at k^2 = mult^2 i for i = 0 .. 3 imax^2 (0 at i = 0), in
+// Float64 rounded once.  A mode's amplitude in the kernels was the bigger part
+// of their Float64 work: the table holds a few hundred thousand values for
+// the up to 10^9 modes of a grid.
+inline long long amp_count(int imax) { return 3ll * imax * imax + 1; }
+int amp_table(pp_ctx *ctx, const PkLog &T, double mult, double dk3, double n3, long long count, float *out);
+
+struct GridPlan {
+    LineFft row, col, ycol;
+    LineShape rs, cs, ys;  // rows; columns along z; columns along y
+    SpecGeo g;
+    hipStream_t stream;
+};
+
+int grid_plan(pp_ctx *ctx, int n, GridPlan *G);
+int rows_real(const GridPlan &G, const float *in, float2 *out);
+int rows_noise(const GridPlan &G, uint64_t seed, float2 *out);
+int cols_y_fwd(const GridPlan &G, float2 *s);
+int cols_z(const GridPlan &G, const ZArgs &A);
+int cols_y_inv(const GridPlan &G, const YArgs &Y);
+int rows_inv(const GridPlan &G, const XArgs &X);
+int rows_src(const GridPlan &G, const SrcArgs &S);
+void src_inputs(SrcArgs &S, const float2 *a, const float2 *a1, const float2 *a2, const float2 *b, const float2 *b1,
+                const float2 *c);
+int second_order(const GridPlan &G, float2 *const s[3], double mult, double scale,
+                 float *const out[3]);
+
+}  // namespace pp

@@ -17,9 +17,13 @@
 // space in the reference's order, so only the diagonal potentials and the
 // running sum are held at once.
 #include <cmath>
+#include <vector>
 
 #include "pp_common.h"
+#include "pp_fft.h"
+#include "pp_fields.h"
 #include "pp_kspace.h"
+#include "pp_noise.h"
 
 namespace pp {
 
@@ -112,6 +116,553 @@ __global__ void __launch_bounds__(256) k_src2(float *__restrict__ src, const flo
 
 int launch_noise(pp_ctx *ctx, float *out, int64_t ncells, uint64_t seed);  // pp_filter.hip
 
+// ------------------------------------------------------- line-transform path
+// The passes of a periodic grid with line transforms (pp_fft.h).
+
+// spectra of a row pair from its transformed line
+__device__ __forceinline__ void store_row_pair(const RowAddr &at, const LineFft &P, const SpecGeo &g, float2 *out,
+                                               long long r, bool two, int jj)
+{
+    const long long z = r / g.n, z2 = (r + 1) / g.n;
+    float2 *a = out + z * g.plane + (r - z * g.n) * g.pitch, *b = out + z2 * g.plane + (r + 1 - z2 * g.n) * g.pitch;
+#pragma unroll
+    for (int q = 0; q < kRowBins; q++) {
+        const int k = jj + q * P.tj;
+        if (k >= g.nk) break;
+        float2 va, vb;
+        split_rows(at(k), at(k == 0 ? 0 : g.n - k), va, vb);
+        a[k] = va;
+        if (two) b[k] = vb;
+    }
+}
+
+// x-forward of the white noise, drawn where it is transformed: the 2 n cells
+// of a row pair are n whole Threefry counter pairs
+template <bool FIVE>
+__global__ void __launch_bounds__(512) k_rows_noise(SpecGeo g, LineFft P, float2 *__restrict__ out, uint64_t seed)
+{
+    extern __shared__ float2 lds[];
+    const int n = g.n, line = threadIdx.x / P.tj, jj = threadIdx.x - line * P.tj;
+    const long long rows = (long long)n * n, rp = (long long)blockIdx.x * (blockDim.x / P.tj) + line, r = 2 * rp;
+    const RowAddr at(lds + line * row_pitch(n));
+    const bool two = r + 1 < rows;
+    if (r < rows) {
+        for (int e = jj; e < n; e += P.tj) {
+            double g1, g2;
+            threefry_normals((uint64_t)(rp * n + e), seed, g1, g2);
+            const int c1 = 2 * e, c2 = c1 + 1;
+            const float v1 = (float)g1, v2 = (float)g2;
+            if (c1 < n) at(c1).x = v1;
+            else at(c1 - n).y = two ? v1 : 0.f;
+            if (c2 < n) at(c2).x = v2;
+            else at(c2 - n).y = two ? v2 : 0.f;
+        }
+    }
+    __syncthreads();
+    line_fft<-1, FIVE>(at, P, jj);
+    if (r < rows) store_row_pair(at, P, g, out, r, two, jj);
+}
+
+// x-forward of a real field
+template <bool FIVE>
+__global__ void __launch_bounds__(512) k_rows_real(SpecGeo g, LineFft P, const float *__restrict__ in, float2 *__restrict__ out)
+{
+    extern __shared__ float2 lds[];
+    const int n = g.n, line = threadIdx.x / P.tj, jj = threadIdx.x - line * P.tj;
+    const long long rows = (long long)n * n, r = 2 * ((long long)blockIdx.x * (blockDim.x / P.tj) + line);
+    const RowAddr at(lds + line * row_pitch(n));
+    const bool two = r + 1 < rows;
+    if (r < rows) {
+        const float *pa = in + r * n, *pb = two ? pa + n : pa;
+        float2 x[kLineEpt];
+#pragma unroll
+        for (int q = 0; q < kLineEpt; q++) {
+            const int e = min(jj + q * P.tj, n - 1);
+            x[q] = make_float2(pa[e], pb[e]);
+        }
+        line_put(at, P, jj, x);
+    }
+    __syncthreads();
+    line_fft<-1, FIVE>(at, P, jj);
+    if (r < rows) store_row_pair(at, P, g, out, r, two, jj);
+}
+
+// A workgroup's tile of columns: lines kx of one plane, stride between a
+// line's elements
+struct ColTile {
+    int l, jj, kx;  // kx up to the row's pitch: the padding is carried along
+};
+
+__device__ __forceinline__ ColTile col_tile(const SpecGeo &g, int logl)
+{
+    ColTile t;
+    t.l = threadIdx.x & ((1 << logl) - 1);
+    t.jj = threadIdx.x >> logl;
+    t.kx = (blockIdx.x << logl) + t.l;
+    return t;
+}
+
+// column kx of plane z of an array
+__device__ __forceinline__ Line32 plane_line(const SpecGeo &g, const float2 *s, int z, int kx)
+{
+    return Line32{(char *)(s + z * g.plane), 8u * (unsigned)kx, 8u * (unsigned)g.pitch};
+}
+
+// y-forward, in place: grid (tiles, kz or z planes)
+template <bool FIVE>
+__global__ void __launch_bounds__(1024) k_cols_y_fwd(SpecGeo g, LineFft P, int logl, float2 *__restrict__ s)
+{
+    extern __shared__ float2 lds[];
+    const ColTile t = col_tile(g, logl);
+    const ColAddr at(lds, t.l, logl);
+    const Line32 io = plane_line(g, s, blockIdx.y, t.kx);
+    float2 x[kLineEpt];
+    line_load(P, t.jj, x, io);
+    line_put(at, P, t.jj, x);
+    __syncthreads();
+    line_fft<-1, FIVE>(at, P, t.jj);
+    line_store(at, P, t.jj, io);
+}
+
+// z-forward, transfer, z-inverse: one read of the spectrum gives every
+// output.  The mode X (times its amplitude with A.amp) stays in registers
+// while the outputs are formed one after the other in LDS.
+template <bool FIVE>
+__global__ void __launch_bounds__(1024) k_cols_z(SpecGeo g, LineFft P, int logl, ZArgs A)
+{
+#pragma clang fp contract(off)
+    extern __shared__ float2 lds[];
+    const ColTile t = col_tile(g, logl);
+    const ColAddr at(lds, t.l, logl);
+    const int n = g.n, iy = blockIdx.y, half = n / 2;
+    const long long base = (long long)iy * g.pitch + t.kx;
+    float2 X[kLineEpt];
+    line_load(P, t.jj, X, Line64{(char *)(A.in + base), 8 * g.plane});
+    line_put(at, P, t.jj, X);
+    __syncthreads();
+    line_fft<-1, FIVE>(at, P, t.jj);
+    line_get(at, P, t.jj, X);
+    const int kx = min(t.kx, g.nk - 1), fy = iy < (n + 1) / 2 ? iy : iy - n, ixy = kx * kx + fy * fy;
+    const bool nyq_xy = kx == g.nk - 1 || iy == half;
+    float ik[kLineEpt];  // scale / k^2
+#pragma unroll
+    for (int q = 0; q < kLineEpt; q++) {
+        const int e = min(t.jj + q * P.tj, n - 1), fz = e < (n + 1) / 2 ? e : e - n, i2 = ixy + fz * fz;
+        if (A.amp) {
+            const float a = A.amp[i2];
+            X[q] = make_float2(X[q].x * a, X[q].y * a);
+        }
+        const float d = (float)i2, r = __builtin_amdgcn_rcpf(d);
+        ik[q] = i2 == 0 ? 0.f : A.inv * __builtin_fmaf(__builtin_fmaf(-d, r, 1.f), r, r);
+    }
+    for (int o = 0; o < A.nout; o++) {
+        const int kind = A.out[o].kind, nyq = A.out[o].nyq;
+        int jj = t.jj;
+        asm volatile("" : "+v"(jj));  // per-element values are formed anew, not held for every output
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < kLineEpt; q++) {
+            const int e = jj + q * P.tj, fz = e < (n + 1) / 2 ? e : e - n;
+            float f;
+            if (kind == Z_X) {
+                f = A.scale;
+            } else if (kind == Z_K2F) {
+                // k and the product in Float32, both normalisations (_compute_laplacian)
+                const float fx = (float)kx * A.dkf, fyf = (float)(iy <= half ? iy : iy - n) * A.dkf,
+                            fzf = (float)(e <= half ? e : e - n) * A.dkf;
+                f = (fx * fx + fyf * fyf + fzf * fzf) * A.scale * A.scale;
+            } else if (kind == Z_K2) {
+                f = A.k2 * (float)(ixy + fz * fz);
+            } else {
+                const float kz = (float)fz * A.mult;
+                f = kind == Z_INV ? ik[q] : kind == Z_INV_Z ? ik[q] * kz : ik[q] * kz * kz;
+            }
+            if (nyq && (nyq_xy || e == half)) f = 0.f;
+            if (e < n) at(e) = make_float2(X[q].x * f, X[q].y * f);
+        }
+        __syncthreads();
+        line_fft<1, FIVE>(at, P, jj);
+        line_store(at, P, jj, Line64{(char *)(A.out[o].p + base), 8 * g.plane});
+    }
+}
+
+__global__ void __launch_bounds__(256) k_amp_table(PkLog T, double mult2, double dk3, double n3, long long count,
+                                                   float *__restrict__ out)
+{
+#pragma clang fp contract(off)
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= count) return;
+    const double k2 = (double)i * mult2;
+    out[i] = i == 0 ? 0.f : (float)sqrt(pk_eval(T.lk, T.lp, T.np, sqrt(k2), T.even[0], T.even[1]) * dk3 * n3);
+}
+
+// logarithms of k and P (one block) and whether log k is evenly spaced, to
+// 1e-9 of the spacing
+__global__ void __launch_bounds__(1024) k_pk_log(const double *__restrict__ k, const double *__restrict__ P, int np,
+                                                 double *lk, double *__restrict__ lp, double *__restrict__ even)
+{
+    __shared__ int uneven;
+    if (threadIdx.x == 0) uneven = 0;
+    for (int q = threadIdx.x; q < np; q += blockDim.x) {
+        lk[q] = log(k[q]);
+        lp[q] = log(P[q]);
+    }
+    __syncthreads();
+    const double d = (lk[np - 1] - lk[0]) / (np - 1);
+    bool off = np < 3 || !(d > 0.0);
+    for (int q = 1 + threadIdx.x; q < np; q += blockDim.x) off = off || fabs((lk[q] - lk[q - 1]) - d) > 1e-9 * d;
+    if (off) uneven = 1;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        even[0] = lk[0];
+        even[1] = uneven ? 0.0 : 1.0 / d;
+    }
+}
+
+// y-inverse of the arrays of Y, each times the powers of ky asked for: grid
+// (tiles, z planes, arrays); an output may be its input
+template <bool FIVE>
+__global__ void __launch_bounds__(1024) k_cols_y_inv(SpecGeo g, LineFft P, int logl, YArgs Y)
+{
+    extern __shared__ float2 lds[];
+    const ColTile t = col_tile(g, logl);
+    const ColAddr at(lds, t.l, logl);
+    const YArgs::Arr &R = Y.arr[blockIdx.z];
+    const int n = g.n;
+    float2 X[kLineEpt];
+    line_load(P, t.jj, X, plane_line(g, R.in, blockIdx.y, t.kx));
+    for (int o = 0; o < 3; o++) {
+        float2 *w = R.out[o];  // ky^o
+        if (!w) continue;
+        int jj = t.jj;
+        asm volatile("" : "+v"(jj));
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < kLineEpt; q++) {
+            const int e = jj + q * P.tj;
+            const float ky = (float)(e < (n + 1) / 2 ? e : e - n) * Y.mult, f = o == 0 ? 1.f : o == 1 ? ky : ky * ky;
+            if (e < n) at(e) = make_float2(X[q].x * f, X[q].y * f);
+        }
+        __syncthreads();
+        line_fft<1, FIVE>(at, P, jj);
+        line_store(at, P, jj, plane_line(g, w, blockIdx.y, t.kx));
+    }
+}
+
+// the line of a row pair from an x-spectrum times re_f or i im_f = f kx^pow
+__device__ __forceinline__ void load_row_pair(const RowAddr &at, const LineFft &P, const SpecGeo &g,
+                                              const float2 *in, long long r, bool two, int jj, int pow, bool imag,
+                                              float f, float mult)
+{
+    const long long z = r / g.n, z2 = (r + 1) / g.n;
+    const float2 *a = in + z * g.plane + (r - z * g.n) * g.pitch,
+                 *b = in + z2 * g.plane + (r + 1 - z2 * g.n) * g.pitch;
+    float2 va[kRowBins], vb[kRowBins];
+#pragma unroll
+    for (int q = 0; q < kRowBins; q++) {
+        const int k = min(jj + q * P.tj, g.nk - 1);
+        va[q] = a[k];
+        vb[q] = two ? b[k] : make_float2(0.f, 0.f);
+    }
+#pragma unroll
+    for (int q = 0; q < kRowBins; q++) {
+        const int k = jj + q * P.tj;
+        if (k >= g.nk) break;
+        const float kx = (float)k * mult, c = pow == 0 ? f : pow == 1 ? f * kx : f * kx * kx;
+        const float2 u = va[q], v = vb[q];
+        join_rows(at, g.n, k, imag ? make_float2(-c * u.y, c * u.x) : make_float2(c * u.x, c * u.y),
+                  imag ? make_float2(-c * v.y, c * v.x) : make_float2(c * v.x, c * v.y));
+    }
+}
+
+// x-inverse: grid (row pairs, outputs)
+template <bool FIVE>
+__global__ void __launch_bounds__(512) k_rows_inv(SpecGeo g, LineFft P, XArgs X)
+{
+    extern __shared__ float2 lds[];
+    const int n = g.n, line = threadIdx.x / P.tj, jj = threadIdx.x - line * P.tj;
+    const long long rows = (long long)n * n, r = 2 * ((long long)blockIdx.x * (blockDim.x / P.tj) + line);
+    const RowAddr at(lds + line * row_pitch(n));
+    const bool two = r + 1 < rows;
+    const XArgs::Op &O = X.op[blockIdx.y];
+    if (r < rows) load_row_pair(at, P, g, O.in, r, two, jj, O.pow, O.imag, O.f, X.mult);
+    __syncthreads();
+    line_fft<1, FIVE>(at, P, jj);
+    if (r < rows) {
+        float2 x[kLineEpt];
+        line_get(at, P, jj, x);
+        float *pa = O.out + r * n, *pb = pa + n;
+#pragma unroll
+        for (int q = 0; q < kLineEpt; q++) {
+            const int e = jj + q * P.tj;
+            if (e < n) {
+                pa[e] = x[q].x;
+                if (two) pb[e] = x[q].y;
+            }
+        }
+    }
+}
+
+// The second-order source: the six potentials of a row pair one after the
+// other through the same line, the running sum in registers, then its
+// x-forward; only the source's spectrum is written.  The source is quadratic
+// in the potentials, whose common sign is left out.  delta: null for
+// run_tile's source p11 p22 + (p11 + p22) p33 - p12^2 - p13^2 - p23^2, else
+// the split tiles' delta^2 / 2 - sum phi_dd^2 / 2 - sum phi_ab^2, in Float32.
+template <bool FIVE>
+__global__ void __launch_bounds__(512) k_rows_src(SpecGeo g, LineFft P, SrcArgs S)
+{
+#pragma clang fp contract(off)
+    extern __shared__ float2 lds[];
+    const int n = g.n, line = threadIdx.x / P.tj, jj = threadIdx.x - line * P.tj;
+    const long long rows = (long long)n * n, r = 2 * ((long long)blockIdx.x * (blockDim.x / P.tj) + line);
+    const RowAddr at(lds + line * row_pitch(n));
+    const bool two = r + 1 < rows, live = r < rows;
+    float2 src[kLineEpt], sum[kLineEpt];
+#pragma unroll
+    for (int q = 0; q < kLineEpt; q++) {
+        const int e = min(jj + q * P.tj, n - 1);
+        src[q] = sum[q] = make_float2(0.f, 0.f);
+        if (S.delta && live) {
+            const float d1 = S.delta[r * n + e], d2 = two ? S.delta[(r + 1) * n + e] : 0.f;
+            src[q] = make_float2((d1 * d1) * 0.5f, (d2 * d2) * 0.5f);
+        }
+    }
+    for (int v = 0; v < 6; v++) {  // 11 22 33 12 13 23
+        int j2 = jj;
+        asm volatile("" : "+v"(j2));
+        __syncthreads();
+        if (live) load_row_pair(at, P, g, S.in[v], r, two, j2, S.pow[v], false, 1.f, S.mult);
+        __syncthreads();
+        line_fft<1, FIVE>(at, P, j2);
+#pragma unroll
+        for (int q = 0; q < kLineEpt; q++) {
+            const float2 p = at(min(j2 + q * P.tj, n - 1));
+            if (S.delta || v >= 3) {
+                const float co = v < 3 ? 0.5f : 1.0f;
+                src[q].x = src[q].x - (p.x * p.x) * co;
+                src[q].y = src[q].y - (p.y * p.y) * co;
+            } else {
+                src[q].x = src[q].x + sum[q].x * p.x;
+                src[q].y = src[q].y + sum[q].y * p.y;
+                sum[q] = fadd(sum[q], p);
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kLineEpt; q++) {
+        const int e = jj + q * P.tj;
+        if (e < n) at(e) = two ? src[q] : make_float2(src[q].x, 0.f);
+    }
+    __syncthreads();
+    line_fft<-1, FIVE>(at, P, jj);
+    if (live) store_row_pair(at, P, g, S.out, r, two, jj);
+}
+
+// ---- launches
+static unsigned row_blocks(const SpecGeo &g, const LineShape &s)
+{
+    const long long pairs = ((long long)g.n * g.n + 1) / 2;
+    return (unsigned)((pairs + s.nl - 1) / s.nl);
+}
+
+int grid_plan(pp_ctx *ctx, int n, GridPlan *G)
+{
+    PP_CHECK(line_plan(ctx, n, &G->row));
+    G->col = G->row;
+    G->rs = row_shape(G->row);
+    G->cs = col_shape(G->col, 512);
+    // the y passes fit 64 registers, so that two workgroups of 1024 threads
+    // (16 columns of a long line) share a CU; the z pass and the radices 5 and
+    // 7 take more and keep to 512 threads
+    G->ycol = G->col;
+    G->ys = col_shape(G->ycol, G->col.five ? 512 : 1024);
+    G->g = spec_geo(n, n);
+    G->stream = ctx->stream;
+    return PP_OK;
+}
+
+int rows_real(const GridPlan &G, const float *in, float2 *out)
+{
+    PP_LINE_LAUNCH(G.row, k_rows_real, dim3(row_blocks(G.g, G.rs)), dim3(G.rs.block), G.rs.lds, G.stream, G.g, G.row, in,
+                       out);
+    return PP_OK;
+}
+
+int rows_noise(const GridPlan &G, uint64_t seed, float2 *out)
+{
+    PP_LINE_LAUNCH(G.row, k_rows_noise, dim3(row_blocks(G.g, G.rs)), dim3(G.rs.block), G.rs.lds, G.stream, G.g, G.row,
+                       out, seed);
+    return PP_OK;
+}
+
+int cols_y_fwd(const GridPlan &G, float2 *s)
+{
+    PP_LINE_LAUNCH(G.ycol, k_cols_y_fwd, dim3(G.ys.tiles(G.g.nk), G.g.n), dim3(G.ys.block), G.ys.lds, G.stream, G.g,
+                       G.ycol, G.ys.logl, s);
+    return PP_OK;
+}
+
+int cols_z(const GridPlan &G, const ZArgs &A)
+{
+    PP_LINE_LAUNCH(G.col, k_cols_z, dim3(G.cs.tiles(G.g.nk), G.g.n), dim3(G.cs.block), G.cs.lds, G.stream, G.g, G.col,
+                       G.cs.logl, A);
+    return PP_OK;
+}
+
+int cols_y_inv(const GridPlan &G, const YArgs &Y)
+{
+    PP_LINE_LAUNCH(G.ycol, k_cols_y_inv, dim3(G.ys.tiles(G.g.nk), G.g.n, Y.narr), dim3(G.ys.block), G.ys.lds, G.stream,
+                       G.g, G.ycol, G.ys.logl, Y);
+    return PP_OK;
+}
+
+int rows_inv(const GridPlan &G, const XArgs &X)
+{
+    PP_LINE_LAUNCH(G.row, k_rows_inv, dim3(row_blocks(G.g, G.rs), X.nop), dim3(G.rs.block), G.rs.lds, G.stream, G.g,
+                       G.row, X);
+    return PP_OK;
+}
+
+int rows_src(const GridPlan &G, const SrcArgs &S)
+{
+    PP_LINE_LAUNCH(G.row, k_rows_src, dim3(row_blocks(G.g, G.rs)), dim3(G.rs.block), G.rs.lds, G.stream, G.g, G.row, S);
+    return PP_OK;
+}
+
+int amp_table(pp_ctx *ctx, const PkLog &T, double mult, double dk3, double n3, long long count, float *out)
+{
+    hipLaunchKernelGGL(k_amp_table, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, ctx->stream, T, mult * mult,
+                       dk3, n3, count, out);
+    PP_HIP(hipGetLastError());
+    return PP_OK;
+}
+
+int pk_log_device(pp_ctx *ctx, const pp_pk_table *pk, double *buf, PkLog *out)
+{
+    const int np = pk->npk;
+    double *lk = buf, *lp = lk + np, *k = lp + np, *P = k + np, *even = P + np;
+    PP_HIP(hipMemcpyAsync(k, pk->k, np * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
+    PP_HIP(hipMemcpyAsync(P, pk->P, np * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
+    hipLaunchKernelGGL(k_pk_log, dim3(1), dim3(1024), 0, ctx->stream, (const double *)k, (const double *)P, np, lk, lp,
+                       even);
+    PP_HIP(hipGetLastError());
+    *out = PkLog{lk, lp, even, np};
+    return PP_OK;
+}
+
+// The six potentials' arrays: y-inverses of X / k^2, kz X / k^2, kz^2 X / k^2
+// times powers of ky, in the order 11 22 33 12 13 23 with their powers of kx
+void src_inputs(SrcArgs &S, const float2 *a, const float2 *a1, const float2 *a2, const float2 *b, const float2 *b1,
+                const float2 *c)
+{
+    const float2 *in[6] = {a, a2, c, a1, b, b1};
+    const int pow[6] = {2, 0, 0, 1, 1, 0};
+    for (int q = 0; q < 6; q++) {
+        S.in[q] = in[q];
+        S.pow[q] = pow[q];
+    }
+}
+
+// eta2 = -i k / k^2 src_k from the x-spectrum of the source in s[0] (three
+// arrays of work space)
+int second_order(const GridPlan &G, float2 *const s[3], double mult, double scale, float *const out[3])
+{
+    PP_CHECK(cols_y_fwd(G, s[0]));
+    ZArgs Z{};
+    Z.in = s[0];
+    Z.set(mult, scale);
+    Z.add(s[0], Z_INV, 1);
+    Z.add(s[1], Z_INV_Z, 1);
+    PP_CHECK(cols_z(G, Z));
+    YArgs Y{};
+    Y.mult = (float)mult;
+    Y.add(s[0], s[0], s[2], nullptr);
+    Y.add(s[1], s[1], nullptr, nullptr);
+    PP_CHECK(cols_y_inv(G, Y));
+    XArgs X{};
+    X.mult = (float)mult;
+    X.add(s[0], out[0], 1, true, -1.f);
+    X.add(s[2], out[1], 0, true, -1.f);
+    X.add(s[1], out[2], 0, true, -1.f);
+    return rows_inv(G, X);
+}
+
+// pp_make_tile_fields with line transforms.  The spectrum of delta is the
+// noise's times the amplitude (rfft of its own inverse transform), so delta
+// is not transformed again.
+static int make_tile_lines(pp_ctx *ctx, int n, double boxsize, uint64_t seed, const pp_pk_table *pk, pp_tile_fields *f)
+{
+    const bool lpt2 = f->eta2x != nullptr;
+    GridPlan G;
+    PP_CHECK(grid_plan(ctx, n, &G));
+    const size_t arr = (size_t)G.g.plane * n;  // complex values of one array
+    // delta / source, A', B', ky A', L, and with 2LPT A, B, C, ky A, ky^2 A, ky B
+    const int narr = 4 + (f->lapd ? 1 : 0) + (lpt2 ? 6 : 0);
+    PP_CHECK(ctx->d_spec.grow(arr * narr * sizeof(float2)));
+    float2 *s[11];
+    for (int q = 0; q < narr; q++) s[q] = ctx->d_spec.as<float2>() + arr * q;
+    float2 *L = f->lapd ? s[4] : nullptr, **W = s + 4 + (f->lapd ? 1 : 0);
+    PP_CHECK(rows_noise(G, seed, s[0]));
+    PP_CHECK(cols_y_fwd(G, s[0]));
+    const double dk = 2.0 * M_PI / boxsize, mult = ((double)n * dk) / (double)n, n3 = (double)n * n * n;
+    const long long count = amp_count(n / 2);
+    PP_CHECK(ctx->d_misc.grow(pk_log_doubles(pk->npk) * sizeof(double) + count * sizeof(float)));
+    double *d_pk = ctx->d_misc.as<double>();
+    float *amp = (float *)(d_pk + pk_log_doubles(pk->npk));
+    PkLog T;
+    PP_CHECK(pk_log_device(ctx, pk, d_pk, &T));
+    PP_CHECK(amp_table(ctx, T, mult, dk * dk * dk, n3, count, amp));
+    ZArgs Z{};
+    Z.in = s[0];
+    Z.set(mult, 1.0 / n3);
+    Z.amp = amp;
+    Z.dkf = (float)dk;
+    Z.add(s[0], Z_X, 0);
+    Z.add(s[1], Z_INV, 1);
+    Z.add(s[2], Z_INV_Z, 1);
+    if (L) Z.add(L, Z_K2F, 0);
+    if (lpt2) {
+        Z.add(W[0], Z_INV, 0);
+        Z.add(W[1], Z_INV_Z, 0);
+        Z.add(W[2], Z_INV_ZZ, 0);
+    }
+    PP_CHECK(cols_z(G, Z));
+    YArgs Y{};
+    Y.mult = (float)mult;
+    Y.add(s[0], s[0], nullptr, nullptr);
+    Y.add(s[1], s[1], s[3], nullptr);
+    Y.add(s[2], s[2], nullptr, nullptr);
+    if (L) Y.add(L, L, nullptr, nullptr);
+    if (lpt2) {
+        Y.add(W[0], W[0], W[3], W[4]);
+        Y.add(W[1], W[1], W[5], nullptr);
+        Y.add(W[2], W[2], nullptr, nullptr);
+    }
+    PP_CHECK(cols_y_inv(G, Y));
+    XArgs X{};
+    X.mult = (float)mult;
+    X.add(s[0], f->delta, 0, false, 1.f);
+    X.add(s[1], f->etax, 1, true, 1.f);
+    X.add(s[3], f->etay, 0, true, 1.f);
+    X.add(s[2], f->etaz, 0, true, 1.f);
+    if (L) X.add(L, f->lapd, 0, false, 1.f);
+    PP_CHECK(rows_inv(G, X));
+    if (lpt2) {
+        SrcArgs S{};
+        S.mult = (float)mult;
+        S.out = s[0];
+        src_inputs(S, W[0], W[3], W[4], W[1], W[5], W[2]);
+        PP_CHECK(rows_src(G, S));
+        float2 *w[3] = {s[0], s[1], s[2]};
+        float *out[3] = {f->eta2x, f->eta2y, f->eta2z};
+        PP_CHECK(second_order(G, w, mult, 1.0 / n3, out));
+    }
+    PP_HIP(hipStreamSynchronize(ctx->stream));
+    return PP_OK;
+}
+
 }  // namespace pp
 
 using namespace pp;
@@ -129,6 +680,7 @@ extern "C" int pp_make_tile_fields(pp_ctx *ctx, int n, double boxsize, uint64_t 
         PP_ARG(q == 0 || pk->k[q] > pk->k[q - 1], "P(k) table k not increasing at row %d", q);
     }
     PP_CHECK(ensure_device(ctx));
+    if (line_supported(n)) return make_tile_lines(ctx, n, boxsize, seed, pk, f);
     PP_CHECK(fft_prepare(ctx, n));
     const int nk = n / 2 + 1;
     const long long total = (long long)nk * n * n;

@@ -1,0 +1,56 @@
+"""The field kernels on line transforms (csrc/pp_fft.h) at the lengths where
+their stages and tiles can go wrong: the shortest and an odd one, every radix
+alone and mixed, butterflies that do not divide the threads, tiles with a
+remainder of columns, odd numbers of rows; and lengths without a line
+transform, which take rocFFT.
+
+Tolerance: 2e-5 of each field's largest value, as for the fields on rocFFT
+(Float32 transforms against pocketfft in Float64).
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _close(name, got, want):
+    scale = float(np.abs(want).max())
+    err = float(np.abs(got - want).max())
+    assert scale > 0 and err <= 2e-5 * scale, (name, err, scale)
+
+
+@pytest.mark.parametrize("n", [14, 16, 21, 27, 34, 35, 49, 60, 64, 75, 96, 98, 125, 128, 144])
+def test_periodic_fields(ctx, n):
+    from oracle import fields as OF
+    from peakpatch_hip import synth
+    box = 1.3 * n
+    t = synth.make_tile(ctx, n, box, seed=n, ilpt=2, want_lapd=True)
+    ref = OF.make_tile(n, box, n, OF.PkTable(*synth.pk_table()))
+    host = lambda a: a.cpu().numpy()
+    _close("delta", host(t.delta), ref.delta)
+    _close("lapd", host(t.lapd), ref.lapd)
+    for q in range(3):
+        _close(f"eta{q}", host(t.eta[q]), ref.eta[q])
+        _close(f"eta2{q}", host(t.eta2[q]), ref.eta2[q])
+
+
+def test_uneven_power_table(ctx):
+    """A P(k) table whose rows are not evenly spaced in log k."""
+    import ctypes as C
+
+    import torch
+    from oracle import fields as OF
+    from peakpatch_hip import _lib as L
+    from peakpatch_hip import synth
+    n, box = 40, 60.0
+    k, P = synth.pk_table()
+    pick = np.unique(np.concatenate([np.arange(0, 1200, 7), np.arange(1200, 2001, 3)]))
+    k, P = np.ascontiguousarray(k[pick]), np.ascontiguousarray(P[pick])
+    f = [torch.empty((n, n, n), device="cuda") for _ in range(4)]
+    tab = L.PkTable(len(k), k.ctypes.data, P.ctypes.data)
+    out = L.TileFields(*(a.data_ptr() for a in f), None, None, None, None)
+    ctx._call(lambda: ctx.lib.pp_make_tile_fields(ctx.h, n, box, 5, C.byref(tab), C.byref(out)), True)
+    ref = OF.make_tile(n, box, 5, OF.PkTable(k, P), ilpt=1, want_lapd=False)
+    _close("delta", f[0].cpu().numpy(), ref.delta)
+    for q in range(3):
+        _close(f"eta{q}", f[1 + q].cpu().numpy(), ref.eta[q])
