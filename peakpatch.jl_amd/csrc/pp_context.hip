@@ -174,15 +174,24 @@ int line_plan(pp_ctx *ctx, int n, LineFft *out)
         f.n = n;
         int rest = n, e2 = 0;
         while (rest % 2 == 0) { rest /= 2; e2++; }
-        // powers of two as few stages as radix 8 and 4 give (8 8 2 -> 8 4 4)
+        // powers of two in as few stages as radix 8 and 4 give (8 8 2 -> 8 4 4);
+        // a multiple of 64 with radix 8 at both ends
         std::vector<int> rad;
+        const bool reg = n % 64 == 0;
+        if (reg) {
+            e2 -= 6;
+            rad.push_back(8);
+        }
         while (e2 > 0) {
             const int take = e2 == 4 || e2 == 2 ? 2 : e2 >= 3 ? 3 : 1;
             rad.push_back(1 << take);
             e2 -= take;
         }
+        bool seven = false;
         for (int p : {3, 5, 7})
-            while (rest % p == 0) { rest /= p; rad.push_back(p); f.five |= p > 3; }
+            while (rest % p == 0) { rest /= p; rad.push_back(p); seven = seven || p > 3; }
+        if (reg) rad.push_back(8);
+        f.mode = !reg ? kLineAny : seven ? kLineReg7 : kLineReg;
         PP_ARG(rad.size() <= 8, "line length %d takes %zu stages", n, rad.size());
         std::vector<float2> t;
         auto root = [&](double num, double den) {  // exp(-i pi num / den)
@@ -229,15 +238,15 @@ void line_release(pp_ctx *ctx)
 LineShape col_shape(LineFft &P, int max_block)
 {
     // 16 columns (128-byte pieces of a row) where their threads fit the
-    // workgroup and the tile fits 64 KB, else 8
+    // workgroup and two tiles fit a CU's LDS, else 8
     LineShape s{};
-    for (s.logl = 4; s.logl >= 3; s.logl--) {
+    for (s.logl = 4;; s.logl--) {
         const int step = 64 >> s.logl;  // whole wavefronts
         P.tj = ((P.n + kLineEpt - 1) / kLineEpt + step - 1) / step * step;
         s.nl = 1 << s.logl;
         s.block = P.tj << s.logl;
-        s.lds = sizeof(float2) * ((size_t)P.n << s.logl);
-        if ((s.block <= max_block && s.lds <= 65536) || s.logl == 3) break;
+        s.lds = sizeof(float2) * ((size_t)(P.mode == kLineAny ? P.n : P.n + P.n / 8) << s.logl);
+        if ((s.block <= max_block && s.lds <= 72 * 1024) || s.logl == 3) break;
     }
     return s;
 }
@@ -247,9 +256,10 @@ LineShape row_shape(LineFft &P)
     // one wavefront where it holds whole lines (its barriers cost nothing),
     // else the fewest lines that fill whole wavefronts
     LineShape s{};
-    P.tj = ((P.n + kLineEpt - 1) / kLineEpt + 15) / 16 * 16;
+    P.tj = P.mode == kLineAny ? ((P.n + kLineEpt - 1) / kLineEpt + 15) / 16 * 16 : P.n / 8;
     s.nl = 1;
     while (s.nl * P.tj % 64) s.nl++;
+    if (s.nl * P.tj > 512) s.nl = std::max(1, 256 / P.tj);
     s.block = s.nl * P.tj;
     s.lds = sizeof(float2) * (size_t)s.nl * row_pitch(P.n);
     return s;

@@ -39,7 +39,7 @@ constexpr int kRowBins = 5;    // bins of a half spectrum a thread handles, >= (
 struct LineFft {
     int n, nst;
     int tj;                  // threads per line, >= n / kLineEpt
-    int five;                // a stage of radix 5 or 7
+    int mode;                // LineMode
     int rad[8], ns[8], nr[8], lin[8];  // radix, sub-length, butterflies; rows: constant strides
     unsigned magic[8];       // floor(2^22 / ns) + 1: j / ns = j magic >> 22 for j < 2048
     int two[8];              // a stage's twiddles exp(-2 pi i k r / (ns R)) at tw[two + k R + r]
@@ -56,11 +56,13 @@ struct LinePlan {
 bool line_supported(int n);                              // pp_context.hip
 int line_plan(pp_ctx *ctx, int n, LineFft *out);         // a cached plan (the tables stay on the device)
 
-// A half spectrum's layout: rows of pitch complex values, planes of plane.
+// A half spectrum's layout: rows of pitch complex values, planes of z.
 struct SpecGeo {
     int n, nk;
     int pitch;
     long long plane;
+    __host__ __device__ long long row(int z, int y) const { return z * plane + (long long)y * pitch; }
+    size_t size(int nz) const { return (size_t)plane * nz; }
 };
 
 inline SpecGeo spec_geo(int n, int rows)
@@ -69,7 +71,10 @@ inline SpecGeo spec_geo(int n, int rows)
     g.n = n;
     g.nk = n / 2 + 1;
     g.pitch = (g.nk + 15) / 16 * 16;  // whole tiles of columns: the kernels carry the padding along
-    // three 128-byte lines on top keep the planes off a common power of two
+    // three 128-byte lines on top keep the planes off a common power of two.
+    // (Slabs of 16 z side by side, so that a column along z touches 32 places
+    // instead of 512, change nothing: the passes are not bound by address
+    // translation.)
     g.plane = (long long)g.pitch * rows + 48;
     return g;
 }
@@ -153,18 +158,20 @@ template <int R, int SIGN> __device__ __forceinline__ void butterfly(float2 *v)
     }
 }
 
-// LDS addresses of this thread's line, in bytes.  Columns: element e of
-// 2^logl interleaved lines.  Rows: one float2 of padding every eight, so the
-// strided writes of the first stages spread over the banks; a stage whose
-// strides are whole eights (or whose outputs fill one eight) still advances
-// by a constant.
-struct ColAddr {
+// LDS addresses of this thread's line, in bytes.  Both layouts leave one
+// element of padding every eight, so the strided writes of the first stage
+// spread over the banks; a stage whose strides are whole eights (or whose
+// outputs fill one eight) still advances by a constant.  Columns: element e of
+// 2^logl interleaved lines; padded only for the lengths whose strides are
+// always whole eights (the others' columns would lose more by it).
+template <bool PAD> struct ColAddr {
     char *s;
     int logl;
     static constexpr bool kAlwaysLinear = true;
     __device__ __forceinline__ ColAddr(float2 *lds, int l, int logl) : s((char *)(lds + l)), logl(logl + 3) {}
-    __device__ __forceinline__ int off(int e) const { return e << logl; }
-    __device__ __forceinline__ int step(int e) const { return e << logl; }
+    __device__ __forceinline__ int off(int e) const { return (PAD ? e + (e >> 3) : e) << logl; }
+    __device__ __forceinline__ int step(int e) const { return (PAD ? e + (e >> 3) : e) << logl; }
+    __device__ __forceinline__ int step1() const { return 1 << logl; }
     __device__ __forceinline__ float2 &at(int o) const { return *(float2 *)(s + o); }
     __device__ __forceinline__ float2 &operator()(int e) const { return at(off(e)); }
 };
@@ -174,6 +181,7 @@ struct RowAddr {
     __device__ __forceinline__ explicit RowAddr(float2 *line) : s((char *)line) {}
     __device__ __forceinline__ int off(int e) const { return (e + (e >> 3)) << 3; }
     __device__ __forceinline__ int step(int e) const { return (e + (e >> 3)) << 3; }
+    __device__ __forceinline__ int step1() const { return 8; }  // within eight elements
     __device__ __forceinline__ float2 &at(int o) const { return *(float2 *)(s + o); }
     __device__ __forceinline__ float2 &operator()(int e) const { return at(off(e)); }
 };
@@ -247,48 +255,24 @@ __device__ __forceinline__ void line_stage_any(const A &at, const LineFft &P, in
     else line_stage<R, SIGN, FIRST, false>(at, P, st, jj);
 }
 
-// FIVE: the lengths with factors 5 or 7.  Their butterflies need more
-// registers, which the other lengths' kernels are spared (64 instead of 79 in
-// the y-inverse, a quarter more wavefronts).
-template <int SIGN, bool FIRST, bool FIVE, class A>
-__device__ __forceinline__ void line_radix(const A &at, const LineFft &P, int st, int jj)
-{
-    const int R = P.rad[st];
-    if (R == 8) line_stage_any<8, SIGN, FIRST>(at, P, st, jj);
-    else if (R == 4) line_stage_any<4, SIGN, FIRST>(at, P, st, jj);
-    else if (R == 2) line_stage_any<2, SIGN, FIRST>(at, P, st, jj);
-    else if (!FIVE || R == 3) line_stage_any<3, SIGN, FIRST>(at, P, st, jj);
-    else if (R == 5) line_stage_any<5, SIGN, FIRST>(at, P, st, jj);
-    else line_stage_any<7, SIGN, FIRST>(at, P, st, jj);
-}
-
-// Transforms every line of the workgroup in place (no scaling); all threads
-// call it, and the line's elements are in LDS and visible.
-template <int SIGN, bool FIVE, class A> __device__ __forceinline__ void line_fft(const A &at, const LineFft &P, int jj)
-{
-    line_radix<SIGN, true, FIVE>(at, P, 0, jj);
-    for (int st = 1; st < P.nst; st++) line_radix<SIGN, false, FIVE>(at, P, st, jj);
-}
-
-// kernel<FIVE> by the length's factors
-#define PP_LINE_LAUNCH(P, kernel, grid, block, lds, stream, ...)                                          \
-    do {                                                                                                  \
-        if ((P).five) hipLaunchKernelGGL(kernel<true>, grid, block, lds, stream, __VA_ARGS__);            \
-        else hipLaunchKernelGGL(kernel<false>, grid, block, lds, stream, __VA_ARGS__);                    \
-        PP_HIP(hipGetLastError());                                                                        \
-    } while (0)
-
-// A line in global memory: element e at p + e step bytes, p and the step as
-// the kernel's thread sees them.  Line32 addresses within one plane by 32 bits
-// from a base that the whole workgroup shares.
-struct Line64 {
+// A column in global memory.  LineZ: along z at row y.  LineY: along y (row0 +
+// e stride) at plane z, by 32 bits from an address the workgroup shares.
+struct LineZ {
     char *p;
     long long step;
+    __device__ __forceinline__ LineZ(const SpecGeo &g, const float2 *s, int y, int kx)
+        : p((char *)(s + g.row(0, y) + kx)), step(8 * g.plane)
+    {
+    }
     __device__ __forceinline__ float2 *at(int e) const { return (float2 *)(p + e * step); }
 };
-struct Line32 {
+struct LineY {
     char *p;
     unsigned off, step;
+    __device__ __forceinline__ LineY(const SpecGeo &g, const float2 *s, int z, int row0, int stride, int kx)
+        : p((char *)(s + g.row(z, 0))), off(8u * (unsigned)(row0 * g.pitch + kx)), step(8u * (unsigned)(stride * g.pitch))
+    {
+    }
     __device__ __forceinline__ float2 *at(int e) const { return (float2 *)(p + (off + (unsigned)e * step)); }
 };
 
@@ -315,16 +299,121 @@ __device__ __forceinline__ void line_get(const A &at, const LineFft &P, int jj, 
 #pragma unroll
     for (int q = 0; q < kLineEpt; q++) x[q] = at(min(jj + q * P.tj, P.n - 1));
 }
-template <class A, class G>
-__device__ __forceinline__ void line_store(const A &at, const LineFft &P, int jj, const G &g)
+template <class G> __device__ __forceinline__ void line_store(const LineFft &P, int jj, const float2 x[kLineEpt], const G &g)
 {
-    float2 x[kLineEpt];
-    line_get(at, P, jj, x);
 #pragma unroll
     for (int q = 0; q < kLineEpt; q++) {
         const int e = jj + q * P.tj;
         if (e < P.n) *g.at(e) = x[q];
     }
+}
+
+// How a length is transformed (LineFft::mode):
+//  kLineReg   n = 64 m without factors 5 and 7.  The first and the last stage
+//             are of radix 8, whose butterflies take and give exactly the
+//             elements e = jj + q tj that a thread holds, so a line enters and
+//             leaves in registers: half the LDS traffic and barriers of 512 =
+//             8 8 8.
+//  kLineReg7  the same with factors 5 or 7 in between.  Their butterflies
+//             need more registers, which the kernels of kLineReg are spared.
+//  kLineAny   every other length: all stages through LDS.
+enum LineMode { kLineReg = 0, kLineReg7 = 1, kLineAny = 2 };
+
+template <int SIGN, bool FIRST, int M, class A>
+__device__ __forceinline__ void line_radix(const A &at, const LineFft &P, int st, int jj)
+{
+    const int R = P.rad[st];
+    if (R == 8) line_stage_any<8, SIGN, FIRST>(at, P, st, jj);
+    else if (R == 4) line_stage_any<4, SIGN, FIRST>(at, P, st, jj);
+    else if (R == 2) line_stage_any<2, SIGN, FIRST>(at, P, st, jj);
+    else if (M == kLineReg || R == 3) line_stage_any<3, SIGN, FIRST>(at, P, st, jj);
+    else if (R == 5) line_stage_any<5, SIGN, FIRST>(at, P, st, jj);
+    else line_stage_any<7, SIGN, FIRST>(at, P, st, jj);
+}
+
+// Transforms every line of the workgroup (no scaling); all threads call it.
+// Thread jj holds x[q] = element jj + q tj on the way in and out.  IN_LDS: the
+// line is in LDS instead, visible to all.  OUT_LDS: it is left there, visible.
+// LDS may be written by the caller only after a barrier of its own.
+template <int SIGN, int M, bool IN_LDS, bool OUT_LDS, class A>
+__device__ __forceinline__ void line_run(const A &at, const LineFft &P, int jj, float2 x[kLineEpt])
+{
+    if constexpr (M == kLineAny) {
+        if constexpr (!IN_LDS) {
+            __syncthreads();
+            line_put(at, P, jj, x);
+            __syncthreads();
+        }
+        line_radix<SIGN, true, M>(at, P, 0, jj);
+        for (int st = 1; st < P.nst; st++) line_radix<SIGN, false, M>(at, P, st, jj);
+        if constexpr (!OUT_LDS) line_get(at, P, jj, x);
+    } else {
+        asm volatile("" : "+v"(jj));
+        const int wide = at.step(P.tj), one = at.step1();
+        const int own = at.off(jj), first = at.off(8 * jj);
+        if constexpr (IN_LDS) {
+#pragma unroll
+            for (int r = 0; r < 8; r++) x[r] = at.at(own + r * wide);
+        }
+        __syncthreads();
+        butterfly<8, SIGN>(x);
+#pragma unroll
+        for (int r = 0; r < 8; r++) at.at(first + r * one) = x[r];
+        __syncthreads();
+        for (int st = 1; st + 1 < P.nst; st++) line_radix<SIGN, false, M>(at, P, st, jj);
+        const float2 *t = P.tw + (unsigned)(P.two[P.nst - 1] + 8 * jj);
+#pragma unroll
+        for (int r = 0; r < 8; r++) x[r] = at.at(own + r * wide);
+#pragma unroll
+        for (int r = 1; r < 8; r++) x[r] = SIGN < 0 ? fmul(x[r], t[r]) : fmulc(x[r], t[r]);
+        butterfly<8, SIGN>(x);
+        if constexpr (OUT_LDS) {
+#pragma unroll
+            for (int r = 0; r < 8; r++) at.at(own + r * wide) = x[r];
+            __syncthreads();
+        }
+    }
+}
+
+// kernel<mode> by the length
+template <class K, class... Args>
+int line_launch(K kernel, dim3 grid, dim3 block, size_t lds, hipStream_t stream, Args... args)
+{
+    if (lds > 64 * 1024)
+        PP_HIP(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(kernel, grid, block, lds, stream, args...);
+    PP_HIP(hipGetLastError());
+    return PP_OK;
+}
+#define PP_LINE_LAUNCH(P, kernel, grid, block, lds, stream, ...)                                                     \
+    PP_CHECK((P).mode == kLineReg    ? line_launch(kernel<kLineReg>, grid, block, lds, stream, __VA_ARGS__)           \
+             : (P).mode == kLineReg7 ? line_launch(kernel<kLineReg7>, grid, block, lds, stream, __VA_ARGS__)          \
+                                     : line_launch(kernel<kLineAny>, grid, block, lds, stream, __VA_ARGS__))
+
+// A workgroup's tile of columns: lines kx of one plane.  Tiles are numbered
+// along kx first.  For the z passes each XCD takes one run of them (nx = 8;
+// workgroups go round-robin to the eight XCDs), so the neighbours of an
+// 8-column tile, which touch the other halves of its 128-byte lines, find them
+// in the same L2 (4% of the z pass; the y passes, whose neighbours are one row
+// apart, lose 8% by it and go without, nx = 1).
+constexpr int kColXCD = 8;
+struct ColGrid {
+    int logl, nx, tiles, total, per;
+    unsigned blocks() const { return (unsigned)(per * nx); }
+};
+struct ColTile {
+    int l, jj, kx;  // kx up to the row's pitch: the padding is carried along
+    int plane;      // < 0: no tile (the whole workgroup leaves)
+};
+__device__ __forceinline__ ColTile col_tile(const ColGrid &C)
+{
+    const int b = C.nx == 1 ? (int)blockIdx.x : (int)(blockIdx.x % kColXCD) * C.per + (int)(blockIdx.x / kColXCD);
+    ColTile t;
+    t.plane = b < C.total ? b / C.tiles : -1;
+    t.l = threadIdx.x & ((1 << C.logl) - 1);
+    t.jj = threadIdx.x >> C.logl;
+    t.kx = ((b - t.plane * C.tiles) << C.logl) + t.l;
+    return t;
 }
 
 // ------------------------------------------------------------- row joins
@@ -355,7 +444,16 @@ __device__ __forceinline__ void split_rows(float2 z, float2 zc, float2 &a, float
 struct LineShape {
     int logl, nl, block;
     size_t lds;
-    int tiles(int nk) const { return (nk + (1 << logl) - 1) >> logl; }
+    ColGrid grid(int nk, int planes, int nx) const
+    {
+        ColGrid c;
+        c.logl = logl;
+        c.nx = nx;
+        c.tiles = (nk + (1 << logl) - 1) >> logl;
+        c.total = c.tiles * planes;
+        c.per = (c.total + nx - 1) / nx;
+        return c;
+    }
 };
 LineShape col_shape(LineFft &P, int max_block);  // sets P.tj
 LineShape row_shape(LineFft &P);

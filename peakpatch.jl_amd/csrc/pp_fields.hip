@@ -124,7 +124,7 @@ __device__ __forceinline__ void store_row_pair(const RowAddr &at, const LineFft 
                                                long long r, bool two, int jj)
 {
     const long long z = r / g.n, z2 = (r + 1) / g.n;
-    float2 *a = out + z * g.plane + (r - z * g.n) * g.pitch, *b = out + z2 * g.plane + (r + 1 - z2 * g.n) * g.pitch;
+    float2 *a = out + g.row((int)z, (int)(r - z * g.n)), *b = out + g.row((int)z2, (int)(r + 1 - z2 * g.n));
 #pragma unroll
     for (int q = 0; q < kRowBins; q++) {
         const int k = jj + q * P.tj;
@@ -138,7 +138,7 @@ __device__ __forceinline__ void store_row_pair(const RowAddr &at, const LineFft 
 
 // x-forward of the white noise, drawn where it is transformed: the 2 n cells
 // of a row pair are n whole Threefry counter pairs
-template <bool FIVE>
+template <int M>
 __global__ void __launch_bounds__(512) k_rows_noise(SpecGeo g, LineFft P, float2 *__restrict__ out, uint64_t seed)
 {
     extern __shared__ float2 lds[];
@@ -159,12 +159,13 @@ __global__ void __launch_bounds__(512) k_rows_noise(SpecGeo g, LineFft P, float2
         }
     }
     __syncthreads();
-    line_fft<-1, FIVE>(at, P, jj);
+    float2 x[kLineEpt];
+    line_run<-1, M, true, true>(at, P, jj, x);
     if (r < rows) store_row_pair(at, P, g, out, r, two, jj);
 }
 
 // x-forward of a real field
-template <bool FIVE>
+template <int M>
 __global__ void __launch_bounds__(512) k_rows_real(SpecGeo g, LineFft P, const float *__restrict__ in, float2 *__restrict__ out)
 {
     extern __shared__ float2 lds[];
@@ -172,76 +173,49 @@ __global__ void __launch_bounds__(512) k_rows_real(SpecGeo g, LineFft P, const f
     const long long rows = (long long)n * n, r = 2 * ((long long)blockIdx.x * (blockDim.x / P.tj) + line);
     const RowAddr at(lds + line * row_pitch(n));
     const bool two = r + 1 < rows;
+    float2 x[kLineEpt] = {};
     if (r < rows) {
         const float *pa = in + r * n, *pb = two ? pa + n : pa;
-        float2 x[kLineEpt];
 #pragma unroll
         for (int q = 0; q < kLineEpt; q++) {
             const int e = min(jj + q * P.tj, n - 1);
             x[q] = make_float2(pa[e], pb[e]);
         }
-        line_put(at, P, jj, x);
     }
-    __syncthreads();
-    line_fft<-1, FIVE>(at, P, jj);
+    line_run<-1, M, false, true>(at, P, jj, x);
     if (r < rows) store_row_pair(at, P, g, out, r, two, jj);
 }
 
-// A workgroup's tile of columns: lines kx of one plane, stride between a
-// line's elements
-struct ColTile {
-    int l, jj, kx;  // kx up to the row's pitch: the padding is carried along
-};
-
-__device__ __forceinline__ ColTile col_tile(const SpecGeo &g, int logl)
-{
-    ColTile t;
-    t.l = threadIdx.x & ((1 << logl) - 1);
-    t.jj = threadIdx.x >> logl;
-    t.kx = (blockIdx.x << logl) + t.l;
-    return t;
-}
-
-// column kx of plane z of an array
-__device__ __forceinline__ Line32 plane_line(const SpecGeo &g, const float2 *s, int z, int kx)
-{
-    return Line32{(char *)(s + z * g.plane), 8u * (unsigned)kx, 8u * (unsigned)g.pitch};
-}
-
-// y-forward, in place: grid (tiles, kz or z planes)
-template <bool FIVE>
-__global__ void __launch_bounds__(1024) k_cols_y_fwd(SpecGeo g, LineFft P, int logl, float2 *__restrict__ s)
+// y-forward, in place: planes of kz or z
+template <int M>
+__global__ void __launch_bounds__(1024) k_cols_y_fwd(SpecGeo g, LineFft P, ColGrid C, float2 *__restrict__ s)
 {
     extern __shared__ float2 lds[];
-    const ColTile t = col_tile(g, logl);
-    const ColAddr at(lds, t.l, logl);
-    const Line32 io = plane_line(g, s, blockIdx.y, t.kx);
+    const ColTile t = col_tile(C);
+    if (t.plane < 0) return;
+    const ColAddr<M != kLineAny> at(lds, t.l, C.logl);
+    const LineY io(g, s, t.plane, 0, 1, t.kx);
     float2 x[kLineEpt];
     line_load(P, t.jj, x, io);
-    line_put(at, P, t.jj, x);
-    __syncthreads();
-    line_fft<-1, FIVE>(at, P, t.jj);
-    line_store(at, P, t.jj, io);
+    line_run<-1, M, false, false>(at, P, t.jj, x);
+    line_store(P, t.jj, x, io);
 }
 
 // z-forward, transfer, z-inverse: one read of the spectrum gives every
 // output.  The mode X (times its amplitude with A.amp) stays in registers
 // while the outputs are formed one after the other in LDS.
-template <bool FIVE>
-__global__ void __launch_bounds__(1024) k_cols_z(SpecGeo g, LineFft P, int logl, ZArgs A)
+template <int M>
+__global__ void __launch_bounds__(1024) k_cols_z(SpecGeo g, LineFft P, ColGrid C, ZArgs A)
 {
 #pragma clang fp contract(off)
     extern __shared__ float2 lds[];
-    const ColTile t = col_tile(g, logl);
-    const ColAddr at(lds, t.l, logl);
-    const int n = g.n, iy = blockIdx.y, half = n / 2;
-    const long long base = (long long)iy * g.pitch + t.kx;
+    const ColTile t = col_tile(C);
+    if (t.plane < 0) return;
+    const ColAddr<M != kLineAny> at(lds, t.l, C.logl);
+    const int n = g.n, iy = t.plane, half = n / 2;
     float2 X[kLineEpt];
-    line_load(P, t.jj, X, Line64{(char *)(A.in + base), 8 * g.plane});
-    line_put(at, P, t.jj, X);
-    __syncthreads();
-    line_fft<-1, FIVE>(at, P, t.jj);
-    line_get(at, P, t.jj, X);
+    line_load(P, t.jj, X, LineZ(g, A.in, iy, t.kx));
+    line_run<-1, M, false, false>(at, P, t.jj, X);
     const int kx = min(t.kx, g.nk - 1), fy = iy < (n + 1) / 2 ? iy : iy - n, ixy = kx * kx + fy * fy;
     const bool nyq_xy = kx == g.nk - 1 || iy == half;
     float ik[kLineEpt];  // scale / k^2
@@ -259,7 +233,7 @@ __global__ void __launch_bounds__(1024) k_cols_z(SpecGeo g, LineFft P, int logl,
         const int kind = A.out[o].kind, nyq = A.out[o].nyq;
         int jj = t.jj;
         asm volatile("" : "+v"(jj));  // per-element values are formed anew, not held for every output
-        __syncthreads();
+        float2 x[kLineEpt];
 #pragma unroll
         for (int q = 0; q < kLineEpt; q++) {
             const int e = jj + q * P.tj, fz = e < (n + 1) / 2 ? e : e - n;
@@ -278,11 +252,10 @@ __global__ void __launch_bounds__(1024) k_cols_z(SpecGeo g, LineFft P, int logl,
                 f = kind == Z_INV ? ik[q] : kind == Z_INV_Z ? ik[q] * kz : ik[q] * kz * kz;
             }
             if (nyq && (nyq_xy || e == half)) f = 0.f;
-            if (e < n) at(e) = make_float2(X[q].x * f, X[q].y * f);
+            x[q] = make_float2(X[q].x * f, X[q].y * f);
         }
-        __syncthreads();
-        line_fft<1, FIVE>(at, P, jj);
-        line_store(at, P, jj, Line64{(char *)(A.out[o].p + base), 8 * g.plane});
+        line_run<1, M, false, false>(at, P, jj, x);
+        line_store(P, jj, x, LineZ(g, A.out[o].p, iy, t.kx));
     }
 }
 
@@ -319,33 +292,33 @@ __global__ void __launch_bounds__(1024) k_pk_log(const double *__restrict__ k, c
     }
 }
 
-// y-inverse of the arrays of Y, each times the powers of ky asked for: grid
-// (tiles, z planes, arrays); an output may be its input
-template <bool FIVE>
-__global__ void __launch_bounds__(1024) k_cols_y_inv(SpecGeo g, LineFft P, int logl, YArgs Y)
+// y-inverse of the arrays of Y, each times the powers of ky asked for:
+// z planes, grid y the arrays; an output may be its input
+template <int M>
+__global__ void __launch_bounds__(1024, M == kLineReg ? 8 : 4) k_cols_y_inv(SpecGeo g, LineFft P, ColGrid C, YArgs Y)
 {
     extern __shared__ float2 lds[];
-    const ColTile t = col_tile(g, logl);
-    const ColAddr at(lds, t.l, logl);
-    const YArgs::Arr &R = Y.arr[blockIdx.z];
+    const ColTile t = col_tile(C);
+    if (t.plane < 0) return;
+    const ColAddr<M != kLineAny> at(lds, t.l, C.logl);
+    const YArgs::Arr &R = Y.arr[blockIdx.y];
     const int n = g.n;
     float2 X[kLineEpt];
-    line_load(P, t.jj, X, plane_line(g, R.in, blockIdx.y, t.kx));
+    line_load(P, t.jj, X, LineY(g, R.in, t.plane, 0, 1, t.kx));
     for (int o = 0; o < 3; o++) {
         float2 *w = R.out[o];  // ky^o
         if (!w) continue;
         int jj = t.jj;
         asm volatile("" : "+v"(jj));
-        __syncthreads();
+        float2 x[kLineEpt];
 #pragma unroll
         for (int q = 0; q < kLineEpt; q++) {
             const int e = jj + q * P.tj;
             const float ky = (float)(e < (n + 1) / 2 ? e : e - n) * Y.mult, f = o == 0 ? 1.f : o == 1 ? ky : ky * ky;
-            if (e < n) at(e) = make_float2(X[q].x * f, X[q].y * f);
+            x[q] = make_float2(X[q].x * f, X[q].y * f);
         }
-        __syncthreads();
-        line_fft<1, FIVE>(at, P, jj);
-        line_store(at, P, jj, plane_line(g, w, blockIdx.y, t.kx));
+        line_run<1, M, false, false>(at, P, jj, x);
+        line_store(P, jj, x, LineY(g, w, t.plane, 0, 1, t.kx));
     }
 }
 
@@ -355,8 +328,7 @@ __device__ __forceinline__ void load_row_pair(const RowAddr &at, const LineFft &
                                               float f, float mult)
 {
     const long long z = r / g.n, z2 = (r + 1) / g.n;
-    const float2 *a = in + z * g.plane + (r - z * g.n) * g.pitch,
-                 *b = in + z2 * g.plane + (r + 1 - z2 * g.n) * g.pitch;
+    const float2 *a = in + g.row((int)z, (int)(r - z * g.n)), *b = in + g.row((int)z2, (int)(r + 1 - z2 * g.n));
     float2 va[kRowBins], vb[kRowBins];
 #pragma unroll
     for (int q = 0; q < kRowBins; q++) {
@@ -376,7 +348,7 @@ __device__ __forceinline__ void load_row_pair(const RowAddr &at, const LineFft &
 }
 
 // x-inverse: grid (row pairs, outputs)
-template <bool FIVE>
+template <int M>
 __global__ void __launch_bounds__(512) k_rows_inv(SpecGeo g, LineFft P, XArgs X)
 {
     extern __shared__ float2 lds[];
@@ -387,10 +359,9 @@ __global__ void __launch_bounds__(512) k_rows_inv(SpecGeo g, LineFft P, XArgs X)
     const XArgs::Op &O = X.op[blockIdx.y];
     if (r < rows) load_row_pair(at, P, g, O.in, r, two, jj, O.pow, O.imag, O.f, X.mult);
     __syncthreads();
-    line_fft<1, FIVE>(at, P, jj);
+    float2 x[kLineEpt];
+    line_run<1, M, true, false>(at, P, jj, x);
     if (r < rows) {
-        float2 x[kLineEpt];
-        line_get(at, P, jj, x);
         float *pa = O.out + r * n, *pb = pa + n;
 #pragma unroll
         for (int q = 0; q < kLineEpt; q++) {
@@ -409,7 +380,7 @@ __global__ void __launch_bounds__(512) k_rows_inv(SpecGeo g, LineFft P, XArgs X)
 // in the potentials, whose common sign is left out.  delta: null for
 // run_tile's source p11 p22 + (p11 + p22) p33 - p12^2 - p13^2 - p23^2, else
 // the split tiles' delta^2 / 2 - sum phi_dd^2 / 2 - sum phi_ab^2, in Float32.
-template <bool FIVE>
+template <int M>
 __global__ void __launch_bounds__(512) k_rows_src(SpecGeo g, LineFft P, SrcArgs S)
 {
 #pragma clang fp contract(off)
@@ -434,10 +405,11 @@ __global__ void __launch_bounds__(512) k_rows_src(SpecGeo g, LineFft P, SrcArgs 
         __syncthreads();
         if (live) load_row_pair(at, P, g, S.in[v], r, two, j2, S.pow[v], false, 1.f, S.mult);
         __syncthreads();
-        line_fft<1, FIVE>(at, P, j2);
+        float2 x[kLineEpt];
+        line_run<1, M, true, false>(at, P, j2, x);
 #pragma unroll
         for (int q = 0; q < kLineEpt; q++) {
-            const float2 p = at(min(j2 + q * P.tj, n - 1));
+            const float2 p = x[q];
             if (S.delta || v >= 3) {
                 const float co = v < 3 ? 0.5f : 1.0f;
                 src[q].x = src[q].x - (p.x * p.x) * co;
@@ -449,14 +421,11 @@ __global__ void __launch_bounds__(512) k_rows_src(SpecGeo g, LineFft P, SrcArgs 
             }
         }
     }
-    __syncthreads();
+    if (!two) {
 #pragma unroll
-    for (int q = 0; q < kLineEpt; q++) {
-        const int e = jj + q * P.tj;
-        if (e < n) at(e) = two ? src[q] : make_float2(src[q].x, 0.f);
+        for (int q = 0; q < kLineEpt; q++) src[q].y = 0.f;
     }
-    __syncthreads();
-    line_fft<-1, FIVE>(at, P, jj);
+    line_run<-1, M, false, true>(at, P, jj, src);
     if (live) store_row_pair(at, P, g, S.out, r, two, jj);
 }
 
@@ -477,7 +446,7 @@ int grid_plan(pp_ctx *ctx, int n, GridPlan *G)
     // (16 columns of a long line) share a CU; the z pass and the radices 5 and
     // 7 take more and keep to 512 threads
     G->ycol = G->col;
-    G->ys = col_shape(G->ycol, G->col.five ? 512 : 1024);
+    G->ys = col_shape(G->ycol, G->col.mode == kLineReg ? 1024 : 512);
     G->g = spec_geo(n, n);
     G->stream = ctx->stream;
     return PP_OK;
@@ -499,22 +468,23 @@ int rows_noise(const GridPlan &G, uint64_t seed, float2 *out)
 
 int cols_y_fwd(const GridPlan &G, float2 *s)
 {
-    PP_LINE_LAUNCH(G.ycol, k_cols_y_fwd, dim3(G.ys.tiles(G.g.nk), G.g.n), dim3(G.ys.block), G.ys.lds, G.stream, G.g,
-                       G.ycol, G.ys.logl, s);
+    const ColGrid C = G.ys.grid(G.g.nk, G.g.n, 1);
+    PP_LINE_LAUNCH(G.ycol, k_cols_y_fwd, dim3(C.blocks()), dim3(G.ys.block), G.ys.lds, G.stream, G.g, G.ycol, C, s);
     return PP_OK;
 }
 
 int cols_z(const GridPlan &G, const ZArgs &A)
 {
-    PP_LINE_LAUNCH(G.col, k_cols_z, dim3(G.cs.tiles(G.g.nk), G.g.n), dim3(G.cs.block), G.cs.lds, G.stream, G.g, G.col,
-                       G.cs.logl, A);
+    const ColGrid C = G.cs.grid(G.g.nk, G.g.n, kColXCD);
+    PP_LINE_LAUNCH(G.col, k_cols_z, dim3(C.blocks()), dim3(G.cs.block), G.cs.lds, G.stream, G.g, G.col, C, A);
     return PP_OK;
 }
 
 int cols_y_inv(const GridPlan &G, const YArgs &Y)
 {
-    PP_LINE_LAUNCH(G.ycol, k_cols_y_inv, dim3(G.ys.tiles(G.g.nk), G.g.n, Y.narr), dim3(G.ys.block), G.ys.lds, G.stream,
-                       G.g, G.ycol, G.ys.logl, Y);
+    const ColGrid C = G.ys.grid(G.g.nk, G.g.n, 1);
+    PP_LINE_LAUNCH(G.ycol, k_cols_y_inv, dim3(C.blocks(), Y.narr), dim3(G.ys.block), G.ys.lds, G.stream, G.g,
+                   G.ycol, C, Y);
     return PP_OK;
 }
 
@@ -597,7 +567,7 @@ static int make_tile_lines(pp_ctx *ctx, int n, double boxsize, uint64_t seed, co
     const bool lpt2 = f->eta2x != nullptr;
     GridPlan G;
     PP_CHECK(grid_plan(ctx, n, &G));
-    const size_t arr = (size_t)G.g.plane * n;  // complex values of one array
+    const size_t arr = G.g.size(n);  // complex values of one array
     // delta / source, A', B', ky A', L, and with 2LPT A, B, C, ky A, ky^2 A, ky B
     const int narr = 4 + (f->lapd ? 1 : 0) + (lpt2 ? 6 : 0);
     PP_CHECK(ctx->d_spec.grow(arr * narr * sizeof(float2)));

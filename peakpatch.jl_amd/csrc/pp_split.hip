@@ -14,25 +14,25 @@
 //   coarse cell, each lane walking counter pairs along rows (one Threefry
 //   block gives both normals of a pair), Float64 partial sums reduced in a
 //   fixed tree;
-// * the residual is written straight into the zero-padded real buffer of an
-//   in-place (2n)^3 rocFFT transform (rows padded to 2 (n+1) floats), two
-//   cells per lane.  (Transforming only the planes that hold data, with the
-//   z axis as a separate strided 1-D pass, measured slower: rocFFT's strided
-//   1-D z pass costs more than its whole 3-D plan saves.);
-// * each output's spectrum is one pass over the base spectrum that forms the
-//   Float64 transfer factor, rounds the product into ComplexF32 once and,
-//   on the kx = 0 and kx = Nyquist planes, averages the mode with its
-//   conjugate partner (computed by the same lane);
-// * the inverse transform runs in place; one pass then cuts the tile out of
-//   the padded result, applies the Float32 1/(2n)^3 of the normalised
-//   inverse and adds the coarse field's 64-tap Catmull-Rom interpolation in
-//   the reference's Float32 order;
+// * the isolated convolution of the residual runs on line transforms
+//   (pp_fft.h) that never store the zero padding: the noise is drawn in the x
+//   pass, the transfer functions sit between the forward and the inverse
+//   transform of the z pass, and the last pass cuts the tile out and adds the
+//   coarse field's Catmull-Rom interpolation, contracted along y and z once
+//   per row;
+// * meshes without a line transform (odd, or with a prime factor above 7) go
+//   through an in-place (2n)^3 rocFFT transform of the padded residual (rows
+//   padded to 2 (n+1) floats), one pass over the base spectrum per output
+//   (Float64 transfer factor, the kx = 0 and Nyquist planes averaged with
+//   their conjugate partners) and one pass that cuts and interpolates with
+//   64 taps a cell;
 // * 2LPT: the source is accumulated in real space in the reference's order,
 //   one potential at a time (two spectra and two real fields resident).
 #include <cmath>
 #include <vector>
 
 #include "pp_common.h"
+#include "pp_fields.h"
 #include "pp_kspace.h"
 #include "pp_noise.h"
 
@@ -41,8 +41,8 @@ struct pp_coarse {
     pp_split_geom g{};
     int N = 0, nsub = 0, block = 0, npk = 0;
     double boxsize_full = 0;
-    double lk0 = 0, inv_dlk = 0;  // the P(k) table's first log k and 1 / spacing when even
-    pp::DevBuf noise, delta, psi, pk;  // M^3 floats; 3 M^3 floats; log k, log P
+    pp::DevBuf noise, delta, psi, pk;  // M^3 floats; 3 M^3 floats; the P(k) table
+    pp::PkLog table{};                 // its logarithms, in pk
 };
 
 namespace pp {
@@ -94,9 +94,7 @@ struct Xfer {
     int nyq_zero;  // zero k = 0's partners on the Nyquist planes (_apply_kernel_inplace!)
     int herm;      // average the kx = 0 / kx = Nyquist planes with their conjugate partners
     double dk3, n3;  // dk^3 and n^3 of the amplitude sqrt((P(k) dk^3) n^3)
-    const double *lk, *lp;
-    int np;
-    double lk0, inv_dlk;  // evenly spaced table: first log k and 1 / spacing (0: bisection)
+    PkLog T;
 };
 
 // the mode at (ix, iy, iz) times its transfer factor, rounded to ComplexF32
@@ -112,11 +110,11 @@ __device__ __forceinline__ float2 xfer_mode(const Xfer &X, const float2 *__restr
     const float2 v = src[ix + (long long)g.nk * (iy + (long long)g.n * iz)];
     switch (X.mode) {
     case XF_AMP: {
-        const double amp = sqrt(pk_eval(X.lk, X.lp, X.np, sqrt(k2), X.lk0, X.inv_dlk) * X.dk3 * X.n3);
+        const double amp = sqrt(pk_eval(X.T.lk, X.T.lp, X.T.np, sqrt(k2), X.T.even[0], X.T.even[1]) * X.dk3 * X.n3);
         return cmul(v, amp, 0.0);
     }
     case XF_AMP_IK: {
-        const double amp = sqrt(pk_eval(X.lk, X.lp, X.np, sqrt(k2), X.lk0, X.inv_dlk) * X.dk3 * X.n3);
+        const double amp = sqrt(pk_eval(X.T.lk, X.T.lp, X.T.np, sqrt(k2), X.T.even[0], X.T.even[1]) * X.dk3 * X.n3);
         return cmul(v, 0.0, amp * (k[X.a] / k2));
     }
     case XF_PHI:
@@ -304,6 +302,450 @@ __global__ void __launch_bounds__(256) k_src_sub(float *__restrict__ src, const 
     }
 }
 
+// ------------------------------------------------- isolated convolution
+// The zero-padded transform of the residual with line transforms
+// (pp_fft.h).  Half of every padded line is zero and half of every result is
+// cut away, so a line of 2 n is two of n and no padding is ever stored or
+// read: with w = exp(-i pi / n),
+//   X[2 m]     = FFT_n(x)[m],        X[2 m + 1] = FFT_n(x w^j)[m],
+//   y[j], j < n = IFFT_n(X[2 m])[j] + w^-j IFFT_n(X[2 m + 1])[j].
+// A spectrum holds n z planes (real space along z) of 2 n rows.  The z pass
+// transforms forward, applies the transfer and transforms back while a
+// column is in LDS, so the (2 n)^3 spectrum never exists in memory; ky A goes to
+// the upper half of A's rows, which the cut leaves free.  delta, psi_x, psi_y
+// and psi_z come from the three arrays X, X / k^2 and kz X / k^2.  Traffic at
+// n = 512: 30 GB in place of 170.
+constexpr int kLineCoarse = 512;  // coarse cells a side whose rows fit LDS beside a line
+struct PadGeo {
+    int n;
+    SpecGeo g;  // nk = n + 1 bins, 2 n rows a plane
+};
+
+// half h (0 even, 1 odd bins) of the transform of x
+template <int M, bool OUT_LDS, class A>
+__device__ __forceinline__ void pad_forward(const A &at, const LineFft &P, int jj, const float2 x[kLineEpt],
+                                            float2 X[kLineEpt], int h)
+{
+#pragma unroll
+    for (int q = 0; q < kLineEpt; q++) X[q] = h ? fmul(x[q], P.half[min(jj + q * P.tj, P.n - 1)]) : x[q];
+    line_run<-1, M, false, OUT_LDS>(at, P, jj, X);
+}
+
+// y (+)= the inverse of half h: in x, or in LDS
+template <int M, bool IN_LDS, class A>
+__device__ __forceinline__ void pad_inverse(const A &at, const LineFft &P, int jj, float2 x[kLineEpt],
+                                            float2 y[kLineEpt], int h)
+{
+    line_run<1, M, IN_LDS, false>(at, P, jj, x);
+#pragma unroll
+    for (int q = 0; q < kLineEpt; q++)
+        y[q] = h ? fadd(y[q], fmulc(x[q], P.half[min(jj + q * P.tj, P.n - 1)])) : x[q];
+}
+
+// Residual of a row pair drawn into its line: fine normal minus coarse block
+// mean.  A thread takes two cells of one Threefry counter pair where the row's
+// parity and the wrap allow it.
+__device__ __forceinline__ void residual_row(float *line, const TileGeo &T, const float *__restrict__ coarse, int y,
+                                             int z, int jj, int tj)
+{
+    const int gy = wrap1(T.j0 + y, T.N), gz = wrap1(T.k0 + z, T.N);
+    const long long rowb = ((long long)gy + (long long)gz * T.N) * T.N;
+    const float *crow = coarse + (long long)T.M * (gy / T.b + (long long)T.M * (gz / T.b));
+    const int par = (int)((wrap1(T.i0, T.N) + rowb) & 1);
+    for (int m = jj; 2 * m - par < T.n; m += tj) {
+        long long last = -1;
+        double g1 = 0, g2 = 0;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int x = 2 * m - par + h;
+            if (x < 0 || x >= T.n) continue;
+            const int gx = wrap1(T.i0 + x, T.N);
+            const long long idx = gx + rowb, pr = idx >> 1;
+            if (pr != last) {
+                threefry_normals((uint64_t)pr, T.seed, g1, g2);
+                last = pr;
+            }
+            const float fine = (float)((idx & 1) ? g2 : g1), cm = crow[gx / T.b];
+            line[2 * (x + (x >> 3))] = fine - cm * T.inv_b3;
+        }
+    }
+}
+
+// x-forward of the residual
+template <int M>
+__global__ void __launch_bounds__(512) k_pad_rows_noise(PadGeo G, LineFft P, TileGeo T,
+                                                        const float *__restrict__ coarse, float2 *__restrict__ out)
+{
+    extern __shared__ float2 lds[];
+    const int n = G.n, line = threadIdx.x / P.tj, jj = threadIdx.x - line * P.tj;
+    const long long rows = (long long)n * n, r = 2 * ((long long)blockIdx.x * (blockDim.x / P.tj) + line);
+    float2 *row = lds + line * row_pitch(n);
+    const RowAddr at(row);
+    const bool live = r < rows, two = r + 1 < rows;
+    const int z = (int)(r / n), y = (int)(r - (long long)z * n), z2 = (int)((r + 1) / n),
+              y2 = (int)(r + 1 - (long long)z2 * n);
+    if (live) residual_row((float *)row, T, coarse, y, z, jj, P.tj);
+    if (two) residual_row((float *)row + 1, T, coarse, y2, z2, jj, P.tj);  // n is even, and so are the rows
+    __syncthreads();
+    float2 x[kLineEpt];
+    line_get(at, P, jj, x);
+    float2 *a = out + G.g.row(z, y), *b = out + G.g.row(z2, y2);
+#pragma nounroll
+    for (int h = 0; h < 2; h++) {
+        int j2 = jj;
+        asm volatile("" : "+v"(j2));
+        float2 X[kLineEpt];
+        pad_forward<M, true>(at, P, j2, x, X, h);
+        if (!live) continue;
+#pragma unroll
+        for (int q = 0; q < kRowBins; q++) {
+            const int m = j2 + q * P.tj, k = 2 * m + h;
+            if (k > n) break;
+            float2 va, vb;
+            split_rows(at(m), at(h ? n - 1 - m : (m == 0 ? 0 : n - m)), va, vb);
+            a[k] = va;
+            if (two) b[k] = vb;
+        }
+    }
+}
+
+// y-forward, in place: n rows in, 2 n out
+template <int M>
+__global__ void __launch_bounds__(1024) k_pad_cols_y_fwd(PadGeo G, LineFft P, ColGrid C, float2 *__restrict__ s)
+{
+    extern __shared__ float2 lds[];
+    const ColTile t = col_tile(C);
+    if (t.plane < 0) return;
+    const int jj = t.jj, kx = t.kx;
+    const ColAddr<M != kLineAny> at(lds, t.l, C.logl);
+    float2 x[kLineEpt];
+    line_load(P, jj, x, LineY(G.g, s, t.plane, 0, 1, kx));
+#pragma nounroll
+    for (int h = 0; h < 2; h++) {
+        int j2 = jj;
+        asm volatile("" : "+v"(j2));
+        float2 X[kLineEpt];
+        pad_forward<M, false>(at, P, j2, x, X, h);
+        line_store(P, j2, X, LineY(G.g, s, t.plane, h, 2, kx));
+    }
+}
+
+struct PadZ {
+    const float2 *in;
+    float2 *out[3];    // X, X / k^2, kz X / k^2
+    const float *amp;  // by integer |k|^2
+    float mult, scale, inv;
+};
+
+// z-forward, transfer, z-inverse
+template <int M>
+__global__ void __launch_bounds__(1024) k_pad_cols_z(PadGeo G, LineFft P, ColGrid C, PadZ A)
+{
+    extern __shared__ float2 lds[];
+    const ColTile t = col_tile(C);
+    if (t.plane < 0) return;
+    const int jj0 = t.jj, kxp = t.kx;
+    const ColAddr<M != kLineAny> at(lds, t.l, C.logl);
+    const int n = G.n, iy = t.plane, fy = iy < n ? iy : iy - 2 * n, kx = min(kxp, n), ixy = kx * kx + fy * fy;
+    float2 X[2][kLineEpt];
+    {
+        float2 x[kLineEpt];
+        line_load(P, jj0, x, LineZ(G.g, A.in, iy, kxp));
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            pad_forward<M, false>(at, P, jj0, x, X[h], h);
+#pragma unroll
+            for (int q = 0; q < kLineEpt; q++) {
+                const int e = 2 * min(jj0 + q * P.tj, n - 1) + h, fz = e < n ? e : e - 2 * n;
+                const float a = A.amp[ixy + fz * fz];
+                X[h][q] = make_float2(X[h][q].x * a, X[h][q].y * a);
+            }
+        }
+    }
+    for (int o = 0; o < 3; o++) {
+        int jj = jj0;
+        asm volatile("" : "+v"(jj));
+        float2 y[kLineEpt];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            float2 x[kLineEpt];
+#pragma unroll
+            for (int q = 0; q < kLineEpt; q++) {
+                const int e = jj + q * P.tj, k = 2 * e + h, fz = k < n ? k : k - 2 * n, i2 = ixy + fz * fz;
+                float f = A.scale;
+                if (o > 0) {
+                    const float d = (float)i2, r = __builtin_amdgcn_rcpf(d);
+                    f = i2 == 0 ? 0.f : A.inv * __builtin_fmaf(__builtin_fmaf(-d, r, 1.f), r, r);
+                    if (o == 2) f = f * ((float)fz * A.mult);
+                }
+                x[q] = make_float2(X[h][q].x * f, X[h][q].y * f);
+            }
+            pad_inverse<M, false>(at, P, jj, x, y, h);
+        }
+        line_store(P, jj, y, LineZ(G.g, A.out[o], iy, kxp));
+    }
+}
+
+struct PadY {
+    float2 *s[3];
+    int nvar[3];  // 1, or 2: times ky too, to rows n .. 2 n - 1
+    float mult;
+};
+
+// y-inverse, in place: 2 n rows in, n (per power of ky) out
+template <int M>
+__global__ void __launch_bounds__(1024) k_pad_cols_y_inv(PadGeo G, LineFft P, ColGrid C, PadY A)
+{
+    extern __shared__ float2 lds[];
+    const ColTile t = col_tile(C);
+    if (t.plane < 0) return;
+    const int jj0 = t.jj, kx = t.kx;
+    const ColAddr<M != kLineAny> at(lds, t.l, C.logl);
+    const int n = G.n;
+    float2 *s = A.s[blockIdx.y];
+    float2 X[2][kLineEpt];
+#pragma unroll
+    for (int h = 0; h < 2; h++) line_load(P, jj0, X[h], LineY(G.g, s, t.plane, h, 2, kx));
+    for (int o = 0; o < A.nvar[blockIdx.y]; o++) {
+        int jj = jj0;
+        asm volatile("" : "+v"(jj));
+        float2 y[kLineEpt];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            float2 x[kLineEpt];
+#pragma unroll
+            for (int q = 0; q < kLineEpt; q++) {
+                const int e = jj + q * P.tj, k = 2 * e + h;
+                const float f = o == 0 ? 1.f : (float)(k < n ? k : k - 2 * n) * A.mult;
+                x[q] = make_float2(X[h][q].x * f, X[h][q].y * f);
+            }
+            pad_inverse<M, false>(at, P, jj, x, y, h);
+        }
+        const LineY w(G.g, s, t.plane, o * n, 1, kx);
+        line_store(P, jj, y, w);
+    }
+}
+
+struct PadX {
+    struct Op {
+        const float2 *in;
+        int row0;       // first row of the plane
+        int imag, pow;  // factor 1, i or i kx
+        const float *coarse;
+        float *out;
+    } op[4];
+    float mult;
+};
+
+// Coarse row of tile row (y, z): the sum over the 4 x 4 taps along y and z,
+// after which a cell takes four taps along x instead of 64
+__device__ __forceinline__ void coarse_row(float *rc, const TileGeo &T, const float *__restrict__ coarse, int y, int z,
+                                           int jj, int tj)
+{
+    int by, bz;
+    float ty, tz, wy[4], wz[4];
+    cr_coord(wrap1(T.j0 + y, T.N), T.b, by, ty);
+    cr_coord(wrap1(T.k0 + z, T.N), T.b, bz, tz);
+    cr_weights(ty, wy);
+    cr_weights(tz, wz);
+    for (int i = jj; i < T.M; i += tj) {
+        float v = 0.f;
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const long long row = wrap1(by + q - 2, T.M) + (long long)T.M * wrap1(bz + c - 2, T.M);
+                v += (wy[q] * wz[c]) * coarse[i + T.M * row];
+            }
+        rc[i] = v;
+    }
+}
+
+// x-inverse of the row pairs, plus the interpolated coarse field
+template <int M>
+__global__ void __launch_bounds__(512) k_pad_rows_inv(PadGeo G, LineFft P, TileGeo T, PadX A)
+{
+    extern __shared__ float2 lds[];
+    const int n = G.n, lines = blockDim.x / P.tj, line = threadIdx.x / P.tj, jj = threadIdx.x - line * P.tj;
+    const long long rows = (long long)n * n, r = 2 * ((long long)blockIdx.x * lines + line);
+    const RowAddr at(lds + line * row_pitch(n));
+    float *rc = (float *)(lds + lines * row_pitch(n)) + (size_t)line * 2 * T.M;
+    const bool live = r < rows, two = r + 1 < rows;
+    const PadX::Op &O = A.op[blockIdx.y];
+    const int z = (int)(r / n), y = (int)(r - (long long)z * n), z2 = (int)((r + 1) / n),
+              y2 = (int)(r + 1 - (long long)z2 * n);
+    const float2 *a = O.in + G.g.row(z, O.row0 + y), *b = O.in + G.g.row(z2, O.row0 + y2);
+    if (live) coarse_row(rc, T, O.coarse, y, z, jj, P.tj);
+    if (two) coarse_row(rc + T.M, T, O.coarse, y2, z2, jj, P.tj);
+    float2 v[kLineEpt];
+#pragma nounroll
+    for (int h = 0; h < 2; h++) {
+        int j2 = jj;
+        asm volatile("" : "+v"(j2));
+        __syncthreads();
+        if (live) {
+            float2 va[kRowBins], vb[kRowBins];
+#pragma unroll
+            for (int q = 0; q < kRowBins; q++) {
+                const int k = min(2 * (j2 + q * P.tj) + h, n);
+                va[q] = a[k];
+                vb[q] = two ? b[k] : make_float2(0.f, 0.f);
+            }
+#pragma unroll
+            for (int q = 0; q < kRowBins; q++) {
+                const int m = j2 + q * P.tj, k = 2 * m + h;
+                if (k > n) break;
+                const float c = O.pow ? (float)k * A.mult : 1.f;
+                const float2 p = va[q], s = vb[q];
+                const float2 f1 = O.imag ? make_float2(-c * p.y, c * p.x) : make_float2(c * p.x, c * p.y),
+                             f2 = O.imag ? make_float2(-c * s.y, c * s.x) : make_float2(c * s.x, c * s.y);
+                const int mc = h ? n - 1 - m : (m == 0 ? 0 : n - m);
+                if (k == 0 || k == n) {  // real bins (mc = m)
+                    at(m) = make_float2(f1.x, f2.x);
+                } else {
+                    at(m) = make_float2(f1.x - f2.y, f1.y + f2.x);
+                    at(mc) = make_float2(f1.x + f2.y, f2.x - f1.y);
+                }
+            }
+        }
+        __syncthreads();
+        float2 x[kLineEpt];
+        pad_inverse<M, true>(at, P, j2, x, v, h);
+    }
+    if (!live) return;
+    float *pa = O.out + r * n, *pb = pa + n;
+    const unsigned b2 = 2u * (unsigned)T.b;
+    const float ib2 = 1.f / (float)b2;
+#pragma unroll
+    for (int q = 0; q < kLineEpt; q++) {
+        const int e = jj + q * P.tj;
+        if (e >= n) break;
+        // the base cell and fraction of (g + 1/2) / b + 1/2 (cr_coord), in integers
+        const unsigned num = 2u * (unsigned)wrap1(T.i0 + e, T.N) + 1u + (unsigned)T.b, i = num / b2;
+        float w[4];
+        cr_weights((float)(num - i * b2) * ib2, w);
+        float c1 = 0.f, c2 = 0.f;
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const int c = wrap1((int)i + t - 2, T.M);
+            c1 += w[t] * rc[c];
+            c2 += w[t] * rc[T.M + c];
+        }
+        pa[e] = v[q].x + c1;
+        if (two) pb[e] = v[q].y + c2;
+    }
+}
+
+// pp_split_tile_fields with line transforms
+static int split_tile_lines(pp_ctx *ctx, const pp_coarse *c, const TileGeo &T, pp_tile_fields *f)
+{
+    const pp_split_geom &G = c->g;
+    const int n = G.nmesh, M = G.M;
+    const long long n3 = (long long)n * n * n, M3 = (long long)M * M * M;
+    const bool lpt2 = f->eta2x != nullptr;
+    GridPlan D;
+    PP_CHECK(grid_plan(ctx, n, &D));
+    PadGeo Q;
+    Q.n = n;
+    Q.g = spec_geo(2 * n, 2 * n);
+    // three padded spectra; then, in their place, those of the tile's grid.
+    // Stream ordered and returned when the tile's fields are written, so a
+    // context does not keep them between tiles
+    const size_t pad = Q.g.size(n), arr = D.g.size(n);
+    const int narr = 1 + (f->lapd ? 1 : 0) + (lpt2 ? 6 : 0);  // source or delta, then A .. ky B; L last
+    const size_t need = std::max(3 * pad, (size_t)narr * arr) * sizeof(float2);
+    void *arena = nullptr;
+    hipError_t ea = hipMallocAsync(&arena, need, ctx->stream);
+    if (ea != hipSuccess) {
+        set_error("hipMallocAsync of %zu B: %s", need, hipGetErrorString(ea));
+        return ea == hipErrorOutOfMemory ? PP_ERR_OOM : PP_ERR_HIP;
+    }
+    struct Release {
+        hipStream_t s;
+        void *p;
+        ~Release() { (void)hipFreeAsync(p, s); }
+    } release{ctx->stream, arena};
+    const long long count = amp_count(n);
+    PP_CHECK(ctx->d_misc.grow(count * sizeof(float)));
+    float *amp = ctx->d_misc.as<float>();
+    const int n2 = 2 * n;
+    const double dx = (double)G.nmesh * G.alatt / n, dki = 2.0 * M_PI / (n2 * dx), mi = ((double)n2 * dki) / (double)n2;
+    const double pad3 = (double)n2 * n2 * n2;
+    PP_CHECK(amp_table(ctx, c->table, mi, dki * dki * dki, pad3, count, amp));
+    float2 *s[3];
+    for (int q = 0; q < 3; q++) s[q] = (float2 *)arena + pad * q;
+    const long long pairs = ((long long)n * n + 1) / 2;
+    const dim3 rgrid((unsigned)((pairs + D.rs.nl - 1) / D.rs.nl)), rblock(D.rs.block);
+    const ColGrid cy = D.cs.grid(Q.g.nk, n, 1), cz = D.cs.grid(Q.g.nk, 2 * n, kColXCD);
+    const dim3 gy(cy.blocks()), gz(cz.blocks()), cblock(D.cs.block);
+    PP_LINE_LAUNCH(D.row, k_pad_rows_noise, rgrid, rblock, D.rs.lds, ctx->stream, Q, D.row, T, c->noise.as<float>(),
+                   s[0]);
+    PP_LINE_LAUNCH(D.col, k_pad_cols_y_fwd, gy, cblock, D.cs.lds, ctx->stream, Q, D.col, cy, s[0]);
+    PadZ Z{s[0], {s[0], s[1], s[2]}, amp, (float)mi, (float)(1.0 / pad3), (float)(1.0 / pad3 / (mi * mi))};
+    PP_LINE_LAUNCH(D.col, k_pad_cols_z, gz, cblock, D.cs.lds, ctx->stream, Q, D.col, cz, Z);
+    PadY Y{{s[0], s[1], s[2]}, {1, 2, 1}, (float)mi};
+    PP_LINE_LAUNCH(D.col, k_pad_cols_y_inv, dim3(gy.x, 3), cblock, D.cs.lds, ctx->stream, Q, D.col, cy, Y);
+    PadX X{};
+    X.mult = (float)mi;
+    const float *psi = c->psi.as<float>();
+    X.op[0] = PadX::Op{s[0], 0, 0, 0, c->delta.as<float>(), f->delta};
+    X.op[1] = PadX::Op{s[1], 0, 1, 1, psi, f->etax};
+    X.op[2] = PadX::Op{s[1], n, 1, 0, psi + M3, f->etay};
+    X.op[3] = PadX::Op{s[2], 0, 1, 0, psi + 2 * M3, f->etaz};
+    const size_t rlds = D.rs.lds + (size_t)D.rs.nl * 2 * M * sizeof(float);
+    PP_LINE_LAUNCH(D.row, k_pad_rows_inv, dim3(rgrid.x, 4), rblock, rlds, ctx->stream, Q, D.row, T, X);
+    if (!lpt2 && !f->lapd) {
+        PP_HIP(hipStreamSynchronize(ctx->stream));
+        return PP_OK;
+    }
+    // the tile-periodic k^2 and 2LPT fields from the combined delta
+    float2 *t[8];
+    for (int q = 0; q < narr; q++) t[q] = (float2 *)arena + arr * q;
+    float2 *L = f->lapd ? t[narr - 1] : nullptr;
+    const double dkt = 2.0 * M_PI / ((double)G.nmesh * G.alatt), mt = ((double)n * dkt) / (double)n;
+    PP_CHECK(rows_real(D, f->delta, t[0]));
+    PP_CHECK(cols_y_fwd(D, t[0]));
+    ZArgs Z2{};
+    Z2.in = t[0];
+    Z2.set(mt, 1.0 / (double)n3);
+    YArgs Y2{};
+    Y2.mult = (float)mt;
+    if (L) {
+        Z2.add(L, Z_K2, 1);
+        Y2.add(L, L, nullptr, nullptr);
+    }
+    if (lpt2) {
+        Z2.add(t[0], Z_INV, 1);
+        Z2.add(t[1], Z_INV_Z, 1);
+        Z2.add(t[2], Z_INV_ZZ, 1);
+        Y2.add(t[0], t[0], t[3], t[4]);
+        Y2.add(t[1], t[1], t[5], nullptr);
+        Y2.add(t[2], t[2], nullptr, nullptr);
+    }
+    PP_CHECK(cols_z(D, Z2));
+    PP_CHECK(cols_y_inv(D, Y2));
+    if (L) {
+        XArgs X2{};
+        X2.mult = (float)mt;
+        X2.add(L, f->lapd, 0, false, 1.f);
+        PP_CHECK(rows_inv(D, X2));
+    }
+    if (lpt2) {
+        float2 *src = t[6];
+        SrcArgs S{};
+        S.delta = f->delta;
+        S.mult = (float)mt;
+        S.out = src;
+        src_inputs(S, t[0], t[3], t[4], t[1], t[5], t[2]);
+        PP_CHECK(rows_src(D, S));
+        float2 *w[3] = {src, t[0], t[1]};
+        float *out[3] = {f->eta2x, f->eta2y, f->eta2z};
+        PP_CHECK(second_order(D, w, mt, 1.0 / (double)n3, out));
+    }
+    PP_HIP(hipStreamSynchronize(ctx->stream));
+    return PP_OK;
+}
+
 static int grid_for(pp_ctx *ctx, long long items)
 {
     return (int)std::max<long long>(1, std::min<long long>((items + 255) / 256, (long long)ctx->num_cu * 16));
@@ -329,13 +771,7 @@ static Xfer make_xfer(int n, double dk, int mode, int a, int b, int nyq_zero, co
     X.herm = 1;
     X.dk3 = dk * dk * dk;
     X.n3 = (double)n * n * n;
-    if (c) {
-        X.lk = c->pk.as<double>();
-        X.lp = X.lk + c->npk;
-        X.np = c->npk;
-        X.lk0 = c->lk0;
-        X.inv_dlk = c->inv_dlk;
-    }
+    if (c) X.T = c->table;
     return X;
 }
 
@@ -382,27 +818,16 @@ int pp_coarse_create(pp_ctx *ctx, const pp_split_geom *geom, const pp_pk_table *
     int rc = c->noise.grow(M3 * 4);
     if (rc == PP_OK) rc = c->delta.grow(M3 * 4);
     if (rc == PP_OK) rc = c->psi.grow(3 * M3 * 4);
-    if (rc == PP_OK) rc = c->pk.grow(2 * pk->npk * sizeof(double));
+    if (rc == PP_OK) rc = c->pk.grow(pk_log_doubles(pk->npk) * sizeof(double));
     if (rc != PP_OK) return fail(rc);
-    std::vector<double> lt(2 * pk->npk);
-    for (int q = 0; q < pk->npk; q++) {
-        lt[q] = log(pk->k[q]);
-        lt[pk->npk + q] = log(pk->P[q]);
-    }
-    c->lk0 = lt[0];
-    c->inv_dlk = pk_uniform_inv_spacing(lt.data(), pk->npk);
-    hipError_t e = hipMemcpyAsync(c->pk.ptr, lt.data(), lt.size() * sizeof(double), hipMemcpyHostToDevice,
-                                  ctx->stream);
-    if (e != hipSuccess) {
-        set_error("hipMemcpyAsync: %s", hipGetErrorString(e));
-        return fail(PP_ERR_HIP);
-    }
+    rc = pk_log_device(ctx, pk, c->pk.as<double>(), &c->table);
+    if (rc != PP_OK) return fail(rc);
     // 1. the coarse noise
     const int b = c->block;
     const double norm = sqrt((double)b * (double)b * (double)b);
     hipLaunchKernelGGL(k_coarse_noise, dim3((unsigned)std::min<long long>(M3, 1 << 20)), dim3(256), 0, ctx->stream,
                        c->noise.as<float>(), c->N, M, b, G.seed, norm);
-    e = hipGetLastError();
+    hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         set_error("k_coarse_noise: %s", hipGetErrorString(e));
         return fail(PP_ERR_HIP);
@@ -477,6 +902,19 @@ int pp_split_tile_fields(pp_ctx *ctx, const pp_coarse *c, int it, int jt, int kt
     PP_ARG(!lpt2 || (f->eta2y && f->eta2z), "eta2 outputs come as a set of three");
     PP_CHECK(ensure_device(ctx));
     const int n = G.nmesh, n2 = 2 * n;
+    TileGeo T;
+    T.n = n;
+    T.N = c->N;
+    T.M = G.M;
+    T.b = c->block;
+    T.i0 = (it - 1) * c->nsub - G.nbuff;
+    T.j0 = (jt - 1) * c->nsub - G.nbuff;
+    T.k0 = (kt - 1) * c->nsub - G.nbuff;
+    T.inv_b3 = (float)(1.0 / sqrt(pow((double)c->block, 3)));
+    T.seed = G.seed;
+    // odd n: k_residual_pad's layout (pairs of cells) reaches one cell past the
+    // tile, so its fields are not those of the line transforms
+    if (n % 2 == 0 && line_supported(n) && G.M <= kLineCoarse) return split_tile_lines(ctx, c, T, f);
     const long long n3 = (long long)n * n * n;
     // 1. residual -> padded buffer R; base spectrum in place
     FftPlans *Fi = nullptr;
@@ -509,16 +947,6 @@ int pp_split_tile_fields(pp_ctx *ctx, const pp_coarse *c, int it, int jt, int kt
         PP_HIP(hipMallocAsync(&Wk, Fi->work_need, ctx->stream));
         PP_FFT(rocfft_execution_info_set_work_buffer(Fi->info, Wk, Fi->work_need));
     }
-    TileGeo T;
-    T.n = n;
-    T.N = c->N;
-    T.M = G.M;
-    T.b = c->block;
-    T.i0 = (it - 1) * c->nsub - G.nbuff;
-    T.j0 = (jt - 1) * c->nsub - G.nbuff;
-    T.k0 = (kt - 1) * c->nsub - G.nbuff;
-    T.inv_b3 = (float)(1.0 / sqrt(pow((double)c->block, 3)));
-    T.seed = G.seed;
     hipLaunchKernelGGL(k_residual_pad, dim3(grid_for(ctx, (long long)(n + 1) * n2 * n2)), dim3(256), 0, ctx->stream, R, T,
                        (const float *)c->noise.ptr);
     PP_HIP(hipGetLastError());

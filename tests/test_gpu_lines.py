@@ -54,3 +54,30 @@ def test_uneven_power_table(ctx):
     _close("delta", f[0].cpu().numpy(), ref.delta)
     for q in range(3):
         _close(f"eta{q}", f[1 + q].cpu().numpy(), ref.eta[q])
+
+
+@pytest.mark.parametrize("nmesh,nbuff,ntile,M,tile,second", [
+    (16, 2, 2, 14, (1, 2, 1), True),     # shortest line, block 2
+    (18, 3, 3, 14, (3, 1, 2), True),     # block 3, lines no multiple of the threads' eight
+    (30, 5, 4, 10, (2, 4, 3), True),     # 2 3 5
+    (50, 5, 3, 13, (1, 3, 2), False),    # first order only
+    (56, 4, 2, 8, (1, 1, 1), True),      # radix 7; the wrap in all three axes
+    (96, 8, 2, 11, (2, 2, 1), True),     # 8 4 3
+    (26, 2, 2, 8, (1, 2, 2), True),      # no line transform (factor 13): rocFFT
+])
+def test_split_tile(ctx, nmesh, nbuff, ntile, M, tile, second):
+    from oracle import fields as OF
+    from peakpatch_hip import split, synth
+    g = split.SplitGeom(nmesh, nbuff, ntile, M, 1.1, seed=nmesh)
+    cf = split.CoarseField(ctx, g)
+    t = split.make_split_tile(ctx, cf, *tile, ilpt=2 if second else 1, want_lapd=second)
+    ref = OF.split_tile(OF.SplitGeom(nmesh, nbuff, ntile, M, 1.1), *tile, nmesh, OF.PkTable(*synth.pk_table()))
+    host = lambda a: a.cpu().numpy()
+    _close("delta", host(t.delta), ref.delta)
+    for q in range(3):
+        _close(f"eta{q}", host(t.eta[q]), ref.eta[q])
+        if second:
+            _close(f"eta2{q}", host(t.eta2[q]), ref.eta2[q])
+    if second:
+        _close("lapd", host(t.lapd), ref.lapd)
+    cf.close()
