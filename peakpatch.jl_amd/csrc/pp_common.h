@@ -161,6 +161,7 @@ struct pp_ctx {
     // events: [0,1] whole call, [2..13] persistent-form stage boundaries
     static constexpr int NEV = 15;
     hipEvent_t ev[NEV] = {};
+    hipEvent_t ev_bank = nullptr;  // the filter bank's side work against its main work
     hipEvent_t ev_join = nullptr, ev_join2 = nullptr;  // order the context's streams against a caller's
     pp::Timing timing;
 };

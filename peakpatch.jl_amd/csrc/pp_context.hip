@@ -307,12 +307,14 @@ int pp_ctx_create(int device, pp_ctx **out)
     hipDeviceProp_t prop;
     if (e == hipSuccess) e = hipGetDeviceProperties(&prop, device);
     for (int i = 0; i < pp_ctx::NEV && e == hipSuccess; i++) e = hipEventCreate(&c->ev[i]);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&c->ev_bank, hipEventDisableTiming);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&c->ev_join2, hipEventDisableTiming);
     if (e != hipSuccess) {
         set_error("context creation on device %d failed: %s", device, hipGetErrorString(e));
         for (auto &ev : c->ev)
             if (ev) (void)hipEventDestroy(ev);
+        if (c->ev_bank) (void)hipEventDestroy(c->ev_bank);
         if (c->ev_join) (void)hipEventDestroy(c->ev_join);
         if (c->ev_join2) (void)hipEventDestroy(c->ev_join2);
         if (c->side) (void)hipStreamDestroy(c->side);
@@ -352,6 +354,7 @@ int pp_ctx_destroy(pp_ctx *ctx)
     for (auto &b : ctx->d_in) b.release();
     for (auto &e : ctx->ev)
         if (e) (void)hipEventDestroy(e);
+    if (ctx->ev_bank) (void)hipEventDestroy(ctx->ev_bank);
     if (ctx->ev_join) (void)hipEventDestroy(ctx->ev_join);
     if (ctx->ev_join2) (void)hipEventDestroy(ctx->ev_join2);
     if (ctx->side) (void)hipStreamDestroy(ctx->side);

@@ -79,16 +79,36 @@ inline SpecGeo spec_geo(int n, int rows)
     return g;
 }
 
+// The arithmetic below is written out with its fused operations and without
+// contraction by the compiler, so that a transform gives the same bits in every
+// kernel it is part of.
+#define PP_NO_CONTRACT _Pragma("clang fp contract(off)")
+
 __device__ __forceinline__ float2 fmul(float2 a, float2 b)
 {
-    return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+    PP_NO_CONTRACT
+    return make_float2(__builtin_fmaf(a.x, b.x, -(a.y * b.y)), __builtin_fmaf(a.x, b.y, a.y * b.x));
 }
 __device__ __forceinline__ float2 fmulc(float2 a, float2 b)  // a conj(b)
 {
-    return make_float2(a.x * b.x + a.y * b.y, a.y * b.x - a.x * b.y);
+    PP_NO_CONTRACT
+    return make_float2(__builtin_fmaf(a.x, b.x, a.y * b.y), __builtin_fmaf(a.y, b.x, -(a.x * b.y)));
 }
-__device__ __forceinline__ float2 fadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
-__device__ __forceinline__ float2 fsub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
+__device__ __forceinline__ float2 fadd(float2 a, float2 b)
+{
+    PP_NO_CONTRACT
+    return make_float2(a.x + b.x, a.y + b.y);
+}
+__device__ __forceinline__ float2 fsub(float2 a, float2 b)
+{
+    PP_NO_CONTRACT
+    return make_float2(a.x - b.x, a.y - b.y);
+}
+// a + s b
+__device__ __forceinline__ float2 faxpy(float s, float2 b, float2 a)
+{
+    return make_float2(__builtin_fmaf(s, b.x, a.x), __builtin_fmaf(s, b.y, a.y));
+}
 // times -i (forward) or +i (inverse)
 template <int SIGN> __device__ __forceinline__ float2 rot(float2 a)
 {
@@ -113,15 +133,15 @@ template <int R, int SIGN> __device__ __forceinline__ void butterfly(float2 *v)
         butterfly<4, SIGN>(e);
         butterfly<4, SIGN>(o);
         // odd half times exp(SIGN 2 pi i r / 8)
-        const float2 r1 = rot<SIGN>(o[1]), r3 = rot<SIGN>(o[3]);
-        o[1] = make_float2((o[1].x + r1.x) * h, (o[1].y + r1.y) * h);
-        o[2] = rot<SIGN>(o[2]);
-        o[3] = make_float2((r3.x - o[3].x) * h, (r3.y - o[3].y) * h);
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            v[r] = fadd(e[r], o[r]);
-            v[r + 4] = fsub(e[r], o[r]);
-        }
+        const float2 o1 = fadd(o[1], rot<SIGN>(o[1])), o2 = rot<SIGN>(o[2]), o3 = fsub(rot<SIGN>(o[3]), o[3]);
+        v[0] = fadd(e[0], o[0]);
+        v[4] = fsub(e[0], o[0]);
+        v[1] = faxpy(h, o1, e[1]);
+        v[5] = faxpy(-h, o1, e[1]);
+        v[2] = fadd(e[2], o2);
+        v[6] = fsub(e[2], o2);
+        v[3] = faxpy(h, o3, e[3]);
+        v[7] = faxpy(-h, o3, e[3]);
     } else {
         // odd prime: the sums and differences of conjugate inputs
         constexpr float C3[1] = {-0.5f}, S3[1] = {0.86602540378443865f};
@@ -145,11 +165,9 @@ template <int R, int SIGN> __device__ __forceinline__ void butterfly(float2 *v)
 #pragma unroll
             for (int q = 0; q < H; q++) {
                 const int t = (k * (q + 1)) % R, u = t <= H ? t : R - t;
-                const float c = C[u - 1], s = t <= H ? S[u - 1] : -S[u - 1];
-                a.x += c * p[q].x;
-                a.y += c * p[q].y;
-                b.x += s * m[q].x;
-                b.y += s * m[q].y;
+                const float s = t <= H ? S[u - 1] : -S[u - 1];
+                a = faxpy(C[u - 1], p[q], a);
+                b = faxpy(s, m[q], b);
             }
             b = rot<SIGN>(b);
             v[k] = fadd(a, b);
@@ -421,6 +439,7 @@ __device__ __forceinline__ ColTile col_tile(const ColGrid &C)
 // the DC and Nyquist with real values) as the complex line of both.
 template <class A> __device__ __forceinline__ void join_rows(const A &at, int n, int k, float2 a, float2 b)
 {
+    PP_NO_CONTRACT
     const int kc = k == 0 ? 0 : n - k;
     if (kc == k) {  // DC and, for even n, Nyquist: real
         at(k) = make_float2(a.x, b.x);
@@ -434,6 +453,7 @@ template <class A> __device__ __forceinline__ void join_rows(const A &at, int n,
 // that pairs with k
 __device__ __forceinline__ void split_rows(float2 z, float2 zc, float2 &a, float2 &b)
 {
+    PP_NO_CONTRACT
     a = make_float2(0.5f * (z.x + zc.x), 0.5f * (z.y - zc.y));
     b = make_float2(0.5f * (z.y + zc.y), 0.5f * (zc.x - z.x));
 }

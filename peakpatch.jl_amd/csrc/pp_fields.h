@@ -58,6 +58,7 @@ struct XArgs {
         float f;
     } op[5];
     float mult;
+    int top = 1 << 30;  // bins above it are zero and not read
     void add(const float2 *in, float *out, int pow, bool imag, float f) { op[nop++] = Op{in, out, pow, imag, f}; }
 };
 
@@ -86,6 +87,32 @@ int pk_log_device(pp_ctx *ctx, const pp_pk_table *pk, double *buf, PkLog *out);
 // the up to 10^9 modes of a grid.
 inline long long amp_count(int imax) { return 3ll * imax * imax + 1; }
 int amp_table(pp_ctx *ctx, const PkLog &T, double mult, double dk3, double n3, long long count, float *out);
+
+// the line of a row pair from an x-spectrum times f kx^pow or i f kx^pow; bins
+// above top are zero
+__device__ __forceinline__ void load_row_pair(const RowAddr &at, const LineFft &P, const SpecGeo &g,
+                                              const float2 *in, long long r, bool two, int jj, int pow, bool imag,
+                                              float f, float mult, int top)
+{
+    const long long z = r / g.n, z2 = (r + 1) / g.n;
+    const float2 *a = in + g.row((int)z, (int)(r - z * g.n)), *b = in + g.row((int)z2, (int)(r + 1 - z2 * g.n));
+    float2 va[kRowBins], vb[kRowBins];
+#pragma unroll
+    for (int q = 0; q < kRowBins; q++) {
+        const int k = jj + q * P.tj, kc = min(k, g.nk - 1);
+        va[q] = k <= top ? a[kc] : make_float2(0.f, 0.f);
+        vb[q] = two && k <= top ? b[kc] : make_float2(0.f, 0.f);
+    }
+#pragma unroll
+    for (int q = 0; q < kRowBins; q++) {
+        const int k = jj + q * P.tj;
+        if (k >= g.nk) break;
+        const float kx = (float)k * mult, c = pow == 0 ? f : pow == 1 ? f * kx : f * kx * kx;
+        const float2 u = va[q], v = vb[q];
+        join_rows(at, g.n, k, imag ? make_float2(-c * u.y, c * u.x) : make_float2(c * u.x, c * u.y),
+                  imag ? make_float2(-c * v.y, c * v.x) : make_float2(c * v.x, c * v.y));
+    }
+}
 
 struct GridPlan {
     LineFft row, col, ycol;

@@ -322,31 +322,6 @@ __global__ void __launch_bounds__(1024, M == kLineReg ? 8 : 4) k_cols_y_inv(Spec
     }
 }
 
-// the line of a row pair from an x-spectrum times re_f or i im_f = f kx^pow
-__device__ __forceinline__ void load_row_pair(const RowAddr &at, const LineFft &P, const SpecGeo &g,
-                                              const float2 *in, long long r, bool two, int jj, int pow, bool imag,
-                                              float f, float mult)
-{
-    const long long z = r / g.n, z2 = (r + 1) / g.n;
-    const float2 *a = in + g.row((int)z, (int)(r - z * g.n)), *b = in + g.row((int)z2, (int)(r + 1 - z2 * g.n));
-    float2 va[kRowBins], vb[kRowBins];
-#pragma unroll
-    for (int q = 0; q < kRowBins; q++) {
-        const int k = min(jj + q * P.tj, g.nk - 1);
-        va[q] = a[k];
-        vb[q] = two ? b[k] : make_float2(0.f, 0.f);
-    }
-#pragma unroll
-    for (int q = 0; q < kRowBins; q++) {
-        const int k = jj + q * P.tj;
-        if (k >= g.nk) break;
-        const float kx = (float)k * mult, c = pow == 0 ? f : pow == 1 ? f * kx : f * kx * kx;
-        const float2 u = va[q], v = vb[q];
-        join_rows(at, g.n, k, imag ? make_float2(-c * u.y, c * u.x) : make_float2(c * u.x, c * u.y),
-                  imag ? make_float2(-c * v.y, c * v.x) : make_float2(c * v.x, c * v.y));
-    }
-}
-
 // x-inverse: grid (row pairs, outputs)
 template <int M>
 __global__ void __launch_bounds__(512) k_rows_inv(SpecGeo g, LineFft P, XArgs X)
@@ -357,7 +332,7 @@ __global__ void __launch_bounds__(512) k_rows_inv(SpecGeo g, LineFft P, XArgs X)
     const RowAddr at(lds + line * row_pitch(n));
     const bool two = r + 1 < rows;
     const XArgs::Op &O = X.op[blockIdx.y];
-    if (r < rows) load_row_pair(at, P, g, O.in, r, two, jj, O.pow, O.imag, O.f, X.mult);
+    if (r < rows) load_row_pair(at, P, g, O.in, r, two, jj, O.pow, O.imag, O.f, X.mult, X.top);
     __syncthreads();
     float2 x[kLineEpt];
     line_run<1, M, true, false>(at, P, jj, x);
@@ -403,7 +378,7 @@ __global__ void __launch_bounds__(512) k_rows_src(SpecGeo g, LineFft P, SrcArgs 
         int j2 = jj;
         asm volatile("" : "+v"(j2));
         __syncthreads();
-        if (live) load_row_pair(at, P, g, S.in[v], r, two, j2, S.pow[v], false, 1.f, S.mult);
+        if (live) load_row_pair(at, P, g, S.in[v], r, two, j2, S.pow[v], false, 1.f, S.mult, g.nk);
         __syncthreads();
         float2 x[kLineEpt];
         line_run<1, M, true, false>(at, P, j2, x);

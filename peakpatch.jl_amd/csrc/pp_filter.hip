@@ -25,6 +25,7 @@
 #include <mutex>
 
 #include "pp_common.h"
+#include "pp_fields.h"
 #include "pp_noise.h"
 
 namespace pp {
@@ -324,13 +325,18 @@ __global__ void __launch_bounds__(256) k_peak_emit(const float *__restrict__ d, 
 }
 
 __global__ void k_stencil_finish(const uint64_t *__restrict__ bits, const int *__restrict__ word_off,
-                                 long long nwords, long long max_peaks, long long *__restrict__ counters)
+                                 long long nwords, long long max_peaks, long long *__restrict__ counters,
+                                 long long *__restrict__ range)
 {
     long long found = nwords > 0 ? (long long)word_off[nwords - 1] + __popcll(bits[nwords - 1]) : 0;
     long long kept = found < max_peaks ? found : max_peaks;
     counters[2] = counters[0];
     counters[0] += kept;
     counters[1] += kept;
+    if (range) {  // this filter's peaks, for work that follows on another stream
+        range[0] = counters[2];
+        range[1] = counters[0];
+    }
 }
 
 __global__ void k_sample_field(const float *__restrict__ f, int n1, int n2, const int32_t *__restrict__ pi,
@@ -389,12 +395,12 @@ static StencilScratch stencil_carve(void *base, const StencilGeom &g, size_t tmp
 // counters[0].
 static int run_stencil_with(pp_ctx *ctx, const float *d_field, int8_t *d_mask, const StencilGeom &g,
                             float fcrit, long long max_peaks, int filt, const PeakOut &o, long long *d_counters,
-                            const StencilScratch &s)
+                            const StencilScratch &s, long long *range = nullptr)
 {
     PP_ARG(g.nwords < (1ll << 31), "inner cube too large for the stencil");
     if (g.nwords == 0) {
         hipLaunchKernelGGL(k_stencil_finish, dim3(1), dim3(1), 0, ctx->stream, (const uint64_t *)nullptr,
-                           (const int *)nullptr, 0ll, max_peaks, d_counters);
+                           (const int *)nullptr, 0ll, max_peaks, d_counters, range);
         PP_HIP(hipGetLastError());
         return PP_OK;
     }
@@ -417,21 +423,244 @@ static int run_stencil_with(pp_ctx *ctx, const float *d_field, int8_t *d_mask, c
                        filt, o);
     PP_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_stencil_finish, dim3(1), dim3(1), 0, ctx->stream, (const uint64_t *)s.bits,
-                       (const int *)s.off, g.nwords, max_peaks, d_counters);
+                       (const int *)s.off, g.nwords, max_peaks, d_counters, range);
     PP_HIP(hipGetLastError());
     return PP_OK;
 }
 
 static int run_stencil(pp_ctx *ctx, const float *d_field, int8_t *d_mask, const StencilGeom &g,
                        float fcrit, long long max_peaks, int filt, const PeakOut &o,
-                       long long *d_counters)
+                       long long *d_counters, long long *range = nullptr)
 {
     size_t bytes = 0, tmp = 0;
     PP_CHECK(stencil_scan_bytes(g, &tmp));
     PP_CHECK(stencil_scratch_bytes(g, &bytes));
     PP_CHECK(ctx->d_scan.grow(bytes));
     return run_stencil_with(ctx, d_field, d_mask, g, fcrit, max_peaks, filt, o, d_counters,
-                            stencil_carve(ctx->d_scan.ptr, g, tmp));
+                            stencil_carve(ctx->d_scan.ptr, g, tmp), range);
+}
+
+// ------------------------------------------- the k^2 field at the peaks
+// With want_lapd every filter's k^2-Gaussian field is wanted at its new peaks
+// only.  Its inverse transform (rocFFT: 1.46 ms at 512^3, after half of
+// k_window's 0.31 ms) is done on line transforms (pp_fft.h) instead, as far as
+// the peaks need it: the window goes into the z pass, planes and rows outside
+// the inner cube are not written, modes whose Gaussian is below 1e-20 are not
+// read, and only the row pairs that hold a peak are transformed along x, from
+// where the peaks' values are taken without a field.  The passes run on the
+// side stream beside the next filters' rocFFT kernels, which leave most of
+// HBM's bandwidth free; only the last waits for its filter's stencil.
+// pp_smooth_field with wsmooth = 3 takes the same passes over the whole grid,
+// so both give the same bits.
+struct BankGeo {
+    int n, lo, hi;      // planes [lo, hi)
+    int ylo, yhi;       // rows [ylo, yhi): the inner ones and their partners in row pairs
+    int cut;            // modes |i| > cut on any axis are left out
+    int plain;          // radius 0: no window
+    float mult2, scale; // k^2 = mult2 |i|^2
+    const float *gauss; // exp(-(k Rf)^2 / 8) by index, n / 2 + 1
+};
+
+// exp(-(i dk R)^2 / 8) of every filter, Float64 rounded once
+__global__ void k_gauss_table(const double *__restrict__ Rf, int nfilt, int count, double dk, float *__restrict__ out)
+{
+    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < nfilt * count; t += gridDim.x * blockDim.x) {
+        const int f = t / count, i = t - f * count;
+        const double x = (double)i * dk * Rf[f] / 2.0;
+        out[t] = (float)exp(-(x * x) / 2.0);
+    }
+}
+
+// rocFFT's spectrum (rows of n / 2 + 1) into rows of whole 128-byte lines
+__global__ void __launch_bounds__(256) k_repack(const float2 *__restrict__ in, SpecGeo g, float2 *__restrict__ out)
+{
+    const long long rows = (long long)g.n * g.n;
+    for (long long r = (long long)blockIdx.x * 4 + threadIdx.x / 64; r < rows; r += (long long)gridDim.x * 4) {
+        const int z = (int)(r / g.n);
+        const float2 *a = in + r * g.nk;
+        float2 *b = out + g.row(z, (int)(r - (long long)z * g.n));
+        for (int k = threadIdx.x % 64; k < g.nk; k += 64) b[k] = a[k];
+    }
+}
+
+template <int M>
+__global__ void __launch_bounds__(1024) k_bank_z(SpecGeo g, LineFft P, ColGrid C, BankGeo B,
+                                                 const float2 *__restrict__ in, float2 *__restrict__ out)
+{
+    extern __shared__ float2 lds[];
+    const ColTile t = col_tile(C);
+    if (t.plane < 0) return;
+    // the tile grid counts the rows |fy| <= cut: 0 .. cut, then -cut .. -1
+    const int n = g.n, iy = t.plane <= B.cut || 2 * B.cut + 1 > n ? t.plane : n - (2 * B.cut + 1 - t.plane);
+    const int fy = iy < (n + 1) / 2 ? iy : iy - n, ay = abs(fy), kx = min(t.kx, g.nk - 1), ixy = kx * kx + fy * fy;
+    const ColAddr<M != kLineAny> at(lds, t.l, C.logl);
+    const LineZ src(g, in, iy, t.kx);
+    const float gxy = B.gauss[kx] * B.gauss[ay] * B.scale;
+    float2 X[kLineEpt];
+#pragma unroll
+    for (int q = 0; q < kLineEpt; q++) {
+        const int e = min(t.jj + q * P.tj, n - 1), fz = e < (n + 1) / 2 ? e : e - n, az = abs(fz);
+        X[q] = make_float2(0.f, 0.f);
+        if (az <= B.cut) {
+            const float2 v = *src.at(e);
+            const int i2 = ixy + fz * fz;
+            const float f = i2 == 0 || B.plain ? B.scale : gxy * B.gauss[az] * ((float)i2 * B.mult2);  // k = 0: unscaled
+            X[q] = make_float2(v.x * f, v.y * f);
+        }
+    }
+    line_run<1, M, false, false>(at, P, t.jj, X);
+    const LineZ dst(g, out, iy, t.kx);
+#pragma unroll
+    for (int q = 0; q < kLineEpt; q++) {
+        const int e = t.jj + q * P.tj;
+        if (e >= B.lo && e < B.hi) *dst.at(e) = X[q];
+    }
+}
+
+template <int M>
+__global__ void __launch_bounds__(1024) k_bank_y(SpecGeo g, LineFft P, ColGrid C, BankGeo B, float2 *__restrict__ s)
+{
+    extern __shared__ float2 lds[];
+    const ColTile t = col_tile(C);
+    if (t.plane < 0) return;
+    const int n = g.n;
+    const ColAddr<M != kLineAny> at(lds, t.l, C.logl);
+    const LineY io(g, s, B.lo + t.plane, 0, 1, t.kx);
+    float2 X[kLineEpt];
+#pragma unroll
+    for (int q = 0; q < kLineEpt; q++) {
+        const int e = min(t.jj + q * P.tj, n - 1), fy = e < (n + 1) / 2 ? e : e - n;
+        X[q] = abs(fy) <= B.cut ? *io.at(e) : make_float2(0.f, 0.f);
+    }
+    line_run<1, M, false, false>(at, P, t.jj, X);
+#pragma unroll
+    for (int q = 0; q < kLineEpt; q++) {
+        const int e = t.jj + q * P.tj;
+        if (e >= B.ylo && e < B.yhi) *io.at(e) = X[q];
+    }
+}
+
+// the field at the peaks [range[0], range[1]), which come in the order of
+// their rows: a line looks its row pair up and, if it holds peaks, transforms
+// it as k_rows_inv does
+template <int M>
+__global__ void __launch_bounds__(512) k_bank_rows(SpecGeo g, LineFft P, BankGeo B, const float2 *__restrict__ s,
+                                                   const int32_t *__restrict__ pi, const int32_t *__restrict__ pj,
+                                                   const int32_t *__restrict__ pk, float *__restrict__ out,
+                                                   const long long *__restrict__ range, long long capacity)
+{
+    extern __shared__ float2 lds[];
+    const int n = g.n, line = threadIdx.x / P.tj, jj = threadIdx.x - line * P.tj;
+    // row pairs from the one that holds the first row of plane lo
+    const long long r = 2 * ((long long)B.lo * n / 2 + (long long)blockIdx.x * (blockDim.x / P.tj) + line);
+    const long long hi = min(range[1], capacity);
+    auto row = [&](long long p) { return (long long)pk[p] * n + pj[p]; };
+    long long lo = range[0], top = hi;
+    while (lo < top) {  // the first peak of row r or later
+        const long long mid = (lo + top) >> 1;
+        if (row(mid) < r) lo = mid + 1;
+        else top = mid;
+    }
+    const bool has = lo < hi && row(lo) <= r + 1;
+    if (!__syncthreads_or(has)) return;
+    const RowAddr at(lds + line * row_pitch(n));
+    if (has) load_row_pair(at, P, g, s, r, true, jj, 0, false, 1.f, 0.f, B.cut);
+    __syncthreads();
+    float2 x[kLineEpt];
+    line_run<1, M, true, true>(at, P, jj, x);
+    if (!has) return;
+    for (long long p = lo + jj; p < hi && row(p) <= r + 1; p += P.tj) {
+        const float2 v = at(pi[p]);
+        out[p] = row(p) == r ? v.x : v.y;
+    }
+}
+
+// Device buffers and launch shapes of the above for one pp_find_peaks call
+struct Bank {
+    GridPlan G;
+    BankGeo B{};
+    float2 *R = nullptr, *T = nullptr;
+    float *tables = nullptr;
+    long long *ranges = nullptr;
+    double dk = 0;
+};
+
+// spec: delta_k as rocFFT leaves it, made on the main stream; planes and rows
+// [lo, hi) are wanted
+static int bank_start(pp_ctx *ctx, const void *spec, int n, int lo, int hi, double boxsize, const double *Rf, int nfilt,
+                      Bank &K)
+{
+    PP_CHECK(grid_plan(ctx, n, &K.G));
+    K.G.stream = ctx->side;
+    const SpecGeo &g = K.G.g;
+    const int count = n / 2 + 1;
+    const size_t arr = g.size(n);
+    PP_CHECK(ctx->d_spec.grow(2 * arr * sizeof(float2)));
+    K.R = ctx->d_spec.as<float2>();
+    K.T = K.R + arr;
+    PP_CHECK(ctx->d_misc.grow((size_t)nfilt * (3 * sizeof(double) + count * sizeof(float))));
+    double *d_Rf = ctx->d_misc.as<double>();
+    K.ranges = (long long *)(d_Rf + nfilt);
+    K.tables = (float *)(K.ranges + 2 * nfilt);
+    K.dk = 2.0 * M_PI / boxsize;
+    K.B.n = n;
+    K.B.lo = lo;
+    K.B.hi = hi;
+    K.B.ylo = std::max(0, lo - 1);
+    K.B.yhi = std::min(n, hi + 1);
+    K.B.mult2 = (float)(K.dk * K.dk);
+    K.B.scale = (float)(1.0 / ((double)n * n * n));
+    PP_HIP(hipEventRecord(ctx->ev_bank, ctx->stream));
+    PP_HIP(hipStreamWaitEvent(ctx->side, ctx->ev_bank, 0));
+    PP_HIP(hipMemcpyAsync(d_Rf, Rf, nfilt * sizeof(double), hipMemcpyHostToDevice, ctx->side));
+    hipLaunchKernelGGL(k_gauss_table, dim3((nfilt * count + 255) / 256), dim3(256), 0, ctx->side, (const double *)d_Rf,
+                       nfilt, count, K.dk, K.tables);
+    PP_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_repack, dim3(ctx->num_cu * 16), dim3(256), 0, ctx->side, (const float2 *)spec, g, K.R);
+    PP_HIP(hipGetLastError());
+    return PP_OK;
+}
+
+// main-stream work launched next runs after the side stream's so far
+static int bank_join(pp_ctx *ctx)
+{
+    PP_HIP(hipEventRecord(ctx->ev_bank, ctx->side));
+    PP_HIP(hipStreamWaitEvent(ctx->stream, ctx->ev_bank, 0));
+    return PP_OK;
+}
+
+// filter f's spectrum along z and y (needs no peaks)
+static int bank_transform(pp_ctx *ctx, Bank &K, const double *Rf, int f)
+{
+    const SpecGeo &g = K.G.g;
+    const int n = g.n, half = n / 2;
+    K.B.gauss = K.tables + (size_t)f * (half + 1);
+    // exp(-(c dk R)^2 / 8) < 1e-20: below every Float32 rounding of the result
+    const double c = sqrt(8.0 * 46.0) / fabs(K.dk * Rf[f]);
+    K.B.cut = c < half ? (int)c + 1 : half;
+    K.B.plain = Rf[f] == 0.0;
+    const int rows = std::min(n, 2 * K.B.cut + 1), bins = std::min(K.B.cut, g.nk - 1) + 1;
+    if (K.B.hi <= K.B.lo) return PP_OK;
+    const ColGrid cz = K.G.cs.grid(bins, rows, kColXCD), cy = K.G.ys.grid(bins, K.B.hi - K.B.lo, 1);
+    PP_LINE_LAUNCH(K.G.col, k_bank_z, dim3(cz.blocks()), dim3(K.G.cs.block), K.G.cs.lds, ctx->side, g, K.G.col, cz, K.B,
+                   (const float2 *)K.R, K.T);
+    PP_LINE_LAUNCH(K.G.ycol, k_bank_y, dim3(cy.blocks()), dim3(K.G.ys.block), K.G.ys.lds, ctx->side, g, K.G.ycol, cy,
+                   K.B, K.T);
+    return PP_OK;
+}
+
+// ... and its values at filter f's peaks, once its stencil is done
+static int bank_sample(pp_ctx *ctx, Bank &K, int f, const PeakOut &o, float *d_lapd)
+{
+    PP_HIP(hipEventRecord(ctx->ev_bank, ctx->stream));
+    PP_HIP(hipStreamWaitEvent(ctx->side, ctx->ev_bank, 0));
+    if (K.B.hi <= K.B.lo) return PP_OK;
+    const long long n = K.G.g.n, pairs = (n * K.B.hi + 1) / 2 - n * K.B.lo / 2;
+    const LineShape &S = K.G.rs;
+    PP_LINE_LAUNCH(K.G.row, k_bank_rows, dim3((unsigned)((pairs + S.nl - 1) / S.nl)), dim3(S.block), S.lds, ctx->side,
+                   K.G.g, K.G.row, K.B, (const float2 *)K.T, (const int32_t *)o.i, (const int32_t *)o.j,
+                   (const int32_t *)o.k, d_lapd, (const long long *)(K.ranges + 2 * f), o.capacity);
+    return PP_OK;
 }
 
 // ------------------------------------------- peak finding without allocation
@@ -582,12 +811,25 @@ int pp_smooth_field(pp_ctx *ctx, const void *delta_k, float *out, int on_device,
         src = ctx->d_k0.ptr;
     }
     float inv = (float)(1.0 / ((double)n * n * n));
-    PP_CHECK(launch_window(ctx, src, ctx->d_k1.ptr, n, boxsize, Rf, wsmooth, inv));
     float *dst = out;
     if (!on_device) {
         PP_CHECK(ctx->d_field_a.grow(rb));
         dst = ctx->d_field_a.as<float>();
     }
+    if (wsmooth == PP_WINDOW_K2GAUSS && line_supported(n)) {
+        Bank K;
+        PP_CHECK(bank_start(ctx, src, n, 0, n, boxsize, &Rf, 1, K));
+        PP_CHECK(bank_transform(ctx, K, &Rf, 0));
+        XArgs X{};
+        X.top = K.B.cut;
+        X.add(K.T, dst, 0, false, 1.f);
+        PP_CHECK(rows_inv(K.G, X));
+        PP_CHECK(bank_join(ctx));
+        if (!on_device) PP_HIP(hipMemcpyAsync(out, dst, rb, hipMemcpyDeviceToHost, ctx->stream));
+        PP_HIP(hipStreamSynchronize(ctx->stream));
+        return PP_OK;
+    }
+    PP_CHECK(launch_window(ctx, src, ctx->d_k1.ptr, n, boxsize, Rf, wsmooth, inv));
     void *ib[1] = {ctx->d_k1.ptr}, *ob[1] = {dst};
     PP_FFT(rocfft_execute(ctx->fftp->c2r, ib, ob, ctx->fftp->info));
     if (!on_device) PP_HIP(hipMemcpyAsync(out, dst, rb, hipMemcpyDeviceToHost, ctx->stream));
@@ -648,7 +890,10 @@ int pp_find_peaks(pp_ctx *ctx, const float *delta, int on_device, int n, double 
     PP_CHECK(ctx->d_k0.grow(cb));
     PP_CHECK(ctx->d_k1.grow(cb));
     PP_CHECK(ctx->d_field_a.grow(rb));
-    if (want_lapd) {
+    // the wsmooth = 3 field at the peaks: line transforms where the mesh has
+    // them, else a second rocFFT inverse per filter
+    const bool lines = want_lapd && line_supported(n);
+    if (want_lapd && !lines) {
         PP_CHECK(ctx->d_k2.grow(cb));
         PP_CHECK(ctx->d_field_b.grow(rb));
     }
@@ -674,16 +919,23 @@ int pp_find_peaks(pp_ctx *ctx, const float *delta, int on_device, int n, double 
     PP_CHECK(alloc_peak_out(ctx, out->capacity, o, &d_lapd, &d_counters));
     const StencilGeom g = stencil_geom(n, n, n, nbuff);
     const float inv = (float)(1.0 / ((double)n * n * n));
+    Bank K;
+    if (lines && nfilt > 0) PP_CHECK(bank_start(ctx, ctx->d_k0.ptr, n, nbuff, n - nbuff, boxsize, Rf, nfilt, K));
     for (int f = 0; f < nfilt; f++) {
-        // one read of delta_k gives the filter's spectrum and, with want_lapd,
-        // the wsmooth = 3 spectrum sampled at the filter's new peaks
-        PP_CHECK(launch_window2(ctx, ctx->d_k0.ptr, ctx->d_k1.ptr, wsmooth, want_lapd ? ctx->d_k2.ptr : nullptr,
-                                PP_WINDOW_K2GAUSS, n, boxsize, Rf[f], inv));
+        if (lines) PP_CHECK(bank_transform(ctx, K, Rf, f));
+        // one read of delta_k gives the filter's spectrum and, with want_lapd
+        // and no line transform, the wsmooth = 3 spectrum sampled at the
+        // filter's new peaks
+        PP_CHECK(launch_window2(ctx, ctx->d_k0.ptr, ctx->d_k1.ptr, wsmooth,
+                                want_lapd && !lines ? ctx->d_k2.ptr : nullptr, PP_WINDOW_K2GAUSS, n, boxsize, Rf[f],
+                                inv));
         void *ib[1] = {ctx->d_k1.ptr}, *ob[1] = {ctx->d_field_a.ptr};
         PP_FFT(rocfft_execute(ctx->fftp->c2r, ib, ob, ctx->fftp->info));
         PP_CHECK(run_stencil(ctx, ctx->d_field_a.as<float>(), d_mask, g, fcrit[f], max_peaks_per_filter, f,
-                             o, d_counters));
-        if (want_lapd) {
+                             o, d_counters, lines ? K.ranges + 2 * f : nullptr));
+        if (lines) {
+            PP_CHECK(bank_sample(ctx, K, f, o, d_lapd));
+        } else if (want_lapd) {
             void *ib2[1] = {ctx->d_k2.ptr}, *ob2[1] = {ctx->d_field_b.ptr};
             PP_FFT(rocfft_execute(ctx->fftp->c2r, ib2, ob2, ctx->fftp->info));
             hipLaunchKernelGGL(k_sample_field, dim3(ctx->num_cu * 4), dim3(256), 0, ctx->stream,
@@ -692,6 +944,7 @@ int pp_find_peaks(pp_ctx *ctx, const float *delta, int on_device, int n, double 
             PP_HIP(hipGetLastError());
         }
     }
+    if (lines) PP_CHECK(bank_join(ctx));
     PP_HIP(hipEventRecord(ctx->ev[1], ctx->stream));
     if (mask_inout) PP_HIP(hipMemcpyAsync(mask_inout, d_mask, N, hipMemcpyDeviceToHost, ctx->stream));
     int rc = download_peaks(ctx, o, want_lapd ? d_lapd : nullptr, d_counters, out);

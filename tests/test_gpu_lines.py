@@ -81,3 +81,26 @@ def test_split_tile(ctx, nmesh, nbuff, ntile, M, tile, second):
     if second:
         _close("lapd", host(t.lapd), ref.lapd)
     cf.close()
+
+
+@pytest.mark.parametrize("n,nbuff", [(25, 2), (48, 1), (63, 5), (64, 4), (100, 9), (128, 30), (34, 3)])
+def test_k2_field_at_the_peaks(ctx, n, nbuff):
+    """The wsmooth = 3 field at the peaks of a bank of radii from below a cell
+    (every mode kept) to a quarter of the box (few modes kept) and zero: the
+    bits of pp_smooth_field, and the FP64 field within 2e-5 of its largest
+    value (the Float32 transforms' noise over fewer modes than above)."""
+    import torch
+    from oracle import oracle as O
+    box = 1.0 * n
+    rng = np.random.default_rng(n)
+    delta = rng.normal(size=(n, n, n)).astype(np.float32)
+    Rf = np.array([0.25 * n, 0.1 * n, 3.0, 0.4, 0.0])
+    fcrit = np.array([-1e30, -1e30, -1e30, 0.5, 0.5], np.float32)
+    pk = ctx.find_peaks(torch.as_tensor(delta, device="cuda"), box, Rf, fcrit, want_lapd=True, nbuff=nbuff)
+    assert set(pk.filt.tolist()) >= {1, 2, 3}
+    dk = ctx.rfft(delta)
+    for f, R in enumerate(Rf):
+        at = pk.filt == f
+        s = ctx.smooth_field(dk, n, box, R, 3)
+        np.testing.assert_array_equal(pk.lapd_s[at], s[pk.k[at], pk.j[at], pk.i[at]])
+        _close(f"R={R}", s, O.smooth_field(dk, n, box, R, 3))
