@@ -145,7 +145,7 @@ struct pp_ctx {
     unsigned long long fft_clock = 0;
     // scratch
     pp::DevBuf d_field_a, d_field_b, d_k0, d_k1, d_k2, d_mask, d_misc, d_peaks, d_scan, d_cub;
-    pp::DevBuf d_in[8], d_pk, d_res, d_prof, d_queue, d_walk, d_spec;
+    pp::DevBuf d_in[8], d_pk, d_res, d_prof, d_queue, d_walk, d_cross, d_spec;
     pp::LinePlan *line_cache = nullptr;  // [kLineCache]
     // persistent-form tunables (pp_autotune_shell): small-peak threshold in
     // finalised shells (several peaks per wave), shells per LDS chunk of the
@@ -154,7 +154,7 @@ struct pp_ctx {
     // the post below that count
     int tiny_m = 16;
     int chunk_shells = 64;
-    int coop_m = 64;
+    int coop_m = 1 << 20;
     int gather_waves_cu = 16;
     int post_width = 1;  // lanes per peak of the post below coop_m (1, 4, 8, 16)
     int lane_walk = 0;   // lane post: walks longer than this go to the wave post (0: no limit)

@@ -699,6 +699,8 @@ constexpr int kSmallGridCU = 32;
 constexpr int kWaveGridCU = 16;
 constexpr int kFinishGridCU = 256;
 constexpr int kLaneGridCU = 64;
+constexpr int64_t kWalkBound = 1ll << 26;  // walk records (64 B) reserved from their bound alone
+constexpr int kLaneTableMin = 64;  // a lane class of at most so many peaks gets no order and no walk table
 constexpr int kWalkGridCU = 16;  // 256-lane workgroups per CU of the walk table (grid-stride over the peaks)
 
 // The lane post's order: m descending, then the fcrit crossing descending,
@@ -1406,7 +1408,16 @@ static int run_persistent_impl(pp_ctx *ctx, GatherFields G, ShellRun &S, PostCon
     // lane per peak
     const int small_m = export_all ? 0 : std::min(std::max(ctx->tiny_m, 0), st.small_max);
     const int64_t small_lo = cnt_gt(small_m);
-    const int64_t coop_end = std::min(small_lo, cnt_gt(std::max(ctx->coop_m, 1)));
+    // One lane per peak wins at every batch measured once the walk table feeds
+    // it (wave post for m > 64 against none, whole call: 1.95 M peaks of a
+    // 512^3 tile 21.6 -> 15.5 ms, 180 k of 256^3 4.55 -> 3.36, 9 k large ones
+    // 5.44 -> 4.24, 2 k of 128^3 2.08 -> 2.03), so coop_m starts above every m.
+    // A class too small for the table (cross_order below) would leave its
+    // largest peaks to single lanes: those go to the wave post.
+    int coop_m = std::max(ctx->coop_m, 1);
+    if (ctx->post_width <= 1 && small_lo - std::min(small_lo, cnt_gt(coop_m)) <= kLaneTableMin)
+        coop_m = std::min(coop_m, 64);
+    const int64_t coop_end = std::min(small_lo, cnt_gt(coop_m));
     // 3. profile offsets: exclusive scan of m over all peaks
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
     int64_t tot = 0;
@@ -1541,7 +1552,7 @@ static int run_persistent_impl(pp_ctx *ctx, GatherFields G, ShellRun &S, PostCon
     const int32_t *cross_list = nullptr;
     const int64_t cross_lo = coop_end, cross_hi = small_lo;
     int cmax = 1, cbits = 1;  // the class's largest m; the keys take 2 * cbits bits
-    for (int x = std::min(std::max(ctx->coop_m, 1), nb - 1); x > small_m; x--)
+    for (int x = std::min(coop_m, nb - 1); x > small_m; x--)
         if (hist[x]) { cmax = x; break; }
     while ((1 << cbits) <= cmax) cbits++;
     // The walk table of the same class (k_walk_strain): per peak its crossing
@@ -1553,11 +1564,12 @@ static int run_persistent_impl(pp_ctx *ctx, GatherFields G, ShellRun &S, PostCon
     for (int x = small_m + 1; x <= cmax && x < nb; x++) wrec_max += (int64_t)hist[x] * x;
     auto cross_order = [&]() -> int {
         const int64_t nl = cross_hi - cross_lo;
-        if (ctx->post_width > 1 || nl <= 64) return PP_OK;
-        PP_CHECK(ctx->d_walk.grow(al((size_t)nl * 8) * 2 + (size_t)std::max<int64_t>(wrec_max, 1) * sizeof(WalkRec)));
-        d_wmc = ctx->d_walk.as<int64_t>();
-        d_weoff = (int64_t *)(ctx->d_walk.as<char>() + al((size_t)nl * 8));
-        d_wtab = (WalkRec *)(ctx->d_walk.as<char>() + 2 * al((size_t)nl * 8));
+        if (ctx->post_width > 1 || nl <= kLaneTableMin) return PP_OK;
+        // crossings and offsets apart from the records, whose number is only
+        // bounded here
+        PP_CHECK(ctx->d_cross.grow(al((size_t)nl * 8) * 2));
+        d_wmc = ctx->d_cross.as<int64_t>();
+        d_weoff = (int64_t *)(ctx->d_cross.as<char>() + al((size_t)nl * 8));
         uint32_t *ka = (uint32_t *)W.ka, *kb = (uint32_t *)W.kb;
         hipLaunchKernelGGL(k_crossing_keys, dim3(grid1d(ctx, nl)), dim3(256), 0, ctx->stream, (const PeakParam *)pps,
                            cross_lo, cross_hi, d_rec, (const int64_t *)d_off, C.rad, cmax, cbits, ka, d_wmc);
@@ -1577,7 +1589,20 @@ static int run_persistent_impl(pp_ctx *ctx, GatherFields G, ShellRun &S, PostCon
     };
     // the walk table's records (after the gather's profiles and the crossings)
     auto walk_table = [&]() -> int {
-        if (!d_wtab) return PP_OK;
+        if (!d_wmc) return PP_OK;
+        int64_t nrec_w = wrec_max;
+        if (wrec_max > kWalkBound) {
+            // many large peaks: the crossings lie far inside them, so the exact
+            // number (one read-back) saves most of the memory
+            const int64_t nl = cross_hi - cross_lo;
+            int64_t last[2];
+            PP_HIP(hipMemcpyAsync(&last[0], d_weoff + nl - 1, 8, hipMemcpyDeviceToHost, ctx->stream));
+            PP_HIP(hipMemcpyAsync(&last[1], d_wmc + nl - 1, 8, hipMemcpyDeviceToHost, ctx->stream));
+            PP_HIP(hipStreamSynchronize(ctx->stream));
+            nrec_w = last[0] + last[1];
+        }
+        PP_CHECK(ctx->d_walk.grow((size_t)std::max<int64_t>(nrec_w, 1) * sizeof(WalkRec)));
+        d_wtab = ctx->d_walk.as<WalkRec>();
         // classes: consecutive runs of the lane-post order (m descending)
         WalkClasses K{};
         int64_t want[kWalkClasses], tot = 0, pos = 0;
