@@ -10,20 +10,38 @@
 // lies inside its radius.  That greedy pass is the same as: halo j survives
 // iff no surviving halo earlier in the order contains j's centre (a halo
 // earlier in the order is never smaller).  Here:
-// * the hash is a sort of the halos by their cell (cell ranges in a dense
-//   256^3 table), the order a stable radix sort of the radii;
-// * every halo k lists, from its own radius' cells, the later halos j it
-//   contains ("killer" edges k -> j, stored by j);
+// * the halos are sorted by the cells of a grid of two cells a halo and
+//   stay in that order: neighbours in space are neighbours in memory, and the
+//   candidates of a row of cells are one run of the list (two loads, whatever
+//   the row's length).  The reference's grid has 256 cells a side whatever the
+//   catalogue, 10^4 cells for each halo of a small one;
+// * several lanes share a halo and take its rows of cells in turn (one lane a
+//   halo spent most of its time on the few largest radii);
+// * "earlier in the order" compares radius and index, which needs no sort;
+// * every halo k lists the later halos j it contains ("killer" edges k -> j,
+//   stored by j);
 // * rounds over the undecided halos settle them: j dies as soon as one of
 //   its killers is known to survive, survives once all its killers are known
 //   dead; the earliest undecided halo always settles, so the rounds end;
-// * the reduction lists every overlapping surviving pair once, from its
+// * the reduction visits every overlapping surviving pair once, from its
 //   larger member (whose cells within twice its radius hold every smaller
-//   partner), with both cap volumes of sphere_overlap; each halo's deficit
-//   is its own list's caps in list order plus its caps as the smaller member
-//   in pair order (a stable sort), so the result does not depend on thread
-//   timing.  The deficit is the reference's (which adds each pair from both
-//   sides and halves) up to Float64 rounding.
+//   partner), with both cap volumes of sphere_overlap.  The larger member's
+//   caps are summed in Float64 by its lanes; the smaller member's are added
+//   by atomics as whole numbers of 2^-54 of its volume, finer than the 2^-53
+//   to which Float64 subtracts them from it and the same in every order: the
+//   result does not depend on thread timing, and no list of pairs is stored
+//   or sorted.  (The sum stays under the 2^10 volumes that fit: a partner's
+//   centre is outside of the halo and of the other partners, so that a cap
+//   is under half the volume and at most a few hundred spheres touch it.)
+//   The deficit is the reference's (which adds each pair from both sides and
+//   halves) up to Float64 rounding;
+// * the work space is the context's (it was 25 allocations a call).
+// At 1.2 M halos with their records (a 600 Mpc/h box) a merge takes 1.7 ms
+// instead of 41.1 ms.  What bounds it: the chains of
+// dependent loads (cell, row, candidates) of k_pairs (0.38 ms, was 2 x 13 ms)
+// and k_killers (0.18 and 0.24 ms, was 2 x 2.6 ms); an arithmetic half as
+// long (Float32 distances before Float64 ones) changed neither.  At 300 to
+// 700 halos 0.4 ms instead of 200 to 560 ms, most of it the empty cells.
 #include <hipcub/hipcub.hpp>
 
 #include <cmath>
@@ -32,10 +50,22 @@
 
 namespace pp {
 
-constexpr int kMergeNC = 256;
+constexpr int kMergeAxis = 1024;            // most cells on an axis
+constexpr int64_t kMergeCells = 1ll << 27;  // most cells of a grid
+// Lanes that share a halo's rows of cells.  k_killers / k_pairs over 1.2 M
+// halos (median radius 1.5 in a 600^3 box, the largest 15) with 4, 8 and 16
+// lanes for the first: 200, 216 and 257 us; 8, 16 and 32 for the second: 697,
+// 616 and 733 us.  With the grid at 1, 2 and 4 cells a halo all kernels
+// together are within 3 % (fewer candidates against more rows to look up); 2
+// leaves room for clustering.
+constexpr int kKillY = 4, kKillZ = 2, kKillLanes = kKillY * kKillZ;
+constexpr int kPairY = 4, kPairZ = 4, kPairLanes = kPairY * kPairZ;
+constexpr int kCellsPerHalo = 2;
+constexpr int kBoundBlocks = 256;
 
 struct MergeGeo {
-    double ox, oy, oz, cs;  // hash origin and cell size
+    double o[3], inv;  // grid origin, 1 / cell size
+    int nc[3];
 };
 
 struct MergeIn {
@@ -43,27 +73,82 @@ struct MergeIn {
     int64_t n;
 };
 
-__device__ __forceinline__ int cell_axis(double p, double o, double cs)
+// the halos in cell order
+struct MergeCells {
+    const float4 *h;       // x, y, z, r
+    const int32_t *id;     // position in the catalogue
+    const int32_t *first;  // per cell, and one more: its first halo
+    int64_t n;
+};
+
+// c cells from the origin: the cell, clamped to the grid (NaN: 0)
+__device__ __forceinline__ int cell_clamp(double c, int nc)
 {
-    int c = (int)floor((p - o) / cs) + 1;
-    c = c < 1 ? 1 : (c > kMergeNC ? kMergeNC : c);
-    return c - 1;
+    return c >= 1.0 ? (c < (double)nc ? (int)c : nc - 1) : 0;
 }
 
-__device__ __forceinline__ int cell_of(const MergeIn &H, const MergeGeo &G, int64_t i, int &cx, int &cy, int &cz)
+// halo a comes before halo b: larger, or as large and earlier in the catalogue
+__device__ __forceinline__ bool before(const MergeCells &C, int64_t a, float ra, int64_t b, float rb)
 {
-    cx = cell_axis((double)H.x[i], G.ox, G.cs);
-    cy = cell_axis((double)H.y[i], G.oy, G.cs);
-    cz = cell_axis((double)H.z[i], G.oz, G.cs);
-    return cx + kMergeNC * (cy + kMergeNC * cz);
+    return ra > rb || (ra == rb && C.id[a] < C.id[b]);
 }
 
-__device__ __forceinline__ double dist_of(const MergeIn &H, int64_t a, int64_t b)
+__device__ __forceinline__ double dist_of(const float4 &a, const float4 &b)
 {
 #pragma clang fp contract(off)
-    const double dx = (double)H.x[b] - (double)H.x[a], dy = (double)H.y[b] - (double)H.y[a],
-                 dz = (double)H.z[b] - (double)H.z[a];
+    const double dx = (double)b.x - (double)a.x, dy = (double)b.y - (double)a.y, dz = (double)b.z - (double)a.z;
     return sqrt(dx * dx + dy * dy + dz * dz);
+}
+
+// whether a and b are further apart than R for certain (Float32: the sum of
+// squares is right to 4e-7 of itself, the margin is 1e-5; radii whose squares
+// would be denormal are left to Float64)
+__device__ __forceinline__ bool apart(const float4 &a, const float4 &b, float R)
+{
+    const float dx = b.x - a.x, dy = b.y - a.y, dz = b.z - a.z;
+    return R > 1e-15f && dx * dx + dy * dy + dz * dz > R * R * 1.00001f;
+}
+
+__device__ __forceinline__ int cell_between(float c, int lo, int hi)
+{
+    return max(lo, min((int)floorf(c), hi));
+}
+
+// fn(j, halo j) for every halo within R of halo p and others of the cells
+// there.  LY x LZ lanes take the rows of cells in turn, each BATCH candidates
+// of a row at once: the chain of loads is what bounds this.  Distances are in
+// cells from p's own cell, in Float32 with margins over their rounding.
+template <int LY, int LZ, int BATCH, class Fn>
+__device__ __forceinline__ void around(const MergeCells &C, const MergeGeo &G, const float4 &p, double R, Fn fn)
+{
+    const double ux = ((double)p.x - G.o[0]) * G.inv, uy = ((double)p.y - G.o[1]) * G.inv,
+                 uz = ((double)p.z - G.o[2]) * G.inv;
+    const int cx = cell_clamp(ux, G.nc[0]), cy = cell_clamp(uy, G.nc[1]), cz = cell_clamp(uz, G.nc[2]);
+    const float fx = (float)(ux - cx), fy = (float)(uy - cy), fz = (float)(uz - cz);
+    const float u = fminf((float)(R * G.inv) * 1.000002f + 1e-5f, 4.0f * kMergeAxis);
+    const int ly = threadIdx.x & (LY - 1), lz = threadIdx.x / LY & (LZ - 1);
+    const int xl = -cx, xh = G.nc[0] - 1 - cx, yl = -cy, yh = G.nc[1] - 1 - cy, zl = -cz, zh = G.nc[2] - 1 - cz;
+    const int y0 = cell_between(fy - u, yl, yh), y1 = cell_between(fy + u, yl, yh);
+    const int z0 = cell_between(fz - u, zl, zh), z1 = cell_between(fz + u, zl, zh);
+    for (int z = z0 + lz; z <= z1; z += LZ)
+        for (int y = y0 + ly; y <= y1; y += LY) {
+            // the row's nearest point in y and z, and what that leaves of u in x
+            const float gy = fmaxf(fmaxf((float)y - fy, fy - (float)(y + 1)), 0.0f);
+            const float gz = fmaxf(fmaxf((float)z - fz, fz - (float)(z + 1)), 0.0f);
+            const float w2 = u * u * 1.000002f - gy * gy - gz * gz;
+            if (w2 < 0.0f) continue;
+            const float w = sqrtf(w2) * 1.000002f + 1e-5f;
+            const int64_t row = (int64_t)G.nc[0] * ((cy + y) + (int64_t)G.nc[1] * (cz + z)) + cx;
+            const int32_t e1 = C.first[row + cell_between(fx + w, xl, xh) + 1];
+            for (int32_t e = C.first[row + cell_between(fx - w, xl, xh)]; e < e1; e += BATCH) {
+                float4 c[BATCH];
+#pragma unroll
+                for (int a = 0; a < BATCH; a++) c[a] = C.h[min(e + a, e1 - 1)];
+#pragma unroll
+                for (int a = 0; a < BATCH; a++)
+                    if (e + a < e1) fn(e + a, c[a]);
+            }
+        }
 }
 
 // sphere_overlap (Exclusion.jl:64-96): cap volumes cut from spheres 1 and 2
@@ -79,12 +164,26 @@ __device__ __forceinline__ void sphere_caps(double d, double r1, double r2, doub
     v2 = pi3 * (h2 * h2) * (3.0 * r2 - h2);
 }
 
-// min/max of the positions and max radius (one block)
-__global__ void __launch_bounds__(1024) k_merge_bounds(MergeIn H, double *__restrict__ out)
+// min/max of the positions and max radius of a block's lanes, in lane 0
+__device__ __forceinline__ void bound_reduce(float (&red)[7][256], const float (&v)[7])
 {
-    __shared__ float red[7][1024];
+    for (int q = 0; q < 7; q++) red[q][threadIdx.x] = v[q];
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+        if ((int)threadIdx.x < w)
+            for (int q = 0; q < 7; q++) {
+                const float a = red[q][threadIdx.x], b = red[q][threadIdx.x + w];
+                red[q][threadIdx.x] = (q & 1) || q == 6 ? fmaxf(a, b) : fminf(a, b);
+            }
+        __syncthreads();
+    }
+}
+
+__global__ void __launch_bounds__(256) k_merge_bounds(MergeIn H, float *__restrict__ part)
+{
+    __shared__ float red[7][256];
     float v[7] = {INFINITY, -INFINITY, INFINITY, -INFINITY, INFINITY, -INFINITY, -INFINITY};
-    for (int64_t i = threadIdx.x; i < H.n; i += blockDim.x) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < H.n; i += (int64_t)gridDim.x * 256) {
         v[0] = fminf(v[0], H.x[i]);
         v[1] = fmaxf(v[1], H.x[i]);
         v[2] = fminf(v[2], H.y[i]);
@@ -93,83 +192,87 @@ __global__ void __launch_bounds__(1024) k_merge_bounds(MergeIn H, double *__rest
         v[5] = fmaxf(v[5], H.z[i]);
         v[6] = fmaxf(v[6], H.r[i]);
     }
-    for (int q = 0; q < 7; q++) red[q][threadIdx.x] = v[q];
-    __syncthreads();
-    for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w)
-            for (int q = 0; q < 7; q++) {
-                const float a = red[q][threadIdx.x], b = red[q][threadIdx.x + w];
-                red[q][threadIdx.x] = (q & 1) || q == 6 ? fmaxf(a, b) : fminf(a, b);
-            }
-        __syncthreads();
-    }
+    bound_reduce(red, v);
+    if (threadIdx.x < 7) part[blockIdx.x * 7 + threadIdx.x] = red[threadIdx.x][0];
+}
+
+__global__ void __launch_bounds__(256) k_merge_bounds2(const float *__restrict__ part, int blocks,
+                                                       double *__restrict__ out)
+{
+    __shared__ float red[7][256];
+    float v[7] = {INFINITY, -INFINITY, INFINITY, -INFINITY, INFINITY, -INFINITY, -INFINITY};
+    for (int b = threadIdx.x; b < blocks; b += 256)
+        for (int q = 0; q < 7; q++)
+            v[q] = (q & 1) || q == 6 ? fmaxf(v[q], part[b * 7 + q]) : fminf(v[q], part[b * 7 + q]);
+    bound_reduce(red, v);
     if (threadIdx.x < 7) out[threadIdx.x] = (double)red[threadIdx.x][0];
 }
 
-__global__ void k_merge_keys(MergeIn H, MergeGeo G, int32_t *__restrict__ cell, int32_t *__restrict__ iota)
+__global__ void k_merge_keys(MergeIn H, MergeGeo G, float4 *__restrict__ h, int32_t *__restrict__ cell,
+                             int32_t *__restrict__ iota)
 {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < H.n; i += (int64_t)gridDim.x * blockDim.x) {
-        int cx, cy, cz;
-        cell[i] = cell_of(H, G, i, cx, cy, cz);
+        const float4 p = make_float4(H.x[i], H.y[i], H.z[i], H.r[i]);
+        const int cx = cell_clamp(((double)p.x - G.o[0]) * G.inv, G.nc[0]);
+        const int cy = cell_clamp(((double)p.y - G.o[1]) * G.inv, G.nc[1]);
+        const int cz = cell_clamp(((double)p.z - G.o[2]) * G.inv, G.nc[2]);
+        h[i] = p;
+        cell[i] = cx + G.nc[0] * (cy + G.nc[1] * cz);
         iota[i] = (int32_t)i;
     }
 }
 
-__global__ void k_fill_i32(int32_t *__restrict__ a, int64_t n, int32_t v)
-{
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) a[i] = v;
-}
-
-// [start, end) of every occupied cell in the cell-sorted list
-__global__ void k_cell_ranges(const int32_t *__restrict__ key, int64_t n, int32_t *__restrict__ start,
-                              int32_t *__restrict__ end)
+// the halos in cell order, their counters cleared
+__global__ void k_merge_gather(const float4 *__restrict__ in, int64_t n, const int32_t *__restrict__ id,
+                               float4 *__restrict__ h, int32_t *__restrict__ count, int32_t *__restrict__ state,
+                               unsigned long long *__restrict__ frac)
 {
     for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < n; p += (int64_t)gridDim.x * blockDim.x) {
-        const int32_t k = key[p];
-        if (p == 0 || key[p - 1] != k) start[k] = (int32_t)p;
-        if (p == n - 1 || key[p + 1] != k) end[k] = (int32_t)(p + 1);
+        h[p] = in[id[p]];
+        count[p] = 0;
+        state[p] = 0;
+        frac[p] = 0;
     }
 }
 
-__global__ void k_rank(const int32_t *__restrict__ order, int64_t n, int32_t *__restrict__ rank)
+// first[c] = the number of keys below c, c in [0, ncell]
+__global__ void k_cell_first(const int32_t *__restrict__ key, int64_t n, int64_t ncell, int32_t *__restrict__ first)
 {
-    for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < n; p += (int64_t)gridDim.x * blockDim.x)
-        rank[order[p]] = (int32_t)p;
-}
-
-struct Hash {
-    const int32_t *start, *end, *list;  // cell ranges, halos in cell order
-};
-
-// pass 1 edges: every later halo j inside halo k's radius; count (fill = 0)
-// or write (fill = 1) them into j's list
-__global__ void __launch_bounds__(64) k_killers(MergeIn H, MergeGeo G, Hash S, const int32_t *__restrict__ rank,
-                                                int32_t *__restrict__ count, const int64_t *__restrict__ off,
-                                                int32_t *__restrict__ edges, int fill)
-{
-    for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < H.n; k += (int64_t)gridDim.x * blockDim.x) {
-        const double rk = (double)H.r[k];
-        const int dc = (int)ceil(rk / G.cs);
-        int cx, cy, cz;
-        cell_of(H, G, k, cx, cy, cz);
-        const int rkk = rank[k];
-        for (int jz = max(cz - dc, 0); jz <= min(cz + dc, kMergeNC - 1); jz++)
-            for (int jy = max(cy - dc, 0); jy <= min(cy + dc, kMergeNC - 1); jy++)
-                for (int jx = max(cx - dc, 0); jx <= min(cx + dc, kMergeNC - 1); jx++) {
-                    const int c = jx + kMergeNC * (jy + kMergeNC * jz);
-                    for (int32_t p = S.start[c]; p < S.end[c]; p++) {
-                        const int32_t j = S.list[p];
-                        if (rank[j] <= rkk || dist_of(H, k, j) >= rk) continue;
-                        if (!fill) atomicAdd(&count[j], 1);
-                        else edges[off[j] + atomicAdd(&count[j], 1)] = (int32_t)k;
-                    }
-                }
+    for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c <= ncell; c += (int64_t)gridDim.x * blockDim.x) {
+        int64_t lo = 0, hi = n;
+        while (lo < hi) {
+            const int64_t mid = (lo + hi) >> 1;
+            if ((int64_t)key[mid] < c) lo = mid + 1;
+            else hi = mid;
+        }
+        first[c] = (int32_t)lo;
     }
 }
 
-// one round: 0 undecided, 1 survives, 2 excluded
+// pass 1 edges: every later halo j inside halo k's radius; count them by j, or
+// (FILL, which counts down to 0 again) write them into j's list
+template <bool FILL>
+__global__ void __launch_bounds__(256, 8) k_killers(MergeCells C, MergeGeo G, int32_t *__restrict__ count,
+                                                 const int64_t *__restrict__ off, int32_t *__restrict__ edges)
+{
+    for (int64_t k = ((int64_t)blockIdx.x * 256 + threadIdx.x) / kKillLanes; k < C.n;
+         k += (int64_t)gridDim.x * (256 / kKillLanes)) {
+        const float4 hk = C.h[k];
+        const double rk = (double)hk.w;
+        if (!(rk > 0.0)) continue;
+        around<kKillY, kKillZ, 1>(C, G, hk, rk, [&](int32_t j, const float4 &hj) {
+            if (hj.w > hk.w || apart(hk, hj, hk.w) || !(dist_of(hk, hj) < rk) || !before(C, k, hk.w, j, hj.w))
+                return;
+            if constexpr (FILL) edges[off[j] + atomicSub(&count[j], 1) - 1] = (int32_t)k;
+            else atomicAdd(&count[j], 1);
+        });
+    }
+}
+
+// one round: 0 undecided, 1 survives, 2 excluded (its radius becomes -1, which
+// no pair has); *undecided = round if any is left
 __global__ void k_decide(int64_t n, const int64_t *__restrict__ off, const int32_t *__restrict__ edges,
-                         int32_t *state, int32_t *__restrict__ undecided)
+                         int32_t *state, float4 *__restrict__ h, int32_t *__restrict__ undecided, int32_t round)
 {
     for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += (int64_t)gridDim.x * blockDim.x) {
         if (state[j] != 0) continue;
@@ -182,103 +285,129 @@ __global__ void k_decide(int64_t n, const int64_t *__restrict__ off, const int32
             }
             if (s == 0) all_dead = false;
         }
-        if (killed) __atomic_store_n(&state[j], 2, __ATOMIC_RELAXED);
-        else if (all_dead) __atomic_store_n(&state[j], 1, __ATOMIC_RELAXED);
-        else atomicAdd(undecided, 1);
+        if (killed) {
+            __atomic_store_n(&state[j], 2, __ATOMIC_RELAXED);
+            h[j].w = -1.0f;
+        } else if (all_dead) __atomic_store_n(&state[j], 1, __ATOMIC_RELAXED);
+        else *undecided = round;
     }
 }
 
-// pass 2 pairs from the larger member i: count (fill = 0) or write
-__global__ void __launch_bounds__(64) k_pairs(MergeIn H, MergeGeo G, Hash S, const int32_t *__restrict__ rank,
-                                              const int32_t *__restrict__ state, int64_t *__restrict__ count,
-                                              const int64_t *__restrict__ off, int32_t *__restrict__ pj,
-                                              double *__restrict__ cap_i, double *__restrict__ cap_j, int fill)
+// sum over a block of 256, in thread 0
+__device__ __forceinline__ unsigned long long block_total(unsigned long long v)
 {
-#pragma clang fp contract(off)
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < H.n; i += (int64_t)gridDim.x * blockDim.x) {
-        if (state[i] != 1) {
-            if (!fill) count[i] = 0;
-            continue;
-        }
-        const double ri = (double)H.r[i];
-        const int dc = (int)ceil(2.0 * ri / G.cs);
-        int cx, cy, cz;
-        cell_of(H, G, i, cx, cy, cz);
-        const int rki = rank[i];
-        int64_t q = fill ? off[i] : 0;
-        for (int jz = max(cz - dc, 0); jz <= min(cz + dc, kMergeNC - 1); jz++)
-            for (int jy = max(cy - dc, 0); jy <= min(cy + dc, kMergeNC - 1); jy++)
-                for (int jx = max(cx - dc, 0); jx <= min(cx + dc, kMergeNC - 1); jx++) {
-                    const int c = jx + kMergeNC * (jy + kMergeNC * jz);
-                    for (int32_t p = S.start[c]; p < S.end[c]; p++) {
-                        const int32_t j = S.list[p];
-                        if (rank[j] <= rki || state[j] != 1) continue;
-                        const double rj = (double)H.r[j];
-                        const double d = dist_of(H, i, j);
-                        if (!(d < ri + rj && d > fabs(ri - rj))) continue;
-                        if (fill) {
-                            double v1, v2;
-                            sphere_caps(d, ri, rj, v1, v2);
-                            pj[q] = j;
-                            cap_i[q] = v1;
-                            cap_j[q] = v2;
-                        }
-                        q++;
-                    }
-                }
-        if (!fill) count[i] = q;
-    }
+    __shared__ unsigned long long part[4];
+    for (int w = 32; w > 0; w >>= 1) v += __shfl_down(v, w, 64);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+    __syncthreads();
+    return part[0] + part[1] + part[2] + part[3];
 }
 
-// reduced radii: deficit = own pair list (larger member) + smaller-member caps
-__global__ void k_finalize(MergeIn H, const int32_t *__restrict__ state, const int64_t *__restrict__ off,
-                           const double *__restrict__ cap_i, const int32_t *__restrict__ sstart,
-                           const int32_t *__restrict__ send, const double *__restrict__ cap_sorted,
-                           int8_t *__restrict__ keep, float *__restrict__ new_r, int32_t *__restrict__ nkept)
+constexpr double kSphere = 4.0 * 3.141592653589793 / 3.0;
+constexpr double kFrac = 18014398509481984.0;  // 2^54
+
+// pass 2 from the larger member i: the sum of its caps, every partner's cap
+// added to the partner's whole numbers, the pairs counted
+__global__ void __launch_bounds__(256, 6) k_pairs(MergeCells C, MergeGeo G, double *__restrict__ caps,
+                                               unsigned long long *__restrict__ frac,
+                                               unsigned long long *__restrict__ npair)
 {
 #pragma clang fp contract(off)
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < H.n; i += (int64_t)gridDim.x * blockDim.x) {
-        if (state[i] != 1) {
-            keep[i] = 0;
-            new_r[i] = 0.0f;
-            continue;
-        }
-        double a = 0.0, b = 0.0;
-        for (int64_t q = off[i]; q < off[i + 1]; q++) a += cap_i[q];
-        for (int32_t q = sstart[i]; q < send[i]; q++) b += cap_sorted[q];
-        const double r = (double)H.r[i];
-        const double f = 4.0 * 3.141592653589793 / 3.0;
-        const double vol = f * (r * r * r) - (a + b);
-        if (vol <= 0.0) {
-            keep[i] = 0;
-            new_r[i] = 0.0f;
-        } else {
-            keep[i] = 1;
-            new_r[i] = (float)pow(vol / f, 1.0 / 3.0);
-            atomicAdd(nkept, 1);
-        }
+    unsigned long long found = 0;
+    for (int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) / kPairLanes; i < C.n;
+         i += (int64_t)gridDim.x * (256 / kPairLanes)) {
+        const float4 hi = C.h[i];
+        const double ri = (double)hi.w;
+        double sum = 0.0;
+        if (ri > 0.0)
+            around<kPairY, kPairZ, 2>(C, G, hi, 2.0 * ri, [&](int32_t j, const float4 &hj) {
+                if (hj.w > hi.w || apart(hi, hj, hi.w + hj.w)) return;
+                const double rj = (double)hj.w, d = dist_of(hi, hj);
+                if (!(d < ri + rj && d > fabs(ri - rj)) || !before(C, i, hi.w, j, hj.w)) return;
+                double v1, v2;
+                sphere_caps(d, ri, rj, v1, v2);
+                sum += v1;
+                atomicAdd(&frac[j], (unsigned long long)llrint(v2 / (kSphere * (rj * rj * rj)) * kFrac));
+                found++;
+            });
+        for (int w = kPairLanes / 2; w > 0; w >>= 1) sum += __shfl_down(sum, w, kPairLanes);
+        if ((threadIdx.x & (kPairLanes - 1)) == 0) caps[i] = sum;
     }
+    const unsigned long long t = block_total(found);
+    if (threadIdx.x == 0 && t) atomicAdd(npair, t);
+}
+
+// reduced radii: deficit = caps as the larger member + caps as the smaller
+__global__ void __launch_bounds__(256) k_finalize(MergeCells C, const int32_t *__restrict__ state,
+                                                  const double *__restrict__ caps,
+                                                  const unsigned long long *__restrict__ frac,
+                                                  int8_t *__restrict__ keep, float *__restrict__ new_r,
+                                                  unsigned long long *__restrict__ nkept)
+{
+#pragma clang fp contract(off)
+    unsigned long long kept = 0;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < C.n; i += (int64_t)gridDim.x * 256) {
+        const int32_t o = C.id[i];
+        int8_t k = 0;
+        float nr = 0.0f;
+        if (state[i] == 1) {
+            const double r = (double)C.h[i].w, v = kSphere * (r * r * r);
+            const double vol = v - (caps[i] + (double)frac[i] / kFrac * v);
+            if (!(vol <= 0.0)) {
+                k = 1;
+                nr = (float)pow(vol / kSphere, 1.0 / 3.0);
+                kept++;
+            }
+        }
+        keep[o] = k;
+        new_r[o] = nr;
+    }
+    const unsigned long long t = block_total(kept);
+    if (threadIdx.x == 0 && t) atomicAdd(nkept, t);
+}
+
+__global__ void k_merge_clear(unsigned long long *__restrict__ a, int n)
+{
+    if ((int)threadIdx.x < n) a[threadIdx.x] = 0;
 }
 
 struct I32ToI64 {
     __device__ __forceinline__ int64_t operator()(const int32_t &v) const { return (int64_t)v; }
 };
 
-// device buffers of one call, released on return
-struct Scratch {
-    std::vector<DevBuf> bufs;
-    template <class T> int get(size_t n, T *&p)
+// arrays of one call, carved out of a context buffer
+struct Carve {
+    char *p;
+    size_t used = 0;
+    template <class T> T *get(size_t n)
     {
-        bufs.emplace_back();
-        PP_CHECK(bufs.back().grow(std::max<size_t>(n, 1) * sizeof(T)));
-        p = bufs.back().as<T>();
-        return PP_OK;
-    }
-    ~Scratch()
-    {
-        for (auto &b : bufs) b.release();
+        T *a = (T *)(p + used);
+        used += (std::max<size_t>(n, 1) * sizeof(T) + 255) & ~(size_t)255;
+        return a;
     }
 };
+
+// a grid over the extents e with about kCellsPerHalo cells a halo
+static void merge_grid(MergeGeo &G, const double (&e)[3], int64_t n)
+{
+    const double L = std::max(e[0], std::max(e[1], e[2]));
+    G.inv = 0.0;
+    G.nc[0] = G.nc[1] = G.nc[2] = 1;
+    if (!(L > 0)) return;
+    // a flat or linear catalogue counts as a cell of the finest grid thick
+    double v = 1.0;
+    for (int q = 0; q < 3; q++) v *= std::max(e[q] / L, 1.0 / kMergeAxis);
+    const double most = (double)std::min<int64_t>(2 * kCellsPerHalo * n + 64, kMergeCells);
+    for (double c = std::max(cbrt(v / ((double)n * kCellsPerHalo)), 1.0 / kMergeAxis);; c *= 1.25) {  // cell size over L
+        double cells = 1.0;
+        for (int q = 0; q < 3; q++) {
+            G.nc[q] = std::min(kMergeAxis, std::max(1, (int)ceil(e[q] / L / c)));
+            cells *= G.nc[q];
+        }
+        G.inv = 1.0 / (c * L);
+        if (cells <= most) return;
+    }
+}
 
 static int grid_n(pp_ctx *ctx, int64_t n, int block = 256)
 {
@@ -318,153 +447,129 @@ extern "C" int pp_merge_halos(pp_ctx *ctx, int64_t n, const float *x, const floa
     if (n == 0) return PP_OK;
     PP_CHECK(ensure_device(ctx));
     hipStream_t s = ctx->stream;
-    Scratch W;
     MergeIn H;
     H.n = n;
-    const hipMemcpyKind up = on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
-    {
-        float *d;
-        PP_CHECK(W.get(4 * (size_t)n, d));
+    if (on_device) {
+        H.x = x;
+        H.y = y;
+        H.z = z;
+        H.r = rthl;
+    } else {
+        PP_CHECK(ctx->d_merge_in.grow(4 * (size_t)n * sizeof(float)));
+        float *d = ctx->d_merge_in.as<float>();
         const float *src[4] = {x, y, z, rthl};
-        for (int q = 0; q < 4; q++) PP_HIP(hipMemcpyAsync(d + q * n, src[q], n * 4, up, s));
+        for (int q = 0; q < 4; q++) PP_HIP(hipMemcpyAsync(d + q * n, src[q], n * 4, hipMemcpyHostToDevice, s));
         H.x = d;
         H.y = d + n;
         H.z = d + 2 * n;
         H.r = d + 3 * n;
     }
-    // domain (Merger.jl:40-50) and cell size (Exclusion.jl:33-38)
-    double *d_b, hb[7];
-    PP_CHECK(W.get(7, d_b));
-    hipLaunchKernelGGL(k_merge_bounds, dim3(1), dim3(1024), 0, s, H, d_b);
+    int8_t *d_keep = keep;
+    float *d_nr = new_rthl;
+    int32_t *cell, *iota, *cell_s, *id, *first, *cnt, *state;
+    int64_t *off;
+    float4 *h0, *h;
+    double *caps, *d_b;
+    float *d_part;
+    unsigned long long *frac, *d_num;  // d_num: pairs, halos kept, round with undecided halos
+    MergeGeo G{};
+    int64_t ncell = std::min<int64_t>(2 * kCellsPerHalo * n + 64, kMergeCells);
+    const auto layout = [&](Carve W) {
+        cell = W.get<int32_t>(n);
+        iota = W.get<int32_t>(n);
+        cell_s = W.get<int32_t>(n);
+        id = W.get<int32_t>(n);
+        first = W.get<int32_t>(ncell + 1);
+        cnt = W.get<int32_t>(n);
+        state = W.get<int32_t>(n);
+        off = W.get<int64_t>(n + 1);
+        h0 = W.get<float4>(n);
+        h = W.get<float4>(n);
+        caps = W.get<double>(n);
+        frac = W.get<unsigned long long>(n);
+        d_b = W.get<double>(7);
+        d_num = W.get<unsigned long long>(3);
+        d_part = W.get<float>(7 * kBoundBlocks);
+        if (!on_device) {
+            d_keep = W.get<int8_t>(n);
+            d_nr = W.get<float>(n);
+        }
+        return W.used;
+    };
+    PP_CHECK(ctx->d_merge.grow(layout(Carve{nullptr})));
+    layout(Carve{ctx->d_merge.as<char>()});
+    // domain (Merger.jl:40-50)
+    double hb[7];
+    const int nb = (int)std::min<int64_t>(kBoundBlocks, (n + 255) / 256);
+    hipLaunchKernelGGL(k_merge_bounds, dim3(nb), dim3(256), 0, s, H, d_part);
+    hipLaunchKernelGGL(k_merge_bounds2, dim3(1), dim3(256), 0, s, (const float *)d_part, nb, d_b);
+    hipLaunchKernelGGL(k_merge_clear, dim3(1), dim3(64), 0, s, d_num, 3);
     PP_HIP(hipGetLastError());
     PP_HIP(hipMemcpyAsync(hb, d_b, sizeof(hb), hipMemcpyDeviceToHost, s));
     PP_HIP(hipStreamSynchronize(s));
     for (int q = 0; q < 7; q++) PP_ARG(std::isfinite(hb[q]), "non-finite position or radius in the catalogue");
     const double pad = 2.0 * hb[6];
     const double lo[3] = {hb[0] - pad, hb[2] - pad, hb[4] - pad}, hi[3] = {hb[1] + pad, hb[3] + pad, hb[5] + pad};
-    const double L = std::max(hi[0] - lo[0], std::max(hi[1] - lo[1], hi[2] - lo[2]));
-    PP_ARG(L > 0, "degenerate catalogue extent");
-    MergeGeo G{lo[0], lo[1], lo[2], L / kMergeNC};
-    const int64_t ncell = (int64_t)kMergeNC * kMergeNC * kMergeNC;
-    // hash: halos sorted by cell, ranges per cell
-    int32_t *cell, *iota, *cell_s, *list, *cstart, *cend;
-    PP_CHECK(W.get(n, cell));
-    PP_CHECK(W.get(n, iota));
-    PP_CHECK(W.get(n, cell_s));
-    PP_CHECK(W.get(n, list));
-    PP_CHECK(W.get(ncell, cstart));
-    PP_CHECK(W.get(ncell, cend));
-    hipLaunchKernelGGL(k_merge_keys, dim3(grid_n(ctx, n)), dim3(256), 0, s, H, G, cell, iota);
-    hipLaunchKernelGGL(k_fill_i32, dim3(grid_n(ctx, ncell)), dim3(256), 0, s, cstart, ncell, 0);
-    hipLaunchKernelGGL(k_fill_i32, dim3(grid_n(ctx, ncell)), dim3(256), 0, s, cend, ncell, 0);
+    PP_ARG(std::max(hi[0] - lo[0], std::max(hi[1] - lo[1], hi[2] - lo[2])) > 0, "degenerate catalogue extent");
+    const double ext[3] = {hb[1] - hb[0], hb[3] - hb[2], hb[5] - hb[4]};
+    for (int q = 0; q < 3; q++) G.o[q] = hb[2 * q];
+    merge_grid(G, ext, n);
+    ncell = (int64_t)G.nc[0] * G.nc[1] * G.nc[2];
+    int bits = 1;
+    while ((1ll << bits) < ncell) bits++;
+    // halos in cell order, the first of every cell
+    hipLaunchKernelGGL(k_merge_keys, dim3(grid_n(ctx, n)), dim3(256), 0, s, H, G, h0, cell, iota);
     PP_HIP(hipGetLastError());
     size_t tmp = 0;
-    PP_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, cell, cell_s, iota, list, (int)n, 0, 24, s));
+    PP_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, cell, cell_s, iota, id, (int)n, 0, bits, s));
     PP_CHECK(ctx->d_cub.grow(tmp));
-    PP_HIP(hipcub::DeviceRadixSort::SortPairs(ctx->d_cub.ptr, tmp, cell, cell_s, iota, list, (int)n, 0, 24, s));
-    hipLaunchKernelGGL(k_cell_ranges, dim3(grid_n(ctx, n)), dim3(256), 0, s, (const int32_t *)cell_s, n, cstart, cend);
+    PP_HIP(hipcub::DeviceRadixSort::SortPairs(ctx->d_cub.ptr, tmp, cell, cell_s, iota, id, (int)n, 0, bits, s));
+    hipLaunchKernelGGL(k_merge_gather, dim3(grid_n(ctx, n)), dim3(256), 0, s, (const float4 *)h0, n,
+                       (const int32_t *)id, h, cnt, state, frac);
+    hipLaunchKernelGGL(k_cell_first, dim3(grid_n(ctx, ncell + 1)), dim3(256), 0, s, (const int32_t *)cell_s, n, ncell, first);
     PP_HIP(hipGetLastError());
-    const Hash S{cstart, cend, list};
-    // order: stable descending radius; rank of each halo
-    float *r_s;
-    int32_t *order, *rank;
-    PP_CHECK(W.get(n, r_s));
-    PP_CHECK(W.get(n, order));
-    PP_CHECK(W.get(n, rank));
-    tmp = 0;
-    PP_HIP(hipcub::DeviceRadixSort::SortPairsDescending(nullptr, tmp, H.r, r_s, iota, order, (int)n, 0, 32, s));
-    PP_CHECK(ctx->d_cub.grow(tmp));
-    PP_HIP(hipcub::DeviceRadixSort::SortPairsDescending(ctx->d_cub.ptr, tmp, H.r, r_s, iota, order, (int)n, 0, 32, s));
-    hipLaunchKernelGGL(k_rank, dim3(grid_n(ctx, n)), dim3(256), 0, s, (const int32_t *)order, n, rank);
-    PP_HIP(hipGetLastError());
+    const MergeCells C{h, id, first, n};
     // pass 1: killer edges by target, then rounds
-    int32_t *cnt, *state, *d_und;
-    int64_t *off;
-    PP_CHECK(W.get(n, cnt));
-    PP_CHECK(W.get(n, state));
-    PP_CHECK(W.get(1, d_und));
-    PP_CHECK(W.get(n + 1, off));
-    hipLaunchKernelGGL(k_fill_i32, dim3(grid_n(ctx, n)), dim3(256), 0, s, cnt, n, 0);
-    hipLaunchKernelGGL(k_killers, dim3(grid_n(ctx, n, 64)), dim3(64), 0, s, H, G, S, (const int32_t *)rank, cnt,
-                       (const int64_t *)nullptr, (int32_t *)nullptr, 0);
+    const int gk = grid_n(ctx, n * kKillLanes);
+    hipLaunchKernelGGL(k_killers<false>, dim3(gk), dim3(256), 0, s, C, G, cnt, (const int64_t *)nullptr,
+                       (int32_t *)nullptr);
     PP_HIP(hipGetLastError());
     int64_t nedge = 0;
     {
         hipcub::TransformInputIterator<int64_t, I32ToI64, const int32_t *> it(cnt, I32ToI64());
         PP_CHECK(offsets(ctx, it, off, n, &nedge));
     }
-    int32_t *edges;
-    PP_CHECK(W.get((size_t)nedge, edges));
-    hipLaunchKernelGGL(k_fill_i32, dim3(grid_n(ctx, n)), dim3(256), 0, s, cnt, n, 0);
-    hipLaunchKernelGGL(k_killers, dim3(grid_n(ctx, n, 64)), dim3(64), 0, s, H, G, S, (const int32_t *)rank, cnt,
-                       (const int64_t *)off, edges, 1);
-    hipLaunchKernelGGL(k_fill_i32, dim3(grid_n(ctx, n)), dim3(256), 0, s, state, n, 0);
+    PP_CHECK(ctx->d_merge_edges.grow((size_t)std::max<int64_t>(nedge, 1) * sizeof(int32_t)));
+    int32_t *edges = ctx->d_merge_edges.as<int32_t>();
+    hipLaunchKernelGGL(k_killers<true>, dim3(gk), dim3(256), 0, s, C, G, cnt, (const int64_t *)off, edges);
     PP_HIP(hipGetLastError());
-    for (int64_t round = 0;; round++) {
+    // a few rounds for every look at what is left; a round too many changes nothing
+    constexpr int kRounds = 4;
+    int32_t *d_und = (int32_t *)(d_num + 2);
+    for (int64_t round = 0;; round += kRounds) {
         PP_ARG(round <= n, "exclusion rounds did not settle");
-        int32_t und = 0;
-        hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, s, d_und, (int64_t)1, 0);
-        hipLaunchKernelGGL(k_decide, dim3(grid_n(ctx, n)), dim3(256), 0, s, n, (const int64_t *)off,
-                           (const int32_t *)edges, state, d_und);
+        int32_t last = 0;
+        for (int q = 1; q <= kRounds; q++)
+            hipLaunchKernelGGL(k_decide, dim3(grid_n(ctx, n)), dim3(256), 0, s, n, (const int64_t *)off,
+                               (const int32_t *)edges, state, h, d_und, (int32_t)(round + q));
         PP_HIP(hipGetLastError());
-        PP_HIP(hipMemcpyAsync(&und, d_und, 4, hipMemcpyDeviceToHost, s));
+        PP_HIP(hipMemcpyAsync(&last, d_und, 4, hipMemcpyDeviceToHost, s));
         PP_HIP(hipStreamSynchronize(s));
-        if (und == 0) break;
+        if (last != (int32_t)(round + kRounds)) break;
     }
-    // pass 2: overlapping surviving pairs from the larger member
-    int64_t *pcnt, *poff;
-    PP_CHECK(W.get(n, pcnt));
-    PP_CHECK(W.get(n + 1, poff));
-    hipLaunchKernelGGL(k_pairs, dim3(grid_n(ctx, n, 64)), dim3(64), 0, s, H, G, S, (const int32_t *)rank,
-                       (const int32_t *)state, pcnt, (const int64_t *)nullptr, (int32_t *)nullptr, (double *)nullptr,
-                       (double *)nullptr, 0);
-    PP_HIP(hipGetLastError());
-    int64_t npair = 0;
-    PP_CHECK(offsets(ctx, (const int64_t *)pcnt, poff, n, &npair));
-    PP_ARG(npair < (1ll << 31), "too many overlapping pairs (%lld)", (long long)npair);
-    int32_t *pj, *pj_s, *sstart, *send;
-    double *cap_i, *cap_j, *cap_s;
-    PP_CHECK(W.get((size_t)npair, pj));
-    PP_CHECK(W.get((size_t)npair, pj_s));
-    PP_CHECK(W.get((size_t)npair, cap_i));
-    PP_CHECK(W.get((size_t)npair, cap_j));
-    PP_CHECK(W.get((size_t)npair, cap_s));
-    PP_CHECK(W.get(n, sstart));
-    PP_CHECK(W.get(n, send));
-    hipLaunchKernelGGL(k_pairs, dim3(grid_n(ctx, n, 64)), dim3(64), 0, s, H, G, S, (const int32_t *)rank,
-                       (const int32_t *)state, pcnt, (const int64_t *)poff, pj, cap_i, cap_j, 1);
-    hipLaunchKernelGGL(k_fill_i32, dim3(grid_n(ctx, n)), dim3(256), 0, s, sstart, n, 0);
-    hipLaunchKernelGGL(k_fill_i32, dim3(grid_n(ctx, n)), dim3(256), 0, s, send, n, 0);
-    PP_HIP(hipGetLastError());
-    if (npair > 0) {
-        // the smaller members' caps grouped by halo, pair order kept (stable)
-        tmp = 0;
-        PP_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, pj, pj_s, cap_j, cap_s, (int)npair, 0, 32, s));
-        PP_CHECK(ctx->d_cub.grow(tmp));
-        PP_HIP(hipcub::DeviceRadixSort::SortPairs(ctx->d_cub.ptr, tmp, pj, pj_s, cap_j, cap_s, (int)npair, 0, 32, s));
-        hipLaunchKernelGGL(k_cell_ranges, dim3(grid_n(ctx, npair)), dim3(256), 0, s, (const int32_t *)pj_s, npair,
-                           sstart, send);
-        PP_HIP(hipGetLastError());
-    }
-    int32_t *d_nk, hk = 0;
-    PP_CHECK(W.get(1, d_nk));
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, s, d_nk, (int64_t)1, 0);
-    int8_t *d_keep = keep;
-    float *d_nr = new_rthl;
-    if (!on_device) {
-        PP_CHECK(W.get(n, d_keep));
-        PP_CHECK(W.get(n, d_nr));
-    }
-    hipLaunchKernelGGL(k_finalize, dim3(grid_n(ctx, n)), dim3(256), 0, s, H, (const int32_t *)state,
-                       (const int64_t *)poff, (const double *)cap_i, (const int32_t *)sstart, (const int32_t *)send,
-                       (const double *)cap_s, d_keep, d_nr, d_nk);
+    // pass 2: caps of overlapping survivors, then the radii they leave
+    hipLaunchKernelGGL(k_pairs, dim3(grid_n(ctx, n * kPairLanes)), dim3(256), 0, s, C, G, caps, frac, d_num);
+    hipLaunchKernelGGL(k_finalize, dim3(std::min(grid_n(ctx, n), ctx->num_cu * 4)), dim3(256), 0, s, C, (const int32_t *)state,
+                       (const double *)caps, (const unsigned long long *)frac, d_keep, d_nr, d_num + 1);
     PP_HIP(hipGetLastError());
     if (!on_device) {
         PP_HIP(hipMemcpyAsync(keep, d_keep, n, hipMemcpyDeviceToHost, s));
         PP_HIP(hipMemcpyAsync(new_rthl, d_nr, n * 4, hipMemcpyDeviceToHost, s));
     }
-    PP_HIP(hipMemcpyAsync(&hk, d_nk, 4, hipMemcpyDeviceToHost, s));
+    unsigned long long num[2];
+    PP_HIP(hipMemcpyAsync(num, d_num, sizeof(num), hipMemcpyDeviceToHost, s));
     PP_HIP(hipStreamSynchronize(s));
-    *nkept = hk;
+    PP_ARG(num[0] < (1ull << 31), "too many overlapping pairs (%llu)", num[0]);
+    *nkept = (int64_t)num[1];
     return PP_OK;
 }

@@ -64,7 +64,7 @@ def merge_catalog(ctx, records):
         ctx._call(lambda: ctx.lib.pp_merge_halos(ctx.h, n, *(c.data_ptr() for c in cols), 1, keep.data_ptr(),
                                                  nr.data_ptr(), C.byref(nk)), True)
         sel = keep.bool()
-        out = records[sel].clone()
+        out = records[sel]
         out[:, 6] = nr[sel]
         return out
     rec = np.ascontiguousarray(records, np.float32)
