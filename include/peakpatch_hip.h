@@ -167,7 +167,7 @@ int pp_find_peaks_field(pp_ctx *ctx, const float *delta_s, int8_t *mask, int on_
  * update as pp_find_peaks_field; every pointer is device memory of the
  * context's device and every array of `out` (i, j, k, filt, delta_s; lapd_s
  * is ignored) is required.  The call allocates nothing: its counters, peak
- * bit mask, offsets and scan storage live in a static device array of
+ * bit mask and the mask's sums live in a static device array of
  * PP_NOALLOC_SCRATCH_BYTES per device (held until the process ends), which
  * limits the inner cube to about 8 M 64-cell row words (ceil(in1 / 64) x in2
  * x in3; any nbuff at n = 768); larger grids are refused with PP_ERR_ARG

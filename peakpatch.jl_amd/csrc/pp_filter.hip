@@ -132,7 +132,7 @@ static int launch_window(pp_ctx *ctx, const void *in, void *out, int n, double b
 
 // ------------------------------------------------------------- stencil
 // One pass over the field per filter.  A workgroup takes a 64 x 16 tile of
-// inner (x, y) columns and marches along z through kStencilKZ planes: each
+// inner (x, y) columns and marches along z through kz planes: each
 // plane's (64+2) x (16+2) neighbourhood is staged in LDS, two planes per
 // barrier (four buffers), every column keeps the 3x3 (x, y) maxima of planes
 // z-1, z, z+1 in registers, and the strict
@@ -141,11 +141,17 @@ static int launch_window(pp_ctx *ctx, const void *in, void *out, int n, double b
 // is one 64-bit word of the row's peak bit mask.  The mask byte is read only
 // for cells that pass the field test.
 //
-// A second, small pass turns the bit mask into the output: the exclusive
-// scan of the words' popcounts in (k, j, x) order is the CPU loop's order
-// (k outer, j, i inner), so each set bit is written at its rank with no
-// atomics, the first max_peaks ranks are kept (PeakFind.jl:70-72) and only
-// the kept peak cells are masked.
+// A second, small pass turns the bit mask into the output: the rank of a set
+// bit is the exclusive sum of the words' popcounts in (k, j, x) order, the CPU
+// loop's (k outer, j, i inner), the first max_peaks ranks are kept
+// (PeakFind.jl:70-72) and only the kept peak cells are masked.  The first pass
+// leaves every tile's count per plane; a plane's tiles of equal y are a run of
+// words, so that a workgroup of the second pass, which takes a few runs, gets
+// its first rank from one sum over the counts before (over their sums by
+// workgroup where there are many), and no scan is launched between.  Scan,
+// emission and bookkeeping were four launches of 15.4 us a filter at 128^3 and
+// 23 us at 200^3; one of 4.2 and 8.1 us now, and the filter bank there is
+// bound by the launches left (about 10 us of host each).
 //
 // Tiles are numbered x fastest, then y, then z, and handed out so that each
 // XCD (workgroups go round-robin to the eight XCDs, each with its own L2)
@@ -154,11 +160,21 @@ static int launch_window(pp_ctx *ctx, const void *in, void *out, int n, double b
 // instead of once per tile.
 constexpr int kStencilBlock = 512;
 constexpr int kStencilTY = 16;  // rows of the tile: each wave takes two, 8 apart
-constexpr int kStencilKZ = 32;
+// Planes of a tile: most for a large grid (each tile reads two planes more
+// than it tests), fewer while the tiles would leave CUs idle.
+// k_peak_bits at 128^3 (an inner cube of 100^3): 21.6 us with 32 planes (56
+// tiles), 8.3 with 8, 5.5 with 4, 5.6 with 2; at 200^3 24.5 with 32, 18 with a
+// threshold of one tile a CU, 13.1 with three, 14 with six; from 384^3 on 32.
+constexpr int kStencilKZ = 32, kStencilKZMin = 4;
+constexpr int kStencilTilesPerCU = 3;
 constexpr int kStencilXCD = 8;
+constexpr int kEmitBlocks = 4096;    // at most, doubling the runs of one
+constexpr int kEmitCounts = 1 << 14; // counts up to which k_peak_emit adds them up itself
 
 struct StencilTiles {
     int nbx, nby, nbz, per_xcd;  // tiles along x, y, z; tiles per XCD run
+    int kz;                      // planes of a tile
+    int runs, nruns, per;        // (plane, tile row) runs of a workgroup and of all; counts of a workgroup
 };
 
 struct StencilGeom {
@@ -187,17 +203,19 @@ static StencilGeom stencil_geom(int n1, int n2, int n3, int nbuff)
 // between.
 __global__ void __launch_bounds__(kStencilBlock) k_peak_bits(const float *__restrict__ d,
                                                              const int8_t *__restrict__ mask, StencilGeom g,
-                                                             StencilTiles tl, float fcrit, uint64_t *__restrict__ bits)
+                                                             StencilTiles tl, float fcrit, uint64_t *__restrict__ bits,
+                                                             int *__restrict__ counts)
 {
     constexpr int LX = 64 + 2, LY = kStencilTY + 2, LN = LX * LY, NQ = (LN + kStencilBlock - 1) / kStencilBlock;
+    __shared__ int found[kStencilKZ][kStencilBlock / 64];
     __shared__ float tile[4][LN];  // two pairs of planes: one pair staged while the other is read
     const int t = (int)(blockIdx.x % kStencilXCD) * tl.per_xcd + (int)(blockIdx.x / kStencilXCD);
     if (t >= tl.nbx * tl.nby * tl.nbz) return;  // the whole workgroup leaves before any barrier
     const int tbx = t % tl.nbx, tby = (t / tl.nbx) % tl.nby, tbz = t / (tl.nbx * tl.nby);
     const int lane = threadIdx.x & 63, wy = threadIdx.x >> 6;
     const int x0 = g.nbuff + 64 * tbx, y0 = g.nbuff + kStencilTY * tby;
-    const int z0 = g.nbuff + kStencilKZ * tbz;
-    const int z1 = min(z0 + kStencilKZ, g.nbuff + g.in3);  // planes z0..z1-1; z0-1..z1 are read
+    const int z0 = g.nbuff + tl.kz * tbz;
+    const int z1 = min(z0 + tl.kz, g.nbuff + g.in3);  // planes z0..z1-1; z0-1..z1 are read
     const long long s12 = (long long)g.n1 * g.n2;
     const int x = x0 + lane;
     const int ya = y0 + wy, yb = ya + kStencilTY / 2;
@@ -252,9 +270,11 @@ __global__ void __launch_bounds__(kStencilBlock) k_peak_bits(const float *__rest
         if (ka) ka = mask[x + (long long)ya * g.n1 + (long long)z * s12] != 1;
         if (kb) kb = mask[x + (long long)yb * g.n1 + (long long)z * s12] != 1;
         const unsigned long long wa = __ballot(ka), wb = __ballot(kb);
+        if (lane != 0) return;
         const long long base = (long long)(z - g.nbuff) * word_row + tbx;
-        if (lane == 0 && ya < g.nbuff + g.in2) bits[base + (long long)(ya - g.nbuff) * g.words] = wa;
-        if (lane == 0 && yb < g.nbuff + g.in2) bits[base + (long long)(yb - g.nbuff) * g.words] = wb;
+        if (ya < g.nbuff + g.in2) bits[base + (long long)(ya - g.nbuff) * g.words] = wa;
+        if (yb < g.nbuff + g.in2) bits[base + (long long)(yb - g.nbuff) * g.words] = wb;
+        found[z - z0][wy] = __popcll(wa) + __popcll(wb);
     };
     // two planes per barrier: planes z+1, z+2 (in ra, rb) go to one pair of
     // buffers while z+3, z+4 are fetched; the pair written here was last
@@ -276,11 +296,14 @@ __global__ void __launch_bounds__(kStencilBlock) k_peak_bits(const float *__rest
             ca = c2a; cb = c2b;
         }
     }
+    __syncthreads();
+    if ((int)threadIdx.x < z1 - z0) {
+        int sum = 0;
+#pragma unroll
+        for (int q = 0; q < kStencilBlock / 64; q++) sum += found[threadIdx.x][q];
+        counts[((long long)(z0 - g.nbuff + threadIdx.x) * tl.nby + tby) * tl.nbx + tbx] = sum;
+    }
 }
-
-struct Popc {
-    __device__ __forceinline__ int operator()(const uint64_t &w) const { return __popcll(w); }
-};
 
 struct PeakOut {
     int32_t *i, *j, *k, *filt;
@@ -288,55 +311,109 @@ struct PeakOut {
     long long capacity;
 };
 
-// counters[0] = peaks written so far (all filters), counters[1] = peaks found
-// (capped per filter), counters[2] = first index of the current filter.
-__global__ void __launch_bounds__(256) k_peak_emit(const float *__restrict__ d, int8_t *__restrict__ mask,
-                                                   StencilGeom g, const uint64_t *__restrict__ bits,
-                                                   const int *__restrict__ word_off,
-                                                   const long long *__restrict__ counters, long long max_peaks,
-                                                   int filt, PeakOut o)
+// before a call's first stencil
+__global__ void k_stencil_clear(long long *counters, long long *base)
 {
-    const long long w = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (w >= g.nwords) return;
-    uint64_t b = bits[w];
-    if (!b) return;
-    const long long row = w / g.words;
-    const int wx = (int)(w - row * g.words);
-    const int j = g.nbuff + (int)(row % g.in2), k = g.nbuff + (int)(row / g.in2);
-    long long rank = word_off[w];
-    const long long base = counters[0];
-    while (b) {
-        if (rank >= max_peaks) return;
-        const int bit = __ffsll((unsigned long long)b) - 1;
-        b &= b - 1;
-        const int i = g.nbuff + 64 * wx + bit;
-        const long long c = i + (long long)j * g.n1 + (long long)k * g.n1 * g.n2;
-        mask[c] = 1;
-        const long long slot = base + rank;
-        if (slot < o.capacity) {
-            o.i[slot] = i;
-            o.j[slot] = j;
-            o.k[slot] = k;
-            o.filt[slot] = filt;
-            o.delta_s[slot] = d[c];
+    if (threadIdx.x < 4) counters[threadIdx.x] = 0;
+    if (threadIdx.x < 2) base[threadIdx.x] = 0;
+}
+
+// exclusive sum of v over the workgroup's 256 threads; *total gets the sum
+__device__ __forceinline__ int block_offset(int v, int *wsum, int *total)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int s = v;
+    for (int w = 1; w < 64; w <<= 1) {
+        const int u = __shfl_up(s, w, 64);
+        if (lane >= w) s += u;
+    }
+    __syncthreads();  // the sums of the call before have been read
+    if (lane == 63) wsum[wave] = s;
+    __syncthreads();
+    int before = 0;
+    for (int q = 0; q < 4; q++) before += q < wave ? wsum[q] : 0;
+    *total = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+    return before + s - v;
+}
+
+// the counts' sums by workgroup of k_peak_emit
+__global__ void __launch_bounds__(256) k_peak_sums(const int *__restrict__ counts, long long n, int per, int nsums,
+                                                   int *__restrict__ sums)
+{
+    const int s = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (s >= nsums) return;
+    const long long e = min((long long)(s + 1) * per, n);
+    int sum = 0;
+    for (long long q = (long long)s * per + (threadIdx.x & 63); q < e; q += 64) sum += counts[q];
+    for (int w = 32; w > 0; w >>= 1) sum += __shfl_down(sum, w, 64);
+    if ((threadIdx.x & 63) == 0) sums[s] = sum;
+}
+
+// counters[0] = peaks written so far (all filters), counters[1] = peaks found
+// (capped per filter), counters[2] = first index of the current filter.  A
+// workgroup writes the peaks of tl.runs runs; `before` holds `per` counts or
+// sums for each workgroup.  The filter's first slot is base[parity]; the last
+// workgroup leaves the next one in the other word (counters[0] itself would
+// need every workgroup to have read it: a device-wide fence by each took 0.2
+// ms at 512^3).
+__global__ void __launch_bounds__(256) k_peak_emit(const float *__restrict__ d, int8_t *__restrict__ mask,
+                                                   StencilGeom g, StencilTiles tl, const uint64_t *__restrict__ bits,
+                                                   const int *__restrict__ before, int per,
+                                                   long long *__restrict__ base, int parity,
+                                                   long long *__restrict__ counters, long long max_peaks, int filt,
+                                                   PeakOut o, long long *__restrict__ range)
+{
+    __shared__ int wsum[4];
+    int sum = 0, total;
+    for (long long q = threadIdx.x, e = (long long)blockIdx.x * per; q < e; q += 256) sum += before[q];
+    block_offset(sum, wsum, &total);
+    long long first = total;  // rank of the workgroup's first peak
+    const long long b0 = base[parity];
+    auto word = [&](int run) {  // the run's first word
+        const int z = run / tl.nby, ty = run - z * tl.nby;
+        return ((long long)z * g.in2 + (long long)ty * kStencilTY) * g.words;
+    };
+    const int run1 = min((int)(blockIdx.x + 1) * tl.runs, tl.nruns);
+    const long long w0 = word(blockIdx.x * tl.runs), w1 = run1 < tl.nruns ? word(run1) : g.nwords;
+    for (long long w = w0 + threadIdx.x; w - (int)threadIdx.x < w1; w += 256) {
+        uint64_t b = w < w1 ? bits[w] : 0;
+        long long rank = first + block_offset(__popcll(b), wsum, &total);
+        first += total;
+        const long long row = w / g.words;
+        const int wx = (int)(w - row * g.words);
+        const int j = g.nbuff + (int)(row % g.in2), k = g.nbuff + (int)(row / g.in2);
+        for (; b && rank < max_peaks; b &= b - 1, rank++) {
+            const int i = g.nbuff + 64 * wx + __ffsll((unsigned long long)b) - 1;
+            const long long c = i + (long long)j * g.n1 + (long long)k * g.n1 * g.n2;
+            mask[c] = 1;
+            const long long slot = b0 + rank;
+            if (slot < o.capacity) {
+                o.i[slot] = i;
+                o.j[slot] = j;
+                o.k[slot] = k;
+                o.filt[slot] = filt;
+                o.delta_s[slot] = d[c];
+            }
         }
-        rank++;
+    }
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
+        const long long kept = first < max_peaks ? first : max_peaks;  // first: all of the filter's peaks
+        base[parity ^ 1] = b0 + kept;
+        counters[0] = b0 + kept;
+        counters[1] += kept;
+        counters[2] = b0;
+        if (range) {  // this filter's peaks, for work that follows on another stream
+            range[0] = b0;
+            range[1] = b0 + kept;
+        }
     }
 }
 
-__global__ void k_stencil_finish(const uint64_t *__restrict__ bits, const int *__restrict__ word_off,
-                                 long long nwords, long long max_peaks, long long *__restrict__ counters,
-                                 long long *__restrict__ range)
+// a filter's stencil over an empty inner cube
+__global__ void k_stencil_none(long long *__restrict__ counters, long long *__restrict__ range)
 {
-    long long found = nwords > 0 ? (long long)word_off[nwords - 1] + __popcll(bits[nwords - 1]) : 0;
-    long long kept = found < max_peaks ? found : max_peaks;
     counters[2] = counters[0];
-    counters[0] += kept;
-    counters[1] += kept;
-    if (range) {  // this filter's peaks, for work that follows on another stream
-        range[0] = counters[2];
-        range[1] = counters[0];
-    }
+    if (range) range[0] = range[1] = counters[0];
 }
 
 __global__ void k_sample_field(const float *__restrict__ f, int n1, int n2, const int32_t *__restrict__ pi,
@@ -351,93 +428,95 @@ __global__ void k_sample_field(const float *__restrict__ f, int n1, int n2, cons
         out[s] = f[pi[s] + (long long)pj[s] * n1 + (long long)pk[s] * n1 * n2];
 }
 
-// Device scratch of one stencil pass: the peak bit mask, the words' output
-// offsets and the scan's temporary storage, carved from one buffer.
+// Device scratch of a call's stencils, carved from one buffer: the peak bit
+// mask, the tiles' counts (as many as words at most), their sums, the slots.
 struct StencilScratch {
     uint64_t *bits;
-    int *off;
-    void *tmp;
-    size_t tmp_bytes;
+    int *counts, *sums;
+    long long *base;
 };
 
 static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-static int stencil_scan_bytes(const StencilGeom &g, size_t *tmp)
+static size_t stencil_scratch_bytes(const StencilGeom &g)
 {
-    hipcub::TransformInputIterator<int, Popc, const uint64_t *> it((const uint64_t *)nullptr, Popc());
-    *tmp = 0;
-    PP_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, *tmp, it, (int *)nullptr, (int)std::max(1ll, g.nwords)));
-    return PP_OK;
+    return align256((size_t)g.nwords * 8) + align256((size_t)g.nwords * 4) + align256(kEmitBlocks * sizeof(int)) + 256;
 }
 
-static int stencil_scratch_bytes(const StencilGeom &g, size_t *bytes)
-{
-    size_t tmp = 0;
-    PP_CHECK(stencil_scan_bytes(g, &tmp));
-    *bytes = align256((size_t)g.nwords * 8) + align256((size_t)g.nwords * 4) + align256(tmp);
-    return PP_OK;
-}
-
-static StencilScratch stencil_carve(void *base, const StencilGeom &g, size_t tmp)
+static StencilScratch stencil_carve(void *base, const StencilGeom &g)
 {
     StencilScratch s;
     char *p = (char *)base;
     s.bits = (uint64_t *)p;
     p += align256((size_t)g.nwords * 8);
-    s.off = (int *)p;
+    s.counts = (int *)p;
     p += align256((size_t)g.nwords * 4);
-    s.tmp = p;
-    s.tmp_bytes = tmp;
+    s.sums = (int *)p;
+    p += align256(kEmitBlocks * sizeof(int));
+    s.base = (long long *)p;
     return s;
 }
 
-// Stencil over one field with the scratch given; peaks appended after
+// before a call's first stencil: a kernel rather than a memset node, so that
+// a caller may capture the call in a HIP graph
+static int stencil_clear(pp_ctx *ctx, const StencilScratch &s, long long *d_counters)
+{
+    hipLaunchKernelGGL(k_stencil_clear, dim3(1), dim3(64), 0, ctx->stream, d_counters, s.base);
+    PP_HIP(hipGetLastError());
+    return PP_OK;
+}
+
+// Stencil over one field, the step-th of a call; peaks appended after
 // counters[0].
-static int run_stencil_with(pp_ctx *ctx, const float *d_field, int8_t *d_mask, const StencilGeom &g,
-                            float fcrit, long long max_peaks, int filt, const PeakOut &o, long long *d_counters,
-                            const StencilScratch &s, long long *range = nullptr)
+static int run_stencil(pp_ctx *ctx, const float *d_field, int8_t *d_mask, const StencilGeom &g,
+                       float fcrit, long long max_peaks, int step, const PeakOut &o, long long *d_counters,
+                       const StencilScratch &s, long long *range = nullptr)
 {
     PP_ARG(g.nwords < (1ll << 31), "inner cube too large for the stencil");
     if (g.nwords == 0) {
-        hipLaunchKernelGGL(k_stencil_finish, dim3(1), dim3(1), 0, ctx->stream, (const uint64_t *)nullptr,
-                           (const int *)nullptr, 0ll, max_peaks, d_counters, range);
+        hipLaunchKernelGGL(k_stencil_none, dim3(1), dim3(1), 0, ctx->stream, d_counters, range);
         PP_HIP(hipGetLastError());
         return PP_OK;
     }
     StencilTiles tl;
     tl.nbx = g.words;
     tl.nby = (g.in2 + kStencilTY - 1) / kStencilTY;
-    tl.nbz = (g.in3 + kStencilKZ - 1) / kStencilKZ;
-    const long long ntiles = (long long)tl.nbx * tl.nby * tl.nbz;
+    long long ntiles = 0;
+    for (tl.kz = kStencilKZ;; tl.kz /= 2) {
+        tl.nbz = (g.in3 + tl.kz - 1) / tl.kz;
+        ntiles = (long long)tl.nbx * tl.nby * tl.nbz;
+        if (tl.kz <= kStencilKZMin || ntiles >= (long long)kStencilTilesPerCU * ctx->num_cu) break;
+    }
     PP_ARG(ntiles < (1ll << 30), "inner cube too large for the stencil grid");
     tl.per_xcd = (int)((ntiles + kStencilXCD - 1) / kStencilXCD);
+    tl.nruns = g.in3 * tl.nby;
+    const long long ncounts = (long long)tl.nruns * tl.nbx;
+    for (tl.runs = std::max(1, 256 / (kStencilTY * g.words)); (tl.nruns + tl.runs - 1) / tl.runs > kEmitBlocks;)
+        tl.runs *= 2;
+    const int blocks = (tl.nruns + tl.runs - 1) / tl.runs;
+    tl.per = tl.runs * tl.nbx;
     hipLaunchKernelGGL(k_peak_bits, dim3((unsigned)tl.per_xcd * kStencilXCD), dim3(kStencilBlock), 0, ctx->stream,
-                       d_field, (const int8_t *)d_mask, g, tl, fcrit, s.bits);
+                       d_field, (const int8_t *)d_mask, g, tl, fcrit, s.bits, s.counts);
     PP_HIP(hipGetLastError());
-    hipcub::TransformInputIterator<int, Popc, const uint64_t *> it(s.bits, Popc());
-    size_t tmp = s.tmp_bytes;
-    PP_HIP(hipcub::DeviceScan::ExclusiveSum(s.tmp, tmp, it, s.off, (int)g.nwords, ctx->stream));
-    const unsigned eblocks = (unsigned)((g.nwords + 255) / 256);
-    hipLaunchKernelGGL(k_peak_emit, dim3(eblocks), dim3(256), 0, ctx->stream, d_field, d_mask, g,
-                       (const uint64_t *)s.bits, (const int *)s.off, (const long long *)d_counters, max_peaks,
-                       filt, o);
-    PP_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_stencil_finish, dim3(1), dim3(1), 0, ctx->stream, (const uint64_t *)s.bits,
-                       (const int *)s.off, g.nwords, max_peaks, d_counters, range);
+    const bool sums = ncounts > kEmitCounts;
+    if (sums) {
+        hipLaunchKernelGGL(k_peak_sums, dim3((blocks + 3) / 4), dim3(256), 0, ctx->stream, (const int *)s.counts,
+                           ncounts, tl.per, blocks, s.sums);
+        PP_HIP(hipGetLastError());
+    }
+    hipLaunchKernelGGL(k_peak_emit, dim3(blocks), dim3(256), 0, ctx->stream, d_field, d_mask, g, tl,
+                       (const uint64_t *)s.bits, (const int *)(sums ? s.sums : s.counts), sums ? 1 : tl.per, s.base,
+                       step & 1, d_counters, max_peaks, step, o, range);
     PP_HIP(hipGetLastError());
     return PP_OK;
 }
 
-static int run_stencil(pp_ctx *ctx, const float *d_field, int8_t *d_mask, const StencilGeom &g,
-                       float fcrit, long long max_peaks, int filt, const PeakOut &o,
-                       long long *d_counters, long long *range = nullptr)
+// the state of a call's stencils in the context's scratch, cleared
+static int stencil_start(pp_ctx *ctx, const StencilGeom &g, long long *d_counters, StencilScratch &s)
 {
-    size_t bytes = 0, tmp = 0;
-    PP_CHECK(stencil_scan_bytes(g, &tmp));
-    PP_CHECK(stencil_scratch_bytes(g, &bytes));
-    PP_CHECK(ctx->d_scan.grow(bytes));
-    return run_stencil_with(ctx, d_field, d_mask, g, fcrit, max_peaks, filt, o, d_counters,
-                            stencil_carve(ctx->d_scan.ptr, g, tmp), range);
+    PP_CHECK(ctx->d_scan.grow(stencil_scratch_bytes(g)));
+    s = stencil_carve(ctx->d_scan.ptr, g);
+    return stencil_clear(ctx, s, d_counters);
 }
 
 // ------------------------------------------- the k^2 field at the peaks
@@ -694,13 +773,6 @@ static void *noalloc_scratch(int device)
     return device >= 0 && device < kMaxDevices ? g_scratch_ptr[device] : nullptr;
 }
 
-// clears the counters with a kernel rather than a memset node, so that a
-// caller may capture the call in a HIP graph
-__global__ void k_zero_counters(long long *c)
-{
-    if (threadIdx.x < 4) c[threadIdx.x] = 0;
-}
-
 static int alloc_peak_out(pp_ctx *ctx, long long cap, PeakOut &o, float **lapd, long long **counters)
 {
     size_t per = cap > 0 ? (size_t)cap : 1;
@@ -716,7 +788,6 @@ static int alloc_peak_out(pp_ctx *ctx, long long cap, PeakOut &o, float **lapd, 
     o.delta_s = (float *)p; p += per * sizeof(float);
     *lapd = (float *)p;
     o.capacity = cap;
-    PP_HIP(hipMemsetAsync(*counters, 0, 4 * sizeof(long long), ctx->stream));
     return PP_OK;
 }
 
@@ -862,8 +933,10 @@ int pp_find_peaks_field(pp_ctx *ctx, const float *delta_s, int8_t *mask, int on_
     float *d_lapd;
     long long *d_counters;
     PP_CHECK(alloc_peak_out(ctx, out->capacity, o, &d_lapd, &d_counters));
+    StencilScratch S;
+    PP_CHECK(stencil_start(ctx, g, d_counters, S));
     PP_HIP(hipEventRecord(ctx->ev[0], ctx->stream));
-    PP_CHECK(run_stencil(ctx, d_f, d_m, g, fcrit, max_peaks, 0, o, d_counters));
+    PP_CHECK(run_stencil(ctx, d_f, d_m, g, fcrit, max_peaks, 0, o, d_counters, S));
     PP_HIP(hipEventRecord(ctx->ev[1], ctx->stream));
     if (!on_device) PP_HIP(hipMemcpyAsync(mask, d_m, N, hipMemcpyDeviceToHost, ctx->stream));
     int rc = download_peaks(ctx, o, nullptr, d_counters, out);
@@ -918,6 +991,8 @@ int pp_find_peaks(pp_ctx *ctx, const float *delta, int on_device, int n, double 
     long long *d_counters;
     PP_CHECK(alloc_peak_out(ctx, out->capacity, o, &d_lapd, &d_counters));
     const StencilGeom g = stencil_geom(n, n, n, nbuff);
+    StencilScratch S;
+    PP_CHECK(stencil_start(ctx, g, d_counters, S));
     const float inv = (float)(1.0 / ((double)n * n * n));
     Bank K;
     if (lines && nfilt > 0) PP_CHECK(bank_start(ctx, ctx->d_k0.ptr, n, nbuff, n - nbuff, boxsize, Rf, nfilt, K));
@@ -932,7 +1007,7 @@ int pp_find_peaks(pp_ctx *ctx, const float *delta, int on_device, int n, double 
         void *ib[1] = {ctx->d_k1.ptr}, *ob[1] = {ctx->d_field_a.ptr};
         PP_FFT(rocfft_execute(ctx->fftp->c2r, ib, ob, ctx->fftp->info));
         PP_CHECK(run_stencil(ctx, ctx->d_field_a.as<float>(), d_mask, g, fcrit[f], max_peaks_per_filter, f,
-                             o, d_counters, lines ? K.ranges + 2 * f : nullptr));
+                             o, d_counters, S, lines ? K.ranges + 2 * f : nullptr));
         if (lines) {
             PP_CHECK(bank_sample(ctx, K, f, o, d_lapd));
         } else if (want_lapd) {
@@ -965,10 +1040,13 @@ int pp_find_peaks_field_noalloc(pp_ctx *ctx, const float *delta_s, int8_t *mask,
     PP_CHECK(ensure_device(ctx));
     if (max_peaks <= 0) max_peaks = 2000000;
     const StencilGeom g = stencil_geom(n1, n2, n3, nbuff);
-    size_t need = 0, tmp = 0;
-    PP_CHECK(stencil_scan_bytes(g, &tmp));
-    PP_CHECK(stencil_scratch_bytes(g, &need));
-    need += 256;
+    // the bound callers know: 12 bytes a word and the storage of a scan over
+    // them, more than the bit mask and the runs now take
+    hipcub::CountingInputIterator<int> it(0);
+    size_t tmp = 0;
+    PP_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, it, (int *)nullptr, (int)std::max(1ll, g.nwords)));
+    const size_t need = std::max(align256((size_t)g.nwords * 8) + align256((size_t)g.nwords * 4) + align256(tmp),
+                                 stencil_scratch_bytes(g)) + 256;
     PP_ARG(need <= (size_t)PP_NOALLOC_SCRATCH_BYTES,
            "inner cube %dx%dx%d needs %zu B of scratch, more than the %zu B this entry point has; use "
            "pp_find_peaks_field", g.in1, g.in2, g.in3, need, (size_t)PP_NOALLOC_SCRATCH_BYTES);
@@ -981,11 +1059,10 @@ int pp_find_peaks_field_noalloc(pp_ctx *ctx, const float *delta_s, int8_t *mask,
     PeakOut o;
     o.i = out->i; o.j = out->j; o.k = out->k; o.filt = out->filt; o.delta_s = out->delta_s;
     o.capacity = out->capacity;
-    hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, ctx->stream, d_counters);
-    PP_HIP(hipGetLastError());
+    const StencilScratch S = stencil_carve(base + 256, g);
+    PP_CHECK(stencil_clear(ctx, S, d_counters));
     PP_HIP(hipEventRecord(ctx->ev[0], ctx->stream));
-    PP_CHECK(run_stencil_with(ctx, delta_s, mask, g, fcrit, max_peaks, 0, o, d_counters,
-                              stencil_carve(base + 256, g, tmp)));
+    PP_CHECK(run_stencil(ctx, delta_s, mask, g, fcrit, max_peaks, 0, o, d_counters, S));
     PP_HIP(hipEventRecord(ctx->ev[1], ctx->stream));
     long long cnt[4];
     PP_HIP(hipMemcpyAsync(cnt, d_counters, sizeof cnt, hipMemcpyDeviceToHost, ctx->stream));

@@ -50,9 +50,10 @@ namespace pp {
 // ------------------------------------------------------------ coarse noise
 // _downsample_noise: coarse cell (I, J, K) sums the normals of fine cells
 // I b .. I b + b - 1 (and likewise in y, z), 0-based.  Bound by the
-// instructions of the normals: M = 20, b = 41 (5.5e8 cells)
-// 1.75 ms (3.1 ms with the general functions and a division per pair); 240
-// instructions a pair at the measured 3.9e13 lanes/s are 1.7 ms.
+// instructions of the normals: with M = 20, b = 41 (5.5e8 cells) the coarse
+// fields take 1.98 ms (3.33 ms with the general functions and two divisions a
+// pair), of which 240 instructions a pair at the measured 3.9e13 lanes/s are
+// 1.75 ms.
 __global__ void __launch_bounds__(256) k_coarse_noise(float *__restrict__ out, int N, int M, int b, uint64_t seed,
                                                       double norm)
 {
