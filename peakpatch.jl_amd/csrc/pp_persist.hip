@@ -18,7 +18,8 @@
 //        (peak, shell) position by a wave shuffle and sums runs of equal shell
 //        by a segmented tree into LDS bins.
 //      * other peaks: k_gather, a persistent work-queue kernel (one wave per
-//        peak, peaks pulled from per-XCD atomic counters).  The shells are
+//        peak, up to eight while there are few, peaks pulled from per-XCD
+//        atomic counters).  The shells are
 //        processed in chunks of chunk_shells; within a chunk the host packed
 //        the groups (row-major, so lanes read neighbouring x-runs) into dense
 //        64-lane batches sorted by shell; the lanes of a run of equal shells
@@ -28,9 +29,11 @@
 //   4. Float64 post-process (fcrit crossing, inward walk with strain
 //      eigenvalues and collapse-table look-ups, R_TH, Srb, zvir_half):
 //      k_post_wave (one wave per peak) for m > coop_m, k_post_lane (one lane
-//      per peak) below; the lane post's walk steps are evaluated ahead of it
-//      by lane groups (k_walk_group, the walk table).
-//   5. k_finish: one wave per collapsed non-small peak sums eta, eta2 over the
+//      per peak) or k_post_group (2 to 16, few peaks) below; the latter two's
+//      walk steps are evaluated ahead of them by lane groups (k_walk_group,
+//      the walk table).
+//   5. k_finish: one wave (up to eight, few peaks) per collapsed non-small
+//      peak sums eta, eta2 over the
 //      shells inside m0 and lapd over the cells inside R_TH and writes the
 //      mask; small peaks carry those sums in their profile, from which
 //      k_small_finish forms them.
@@ -529,10 +532,16 @@ __device__ __forceinline__ void neumaier(float *hi, float *lo, float x)
 // run's first lane deposits the sum into the chunk's bins.  The records of a chunk are
 // written with Fbar, whose recursion is carried as the prefix sum
 // Q(s) = Fbar(s) r^3(s) = sum_{t=2..s} (dF(t-1) + dF(t)) / 2 (r^3(t) - r^3(t-1)).
-__global__ void __launch_bounds__(64) k_gather(GatherArgs A)
+//
+// With NW > 1 waves (one workgroup) per peak, the waves take a chunk's batches
+// in turn and deposit in batch order, so that every bin sees the same sums in
+// the same order as with one wave; wave 0 writes the records.
+template <int NW>
+__global__ void __launch_bounds__(64 * NW) k_gather(GatherArgs A)
 {
     extern __shared__ float lds[];
-    const int lane = threadIdx.x;
+    __shared__ int next;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int cs = A.cs;
     float *bh = lds, *bl = bh + P_NB * cs;  // [P_NB][cs] each
     // own XCD's list first, then the others' (the tail of the work)
@@ -540,14 +549,21 @@ __global__ void __launch_bounds__(64) k_gather(GatherArgs A)
     int xq = 0;
     for (;;) {
         int idx = -1;
-        if (lane == 0) {
+        if (threadIdx.x == 0) {
             for (; xq < A.nx; xq++) {
                 const int x = (x0 + xq) % A.nx;
                 const int64_t t = A.xb[x] + atomicAdd(A.queue + 64 * x, 1);
                 if (t < A.xb[x + 1]) { idx = A.xorder[t]; break; }
             }
+            if (NW > 1) next = idx;
         }
-        idx = __shfl(idx, 0, 64);
+        if (NW > 1) {
+            __syncthreads();
+            idx = next;
+            __syncthreads();  // read before thread 0 takes the next peak
+        } else {
+            idx = __shfl(idx, 0, 64);
+        }
         if (idx < 0) break;
         const PeakParam pk = A.pps[idx];
         const int m = pk.m;
@@ -556,40 +572,51 @@ __global__ void __launch_bounds__(64) k_gather(GatherArgs A)
         {
             float v[PR];
             F1 = center_values<false>(A.F, pk, v);
-            if (lane == 0) store_record(A.prof, rec, v, 1);
+            if (threadIdx.x == 0) store_record(A.prof, rec, v, 1);
         }
         double carry = 0.0, dFprev = (double)F1;
         const int nch = m >= 2 ? (m - 2) / cs + 1 : 0;
         for (int c = 0; c < nch; c++) {
             const int s0 = 2 + c * cs, s1 = min(m, s0 + cs - 1), ns = s1 - s0 + 1;
             for (int f = 0; f < P_NB; f++)
-                for (int b = lane; b < ns; b += 64) { bh[f * cs + b] = 0.0f; bl[f * cs + b] = 0.0f; }
+                for (int b = threadIdx.x; b < ns; b += 64 * NW) { bh[f * cs + b] = 0.0f; bl[f * cs + b] = 0.0f; }
             __syncthreads();
             const bool full = s0 + cs - 1 <= m;
             const GroupDesc *tab = A.desc + (full ? A.full_off[c] : A.part_off[m]);
             const int nb = full ? A.full_nb[c] : A.part_nb[m];
-            for (int b = 0; b < nb; b++) {
-                const GroupDesc g = tab[b * 64 + lane];
+            for (int b0 = 0; b0 < nb; b0 += NW) {
+                const int b = b0 + wave;
                 float acc[PR];
+                GroupDesc g;
+                g.s = 0;
+                g.lmn = 0;
+                if (b < nb) {
+                    g = tab[b * 64 + lane];
 #pragma unroll
-                for (int f = 0; f < PR; f++) acc[f] = 0.0f;
-                if (g.s >= 2) group_sum<false>(A.F, pk, g, acc);
-                const int rend = (g.lmn >> 24) & 127;
-                for (int k = 0; k < A.steps; k++) {
-                    const int d = 1 << k;
-                    const bool in = lane + d < rend;
+                    for (int f = 0; f < PR; f++) acc[f] = 0.0f;
+                    if (g.s >= 2) group_sum<false>(A.F, pk, g, acc);
+                    const int rend = (g.lmn >> 24) & 127;
+                    for (int k = 0; k < A.steps; k++) {
+                        const int d = 1 << k;
+                        const bool in = lane + d < rend;
 #pragma unroll
-                    for (int f = 0; f < P_NB; f++) {
-                        const float u = __shfl_down(acc[f], d, 64);
-                        if (in) acc[f] += u;
+                        for (int f = 0; f < P_NB; f++) {
+                            const float u = __shfl_down(acc[f], d, 64);
+                            if (in) acc[f] += u;
+                        }
                     }
                 }
-                if (g.lmn < 0) {  // run head
-                    const int sb = g.s - s0;
 #pragma unroll
-                    for (int f = 0; f < P_NB; f++) neumaier(&bh[f * cs + sb], &bl[f * cs + sb], acc[f]);
+                for (int w = 0; w < NW; w++) {
+                    if (w == wave && g.lmn < 0) {  // run head
+                        const int sb = g.s - s0;
+#pragma unroll
+                        for (int f = 0; f < P_NB; f++) neumaier(&bh[f * cs + sb], &bl[f * cs + sb], acc[f]);
+                    }
+                    if (NW > 1) __syncthreads();
                 }
             }
+            if (wave == 0)
             for (int b0 = 0; b0 < ns; b0 += 64) {
                 const int b = b0 + lane;
                 const bool valid = b < ns;
@@ -697,6 +724,21 @@ __device__ __forceinline__ AosProfile<FULL> profile_at(ProfBuf p, int64_t rb, co
 // (about one peak per wave) 15.10
 constexpr int kSmallGridCU = 32;
 constexpr int kWaveGridCU = 16;
+constexpr int kCrossLanes = 8;  // lanes that search one peak's crossing
+// Lanes per peak in the post of the walk-table class: as many (up to
+// kGroupPost) as keep the lanes per CU below kGroupPostLanesCU, one for a
+// large batch.  Whole calls (peaks with m > small_m in brackets), lane post /
+// 256 / 1024 / 2048 lanes a CU: 256^3 60 k peaks (20 k) 2.70 / 2.01 / 1.81 /
+// 1.78 ms, 300^3 150 k (49 k) 3.41 / 3.30 / 3.09 / 3.01, 512^3 1.95 M (400 k)
+// 15.4, with 4096 15.8.
+constexpr int kGroupPost = 16, kGroupPostLanesCU = 2048;
+// Waves per peak in the gather and the finish pass: 8, 4 and 2 up to so many
+// peaks a CU, above them one (a batch's time is its largest peaks' chains of
+// loads until there are enough waves without).  Whole calls with 8 / 4 / 2 /
+// 1: 26 peaks a CU 1.38 / 1.46 / 1.68 / 2.4 ms, 77 2.17 / 1.78 / 1.95 / 2.66,
+// 191 4.09 / 3.01 / 2.73 / 3.41, 376 7.7 / 5.2 / 5.1 / 5.95, 1550 - / 19.7 /
+// 16.3 / 15.4.
+constexpr int kSharedPeaksPerCU[3] = {40, 120, 800};
 constexpr int kFinishGridCU = 256;
 constexpr int kLaneGridCU = 64;
 constexpr int64_t kWalkBound = 1ll << 26;  // walk records (64 B) reserved from their bound alone
@@ -711,17 +753,21 @@ constexpr int kWalkGridCU = 16;  // 256-lane workgroups per CU of the walk table
 // ascending keys give m and the crossing descending in 2 * cbits bits.
 // The crossing of every peak also goes to mc[t - lo]: the walk table holds
 // shells 1..mc of the peak.
-__global__ void k_crossing_keys(const PeakParam *__restrict__ pps, int64_t lo, int64_t hi, ProfBuf prof,
-                                const int64_t *__restrict__ prof_off, const double *__restrict__ rad,
-                                int cmax, int cbits, uint32_t *__restrict__ keys, int64_t *__restrict__ mc)
+__global__ void __launch_bounds__(256) k_crossing_keys(const PeakParam *__restrict__ pps, int64_t lo, int64_t hi,
+                                                       ProfBuf prof, const int64_t *__restrict__ prof_off,
+                                                       const double *__restrict__ rad, int cmax, int cbits,
+                                                       uint32_t *__restrict__ keys, int64_t *__restrict__ mc)
 {
-    for (int64_t t = lo + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < hi; t += (int64_t)gridDim.x * blockDim.x) {
+    for (int64_t t = lo + ((int64_t)blockIdx.x * 256 + threadIdx.x) / kCrossLanes; t < hi;
+         t += (int64_t)gridDim.x * (256 / kCrossLanes)) {
         const PeakParam pk = pps[t];
         const int64_t rb = prof_off[t];
         const AosProfile<false> P = profile_at<false>(prof, rb, rad, false);
-        const int c = (pk.flags & 2) ? 0 : max(crossing_m0(P, pk), 0);
-        keys[t - lo] = (uint32_t)(cmax - pk.m) << cbits | (uint32_t)(cmax - c);
-        mc[t - lo] = c;
+        const int c = (pk.flags & 2) ? 0 : max(crossing_m0<kCrossLanes>(P, pk), 0);
+        if ((threadIdx.x & (kCrossLanes - 1)) == 0) {
+            keys[t - lo] = (uint32_t)(cmax - pk.m) << cbits | (uint32_t)(cmax - c);
+            mc[t - lo] = c;
+        }
     }
 }
 
@@ -754,6 +800,10 @@ __global__ void k_iota_from(int32_t *__restrict__ o, int64_t n, int32_t first)
 constexpr int kWalkClasses = 4;
 constexpr int kWalkClassW[kWalkClasses] = {16, 8, 4, 4};
 constexpr int kWalkClassM[kWalkClasses] = {256, 96, 48, 0};
+// with few peaks (four waves or more each in the gather) the groups are four
+// times as wide, 64 at most: 2000 peaks of 128^3 0.88 ms (x2 0.91, x1 0.94),
+// 20 k of 256^3 1.31 (1.31, 1.38), 60 k 1.64 (1.65, 1.75)
+constexpr int kWalkWide = 4;
 struct WalkClasses {
     int64_t lo[kWalkClasses], hi[kWalkClasses];  // positions in the lane-post order, relative to its start
     int32_t blk[kWalkClasses + 1];               // first workgroup of each class
@@ -803,6 +853,7 @@ __device__ __forceinline__ void walk_group_class(const PeakParam *__restrict__ p
     }
 }
 
+template <int F>
 __global__ void __launch_bounds__(256) k_walk_group(const PeakParam *__restrict__ pps, int64_t lo,
                                                     const int32_t *__restrict__ list, ProfBuf prof,
                                                     const int64_t *__restrict__ prof_off, PostConst C,
@@ -814,10 +865,10 @@ __global__ void __launch_bounds__(256) k_walk_group(const PeakParam *__restrict_
     const int64_t b0 = K.blk[k], nb = K.blk[k + 1] - K.blk[k];
     if (nb <= 0) return;
     switch (k) {
-    case 0: walk_group_class<kWalkClassW[0]>(pps, lo, K.lo[0], K.hi[0], b0, nb, list, prof, prof_off, C, eoff, mc, out); break;
-    case 1: walk_group_class<kWalkClassW[1]>(pps, lo, K.lo[1], K.hi[1], b0, nb, list, prof, prof_off, C, eoff, mc, out); break;
-    case 2: walk_group_class<kWalkClassW[2]>(pps, lo, K.lo[2], K.hi[2], b0, nb, list, prof, prof_off, C, eoff, mc, out); break;
-    default: walk_group_class<kWalkClassW[3]>(pps, lo, K.lo[3], K.hi[3], b0, nb, list, prof, prof_off, C, eoff, mc, out); break;
+    case 0: walk_group_class<std::min(64, F * kWalkClassW[0])>(pps, lo, K.lo[0], K.hi[0], b0, nb, list, prof, prof_off, C, eoff, mc, out); break;
+    case 1: walk_group_class<std::min(64, F * kWalkClassW[1])>(pps, lo, K.lo[1], K.hi[1], b0, nb, list, prof, prof_off, C, eoff, mc, out); break;
+    case 2: walk_group_class<std::min(64, F * kWalkClassW[2])>(pps, lo, K.lo[2], K.hi[2], b0, nb, list, prof, prof_off, C, eoff, mc, out); break;
+    default: walk_group_class<std::min(64, F * kWalkClassW[3])>(pps, lo, K.lo[3], K.hi[3], b0, nb, list, prof, prof_off, C, eoff, mc, out); break;
     }
 }
 
@@ -894,20 +945,26 @@ __global__ void __launch_bounds__(64) k_post_wave(const PeakParam *__restrict__ 
     }
 }
 
-// W lanes per peak, 64 / W peaks per wave
+// W lanes per peak, 64 / W peaks per wave; list and walk table as k_post_lane's
 template <int W>
 __global__ void __launch_bounds__(64) k_post_group(const PeakParam *__restrict__ pps, int64_t lo, int64_t hi,
                                                    ProfBuf prof, const int64_t *__restrict__ prof_off,
-                                                   PostConst C, ResultView R)
+                                                   PostConst C, ResultView R, const int32_t *__restrict__ list,
+                                                   const WalkRec *__restrict__ wtab, const int64_t *__restrict__ eoff,
+                                                   const int64_t *__restrict__ wmc)
 {
     constexpr int G = 64 / W;
     const int grp = threadIdx.x / W;
     for (int64_t b0 = lo + (int64_t)blockIdx.x * G; b0 < hi; b0 += (int64_t)gridDim.x * G) {
-        const int64_t idx = b0 + grp;
-        if (idx >= hi) continue;  // whole lane groups drop out
+        if (b0 + grp >= hi) continue;  // whole lane groups drop out
+        const int64_t idx = list ? (int64_t)list[b0 + grp - lo] : b0 + grp;
         const PeakParam pk = pps[idx];
         const int64_t rb = prof_off[idx];
-        const AosProfile<false> P = profile_at<false>(prof, rb, C.rad, false);
+        AosProfile<false> P = profile_at<false>(prof, rb, C.rad, false);
+        if (wtab) {
+            P.wt = wtab + eoff[idx - lo];
+            P.wmc = (int)wmc[idx - lo];
+        }
         analyse_post<W, false>(P, pk, C, R, pk.order);
         if ((threadIdx.x & (W - 1)) == 0) R.nshells[pk.order] = pk.m;
     }
@@ -938,9 +995,12 @@ struct FinishArgs {
     ResultView R;
 };
 
-__global__ void __launch_bounds__(64) k_finish(FinishArgs A)
+template <int NW>
+__global__ void __launch_bounds__(64 * NW) k_finish(FinishArgs A)
 {
-    const int lane = threadIdx.x;
+    __shared__ double part[NW][9];
+    __shared__ int left[NW];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const GatherFields &F = A.F;
     const PostConst &C = A.C;
     const ResultView &R = A.R;
@@ -960,7 +1020,7 @@ __global__ void __launch_bounds__(64) k_finish(FinishArgs A)
         const bool inside = pk.flags & 1;
         double Sb[3] = {0, 0, 0}, Sb2[3] = {0, 0, 0}, nS = 0.0, sL = 0.0, nL = 0.0;
         bool oob = false;
-        if (lane == 0) {  // centre cell: shell 1 (in Sbar, in the mask, not in d2F)
+        if (threadIdx.x == 0) {  // centre cell: shell 1 (in Sbar, in the mask, not in d2F)
             const long a = pk.ci + pk.cj * n1 + pk.ck * n12;
             for (int L = 0; L < 3; L++) {
                 Sb[L] += (double)ex[L][a];
@@ -976,7 +1036,7 @@ __global__ void __launch_bounds__(64) k_finish(FinishArgs A)
             const bool full = s0 + A.cs - 1 <= m;
             const GroupDesc *tab = A.desc + (full ? A.full_off[c] : A.part_off[m]);
             const int nb = full ? A.full_nb[c] : A.part_nb[m];
-            for (int b = 0; b < nb; b++) {
+            for (int b = wave; b < nb; b += NW) {
                 const GroupDesc g = tab[b * 64 + lane];
                 const int l = g.lmn & 255, dj = (g.lmn >> 8) & 255, dk = (g.lmn >> 16) & 255;
                 // rows come by increasing dj^2 + dk^2: once a batch's smallest
@@ -1019,18 +1079,40 @@ __global__ void __launch_bounds__(64) k_finish(FinishArgs A)
                 }
             }
         }
-        if (__ballot(oob) != 0ull) {
+        bool out = __ballot(oob) != 0ull;
+        if (NW > 1) {
+            if (lane == 0) left[wave] = out;
+            __syncthreads();
+            for (int w = 0; w < NW; w++) out = out || left[w];
+            __syncthreads();  // read before the next peak's
+        }
+        if (out) {
             // rare: R_TH reaches past the grid edge; the ordered walk
             // recomputes this peak's outputs (its mask writes repeat the same
             // 1s)
-            finish_cells<true>(C, pk, m0, q, ex, e2, R, o);
+            if (wave == 0) finish_cells<true>(C, pk, m0, q, ex, e2, R, o);
             continue;
         }
         for (int L = 0; L < 3; L++) { Sb[L] = wave_sum(Sb[L]); Sb2[L] = wave_sum(Sb2[L]); }
         nS = wave_sum(nS);
         sL = wave_sum(sL);
         nL = wave_sum(nL);
-        if (lane == 0) {
+        if (NW > 1) {
+            if (lane == 0) {
+                double *p = part[wave];
+                for (int L = 0; L < 3; L++) { p[L] = Sb[L]; p[3 + L] = Sb2[L]; }
+                p[6] = nS; p[7] = sL; p[8] = nL;
+            }
+            __syncthreads();
+            if (threadIdx.x == 0)
+                for (int w = 1; w < NW; w++) {
+                    const double *p = part[w];
+                    for (int L = 0; L < 3; L++) { Sb[L] += p[L]; Sb2[L] += p[3 + L]; }
+                    nS += p[6]; sL += p[7]; nL += p[8];
+                }
+            __syncthreads();
+        }
+        if (threadIdx.x == 0) {
             for (int L = 0; L < 3; L++) {
                 R.Sbar[o * 3 + L] = nS > 0.0 ? Sb[L] / nS : 0.0;
                 R.Sbar2[o * 3 + L] = nS > 0.0 ? Sb2[L] / nS : 0.0;
@@ -1418,6 +1500,10 @@ static int run_persistent_impl(pp_ctx *ctx, GatherFields G, ShellRun &S, PostCon
     if (ctx->post_width <= 1 && small_lo - std::min(small_lo, cnt_gt(coop_m)) <= kLaneTableMin)
         coop_m = std::min(coop_m, 64);
     const int64_t coop_end = std::min(small_lo, cnt_gt(coop_m));
+    // waves per peak in the gather and the finish pass
+    int waves = 8;
+    for (int64_t bound : kSharedPeaksPerCU)
+        if (small_lo > ctx->num_cu * bound) waves /= 2;
     // 3. profile offsets: exclusive scan of m over all peaks
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
     int64_t tot = 0;
@@ -1571,7 +1657,7 @@ static int run_persistent_impl(pp_ctx *ctx, GatherFields G, ShellRun &S, PostCon
         d_wmc = ctx->d_cross.as<int64_t>();
         d_weoff = (int64_t *)(ctx->d_cross.as<char>() + al((size_t)nl * 8));
         uint32_t *ka = (uint32_t *)W.ka, *kb = (uint32_t *)W.kb;
-        hipLaunchKernelGGL(k_crossing_keys, dim3(grid1d(ctx, nl)), dim3(256), 0, ctx->stream, (const PeakParam *)pps,
+        hipLaunchKernelGGL(k_crossing_keys, dim3(grid1d(ctx, nl * kCrossLanes)), dim3(256), 0, ctx->stream, (const PeakParam *)pps,
                            cross_lo, cross_hi, d_rec, (const int64_t *)d_off, C.rad, cmax, cbits, ka, d_wmc);
         hipLaunchKernelGGL(k_iota_from, dim3(grid1d(ctx, nl)), dim3(256), 0, ctx->stream, W.iota, nl, (int32_t)cross_lo);
         PP_HIP(hipGetLastError());
@@ -1606,6 +1692,7 @@ static int run_persistent_impl(pp_ctx *ctx, GatherFields G, ShellRun &S, PostCon
         // classes: consecutive runs of the lane-post order (m descending)
         WalkClasses K{};
         int64_t want[kWalkClasses], tot = 0, pos = 0;
+        const bool wide = waves > 2;  // few peaks
         for (int k = 0; k < kWalkClasses; k++) {
             const int mlo = std::max(kWalkClassM[k], small_m + 1);
             const int mhi = k == 0 ? cmax : kWalkClassM[k - 1] - 1;
@@ -1613,7 +1700,7 @@ static int run_persistent_impl(pp_ctx *ctx, GatherFields G, ShellRun &S, PostCon
             for (int x = mlo; x <= std::min(mhi, cmax) && x < nb; x++) cnt += hist[x];
             K.lo[k] = pos;
             K.hi[k] = pos += cnt;
-            want[k] = (cnt * kWalkClassW[k] + 255) / 256;
+            want[k] = (cnt * std::min(64, (wide ? kWalkWide : 1) * kWalkClassW[k]) + 255) / 256;
             tot += want[k];
         }
         if (pos != cross_hi - cross_lo) {
@@ -1628,8 +1715,8 @@ static int run_persistent_impl(pp_ctx *ctx, GatherFields G, ShellRun &S, PostCon
             K.blk[k + 1] = K.blk[k] + (int32_t)b;
         }
         if (K.blk[kWalkClasses] == 0) return PP_OK;
-        hipLaunchKernelGGL(k_walk_group, dim3(K.blk[kWalkClasses]), dim3(256), 0, ctx->stream,
-                           (const PeakParam *)pps, cross_lo, cross_list, d_rec, (const int64_t *)d_off, C,
+        hipLaunchKernelGGL(wide ? k_walk_group<kWalkWide> : k_walk_group<1>, dim3(K.blk[kWalkClasses]), dim3(256), 0,
+                           ctx->stream, (const PeakParam *)pps, cross_lo, cross_list, d_rec, (const int64_t *)d_off, C,
                            (const int64_t *)d_weoff, (const int64_t *)d_wmc, d_wtab, K);
         PP_HIP(hipGetLastError());
         return PP_OK;
@@ -1729,9 +1816,15 @@ static int run_persistent_impl(pp_ctx *ctx, GatherFields G, ShellRun &S, PostCon
         A.prof = d_rec; A.prof_off = d_off; A.rad = C.rad; A.queue = d_q; A.cs = cs; A.steps = st.gsteps;
         A.xorder = W.xg; A.nx = nx;
         for (int x = 0; x <= NXCD; x++) A.xb[x] = xbg[x];
-        if (lds > 64 * 1024)
-            (void)hipFuncSetAttribute((const void *)k_gather, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        hipLaunchKernelGGL(k_gather, dim3(grid), dim3(64), lds, ctx->stream, A);
+        auto launch = [&](auto kern) {
+            if (lds > 64 * 1024)
+                (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * waves), lds, ctx->stream, A);
+        };
+        if (waves == 8) launch(k_gather<8>);
+        else if (waves == 4) launch(k_gather<4>);
+        else if (waves == 2) launch(k_gather<2>);
+        else launch(k_gather<1>);
         PP_HIP(hipGetLastError());
     }
     PP_HIP(hipEventRecord(ctx->ev[4], ctx->stream));
@@ -1740,20 +1833,24 @@ static int run_persistent_impl(pp_ctx *ctx, GatherFields G, ShellRun &S, PostCon
     // 5. posts: the wave post runs on the side stream (before the small
     // peaks' work), beside the lane post on the main stream
     PP_HIP(hipEventRecord(ctx->ev[5], ctx->stream));
-    if (ctx->post_width <= 1) {
-        PP_CHECK(walk_table());
+    if (ctx->post_width <= 1) PP_CHECK(walk_table());
+    // one lane per peak, or groups of lanes as far as that only fills idle SIMDs
+    int width = std::max(ctx->post_width, 1);
+    if (d_wtab && ctx->lane_walk == 0)
+        while (width < kGroupPost && (small_lo - coop_end) * width * 2 <= (int64_t)ctx->num_cu * kGroupPostLanesCU) width *= 2;
+    if (width == 1) {
         PP_CHECK(post_lane(coop_end, small_lo, false));
     } else if (small_lo > coop_end) {
-        const int W = ctx->post_width;
-        const int64_t nwav = (small_lo - coop_end + 64 / W - 1) / (64 / W);
+        const int64_t nwav = (small_lo - coop_end + 64 / width - 1) / (64 / width);
         const int gp = (int)std::max<int64_t>(1, std::min<int64_t>(nwav, (int64_t)ctx->num_cu * 16));
         auto launch = [&](auto kern) {
             hipLaunchKernelGGL(kern, dim3(gp), dim3(64), 0, ctx->stream, (const PeakParam *)pps, coop_end, small_lo,
-                               d_rec, (const int64_t *)d_off, C, S.R);
+                               d_rec, (const int64_t *)d_off, C, S.R, cross_list, (const WalkRec *)d_wtab,
+                               (const int64_t *)d_weoff, (const int64_t *)d_wmc);
         };
-        if (W == 2) launch(k_post_group<2>);
-        else if (W == 4) launch(k_post_group<4>);
-        else if (W == 8) launch(k_post_group<8>);
+        if (width == 2) launch(k_post_group<2>);
+        else if (width == 4) launch(k_post_group<4>);
+        else if (width == 8) launch(k_post_group<8>);
         else launch(k_post_group<16>);
         PP_HIP(hipGetLastError());
     }
@@ -1771,7 +1868,11 @@ static int run_persistent_impl(pp_ctx *ctx, GatherFields G, ShellRun &S, PostCon
         A.full_off = st.d_full_off.as<int64_t>(); A.full_nb = st.d_full_nb.as<int32_t>();
         A.part_off = st.d_part_off.as<int64_t>(); A.part_nb = st.d_part_nb.as<int32_t>();
         A.cs = cs; A.C = C; A.R = S.R;
-        hipLaunchKernelGGL(k_finish, dim3(gf), dim3(64), 0, ctx->stream, A);
+        auto launch = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(gf), dim3(64 * waves), 0, ctx->stream, A); };
+        if (waves == 8) launch(k_finish<8>);
+        else if (waves == 4) launch(k_finish<4>);
+        else if (waves == 2) launch(k_finish<2>);
+        else launch(k_finish<1>);
         PP_HIP(hipGetLastError());
     }
     PP_HIP(hipEventRecord(ctx->ev[7], ctx->stream));

@@ -417,11 +417,11 @@ __device__ __forceinline__ int tab_crossing(const PV &P)
 
 // Ebar of a walk step: the peak's walk-table record for mp when it was formed
 // on the same band (identical to kernel_strain's, which computed it), else
-// kernel_strain itself.  Only the one-lane-per-peak post has a table.
+// kernel_strain itself.  The wave post has no table.
 template <int W, class PV>
 __device__ __forceinline__ Strain walk_strain(const PV &P, const PostConst &C, int mp, int mlow, int mupp)
 {
-    if constexpr (W == 1) {
+    if constexpr (W < 64) {
         if (P.wt && mp <= P.wmc) {
             const WalkRec *r = P.wt + (mp - 1);
             const int2 band = *(const int2 *)&r->mlow;
@@ -597,24 +597,29 @@ __device__ void finish_records(const PV &P, const PeakParam &pk, const PostConst
     }
 }
 
-// The fcrit crossing of one peak, serially (RadialShell.jl:492-538): the m0
-// the inward walk starts from, as analyse_post<1> finds it; 0 when there is
-// none (a DUMP_NO_FCRIT peak).  Used to order the lane post's peaks.
-template <class PV>
+// The fcrit crossing of one peak (RadialShell.jl:492-538), W lanes on W shells
+// at a time: the m0 the inward walk starts from, as analyse_post finds it; 0
+// when there is none (a DUMP_NO_FCRIT peak).  Used to order the lane post's
+// peaks.
+template <int W, class PV>
 __device__ int crossing_m0(const PV &P, const PeakParam &pk)
 {
+    using X = Exec<W>;
+    const int lane = X::lane();
     const double fcrit = pk.fcrit;
-    const int m = pk.m;
-    int m0 = pk.m0;
+    const int m = pk.m, m0 = pk.m0;
     if (P.Fbar(m0) >= fcrit) {
-        for (int mm = m0; mm <= m; mm++)
-            if (P.Fbar(mm) < fcrit) return mm;
+        for (int base = m0; base <= m; base += W) {
+            const int mm = base + lane;
+            const unsigned long long b = X::ballot(mm <= m && P.Fbar(mm) < fcrit);
+            if (b) return base + __ffsll((long long)b) - 1;
+        }
         return m0;
     }
-    const int mstart = m0 - 1 > 1 ? m0 - 1 : 1;
-    for (int mp = mstart; mp >= 1; mp--) {
-        if (P.Fbar(mp) >= fcrit) return m0;
-        m0 = mp;
+    for (int top = m0 - 1 > 1 ? m0 - 1 : 1; top >= 1; top -= W) {
+        const int mp = top - lane;
+        const unsigned long long b = X::ballot(mp >= 1 && P.Fbar(mp) >= fcrit);
+        if (b) return top - (__ffsll((long long)b) - 1) + 1;
     }
     return 0;
 }
@@ -649,8 +654,8 @@ __device__ int analyse_post(const PV &P, const PeakParam &pk, const PostConst &C
         // ---- Phase 4: fcrit crossing (RadialShell.jl:492-538) ----
         const double fcrit = pk.fcrit;
         int m0 = pk.m0, mupp;
-        bool tab = false;  // the walk table (one lane per peak): crossing, bands and steps from it
-        if constexpr (W == 1) tab = P.wt != nullptr;
+        bool tab = false;  // the walk table (lane and group posts): crossing, bands and steps from it
+        if constexpr (W < 64) tab = P.wt != nullptr;
         if (tab) {
             // the crossing crossing_m0 found ahead of the walk (0: none); an
             // outward search that found none (the crossing is pk.m0 itself)
