@@ -115,6 +115,8 @@ struct FftPlans {
     int n = 0, kind = 0;
     unsigned long long last_use = 0;
     size_t work_need = 0;  // work area bytes; kind 1 sets its work area per use (stream ordered)
+    rocfft_plan c2r_pad = nullptr;  // fft_padded's
+    bool pad_asked = false;
     rocfft_plan r2c = nullptr, c2r = nullptr;
     rocfft_execution_info info = nullptr;
     DevBuf work;
@@ -169,6 +171,14 @@ struct pp_ctx {
 namespace pp {
 int fft_prepare(pp_ctx *ctx, int n);                       // makes the n^3 out-of-place set current
 int fft_plans(pp_ctx *ctx, int n, int kind, FftPlans **out);  // a cached set, without changing the current one
+// c2r of a kind 0 set from rows of `pitch` and planes of `plane` elements in *P
+// (the set's plain layout where no better one is known)
+struct FftLayout {
+    rocfft_plan c2r;
+    int pitch;
+    size_t plane;
+};
+int fft_padded(FftPlans &F, FftLayout *P);
 void persist_release(pp_ctx *ctx);    // pp_persist.hip: drops the context's gather tables
 int noalloc_scratch_init(int device);  // pp_filter.hip: device address of the static scratch
 void line_release(pp_ctx *ctx);       // drops the line transforms' tables

@@ -54,6 +54,9 @@ void FftPlans::release()
 {
     if (r2c) rocfft_plan_destroy(r2c);
     if (c2r) rocfft_plan_destroy(c2r);
+    if (c2r_pad) rocfft_plan_destroy(c2r_pad);
+    c2r_pad = nullptr;
+    pad_asked = false;
     if (info) rocfft_execution_info_destroy(info);
     r2c = c2r = nullptr;
     info = nullptr;
@@ -114,6 +117,40 @@ static int fft_create(pp_ctx *ctx, FftPlans &F, int n, int kind)
     }
     F.n = n;
     F.kind = kind;
+    return PP_OK;
+}
+
+// Rows of n / 2 + 1 elements straddle cache lines, which costs rocFFT's column
+// kernels for powers of two a fifth to a quarter of the transform: from rows of
+// whole 64-byte lines and planes apart from a power of two the inverse takes
+// 109 us instead of 152 at 256^3 and 1205 instead of 1490 at 512^3, with the
+// same bits (the same kernels at other strides).  Not below 256 (128^3: 28 us
+// against 24, other kernels and other bits), nor at the other sizes (192 to
+// 480: between 3 % less and 10 % more), nor where a plan needs a work area
+// (1024^3: no gain, and twice the area).
+int fft_padded(FftPlans &F, FftLayout *P)
+{
+    const size_t n = (size_t)F.n, nk = n / 2 + 1, pitch = (nk + 7) / 8 * 8, plane = pitch * n + 24;
+    if (!F.pad_asked && F.kind == 0 && n >= 256 && (n & (n - 1)) == 0 && F.work_need == 0) {
+        size_t len[3] = {n, n, n}, cs[3] = {1, pitch, plane}, rs[3] = {1, n, n * n}, w = 0;
+        rocfft_plan_description d = nullptr;
+        PP_FFT(rocfft_plan_description_create(&d));
+        rocfft_status st = rocfft_plan_description_set_data_layout(d, rocfft_array_type_hermitian_interleaved,
+                                                                   rocfft_array_type_real, nullptr, nullptr, 3, cs,
+                                                                   plane * n, 3, rs, n * n * n);
+        if (st == rocfft_status_success)
+            st = rocfft_plan_create(&F.c2r_pad, rocfft_placement_notinplace, rocfft_transform_type_real_inverse,
+                                    rocfft_precision_single, 3, len, 1, d);
+        rocfft_plan_description_destroy(d);
+        if (st == rocfft_status_success) st = rocfft_plan_get_work_buffer_size(F.c2r_pad, &w);
+        if (F.c2r_pad && (st != rocfft_status_success || w > 0)) {
+            rocfft_plan_destroy(F.c2r_pad);
+            F.c2r_pad = nullptr;
+        }
+    }
+    F.pad_asked = true;
+    if (F.c2r_pad) *P = FftLayout{F.c2r_pad, (int)pitch, plane};
+    else *P = FftLayout{F.c2r, (int)nk, nk * n};
     return PP_OK;
 }
 

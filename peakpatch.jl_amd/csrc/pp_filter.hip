@@ -40,6 +40,8 @@ namespace pp {
 struct WinSel {
     float2 *out;
     int wsmooth;  // PP_WINDOW_*; < 0: no output
+    int pitch;    // elements of a row and of a plane of out
+    size_t plane;
 };
 
 __device__ __forceinline__ double window_value(int wsmooth, double k, double fkR)
@@ -71,13 +73,12 @@ __global__ void __launch_bounds__(256) k_window(const float2 *__restrict__ in, W
     const int ny = iy2 == hy ? 1 : 2, nz = iz2 == hz ? 1 : 2;
     // the (up to) four elements are loaded before the Float64 window is
     // evaluated, so their latency hides behind it
-    size_t el[4];
     float2 vin[4];
 #pragma unroll
     for (int q = 0; q < 4; q++) {
         const int iy = (q & 1) ? iy2 : hy, iz = (q & 2) ? iz2 : hz;
-        el[q] = (size_t)ix + (size_t)nk * ((size_t)iy + (size_t)n * (size_t)iz);
-        if ((q & 1) < ny && (q >> 1) < nz) vin[q] = in[el[q]];
+        if ((q & 1) < ny && (q >> 1) < nz)
+            vin[q] = in[(size_t)ix + (size_t)nk * ((size_t)iy + (size_t)n * (size_t)iz)];
     }
     const double kx = dk * (double)ix, ky = dk * (double)hy, kz = dk * (double)hz;
     const double k = sqrt(kx * kx + ky * ky + kz * kz);
@@ -92,33 +93,35 @@ __global__ void __launch_bounds__(256) k_window(const float2 *__restrict__ in, W
     for (int q = 0; q < 4; q++) {
         if ((q & 1) >= ny || (q >> 1) >= nz) continue;
         {
-            const size_t e = el[q];
+            const int iy = (q & 1) ? iy2 : hy, iz = (q & 2) ? iz2 : hz;
             const float2 v = vin[q];
             float2 r = v;
             if (scaled) { r.x = r.x * wa; r.y = r.y * wa; }
             r.x = r.x * scale;
             r.y = r.y * scale;
-            a.out[e] = r;
+            a.out[ix + (size_t)a.pitch * iy + a.plane * iz] = r;
             if (b.wsmooth >= 0) {
                 float2 s = v;
                 if (scaled) { s.x = s.x * wb; s.y = s.y * wb; }
                 s.x = s.x * scale;
                 s.y = s.y * scale;
-                b.out[e] = s;
+                b.out[ix + (size_t)b.pitch * iy + b.plane * iz] = s;
             }
         }
     }
 }
 
-static int launch_window2(pp_ctx *ctx, const void *in, void *out_a, int ws_a, void *out_b, int ws_b, int n,
-                          double boxsize, double Rf, float scale)
+static int launch_window2(pp_ctx *ctx, const void *in, void *out_a, int ws_a, const FftLayout *lay_a, void *out_b,
+                          int ws_b, int n, double boxsize, double Rf, float scale)
 {
     const int nk = n / 2 + 1, half = n / 2;
     const long long per = (long long)nk * (half + 1);
     PP_ARG(per < (1ll << 31) && half + 1 <= 65535, "mesh %d too large for the window grid", n);
     const double dk = 2.0 * M_PI / boxsize;
     dim3 grid((unsigned)((per + 255) / 256), (unsigned)(half + 1));
-    WinSel a{(float2 *)out_a, ws_a}, b{(float2 *)out_b, out_b ? ws_b : -1};
+    const size_t plane = (size_t)nk * n;
+    WinSel a{(float2 *)out_a, ws_a, lay_a ? lay_a->pitch : nk, lay_a ? lay_a->plane : plane};
+    WinSel b{(float2 *)out_b, out_b ? ws_b : -1, nk, plane};
     hipLaunchKernelGGL(k_window, grid, dim3(256), 0, ctx->stream, (const float2 *)in, a, b, n, nk, dk, Rf, scale);
     PP_HIP(hipGetLastError());
     return PP_OK;
@@ -127,7 +130,7 @@ static int launch_window2(pp_ctx *ctx, const void *in, void *out_a, int ws_a, vo
 static int launch_window(pp_ctx *ctx, const void *in, void *out, int n, double boxsize, double Rf,
                          int wsmooth, float scale)
 {
-    return launch_window2(ctx, in, out, wsmooth, nullptr, -1, n, boxsize, Rf, scale);
+    return launch_window2(ctx, in, out, wsmooth, nullptr, nullptr, -1, n, boxsize, Rf, scale);
 }
 
 // ------------------------------------------------------------- stencil
@@ -960,8 +963,10 @@ int pp_find_peaks(pp_ctx *ctx, const float *delta, int on_device, int n, double 
     if (max_peaks_per_filter <= 0) max_peaks_per_filter = 2000000;
     size_t N = (size_t)n * n * n;
     size_t rb = N * sizeof(float), cb = (size_t)(n / 2 + 1) * n * n * sizeof(float2);
+    FftLayout lay;  // of each filter's spectrum
+    PP_CHECK(fft_padded(*ctx->fftp, &lay));
     PP_CHECK(ctx->d_k0.grow(cb));
-    PP_CHECK(ctx->d_k1.grow(cb));
+    PP_CHECK(ctx->d_k1.grow(lay.plane * n * sizeof(float2)));
     PP_CHECK(ctx->d_field_a.grow(rb));
     // the wsmooth = 3 field at the peaks: line transforms where the mesh has
     // them, else a second rocFFT inverse per filter
@@ -1001,11 +1006,11 @@ int pp_find_peaks(pp_ctx *ctx, const float *delta, int on_device, int n, double 
         // one read of delta_k gives the filter's spectrum and, with want_lapd
         // and no line transform, the wsmooth = 3 spectrum sampled at the
         // filter's new peaks
-        PP_CHECK(launch_window2(ctx, ctx->d_k0.ptr, ctx->d_k1.ptr, wsmooth,
+        PP_CHECK(launch_window2(ctx, ctx->d_k0.ptr, ctx->d_k1.ptr, wsmooth, &lay,
                                 want_lapd && !lines ? ctx->d_k2.ptr : nullptr, PP_WINDOW_K2GAUSS, n, boxsize, Rf[f],
                                 inv));
         void *ib[1] = {ctx->d_k1.ptr}, *ob[1] = {ctx->d_field_a.ptr};
-        PP_FFT(rocfft_execute(ctx->fftp->c2r, ib, ob, ctx->fftp->info));
+        PP_FFT(rocfft_execute(lay.c2r, ib, ob, ctx->fftp->info));
         PP_CHECK(run_stencil(ctx, ctx->d_field_a.as<float>(), d_mask, g, fcrit[f], max_peaks_per_filter, f,
                              o, d_counters, S, lines ? K.ranges + 2 * f : nullptr));
         if (lines) {
