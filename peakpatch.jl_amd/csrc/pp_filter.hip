@@ -527,7 +527,7 @@ static int stencil_start(pp_ctx *ctx, const StencilGeom &g, long long *d_counter
 // only.  Its inverse transform (rocFFT: 1.46 ms at 512^3, after half of
 // k_window's 0.31 ms) is done on line transforms (pp_fft.h) instead, as far as
 // the peaks need it: the window goes into the z pass, planes and rows outside
-// the inner cube are not written, modes whose Gaussian is below 1e-20 are not
+// the inner cube are not written, modes whose Gaussian is below 1e-12 are not
 // read, and only the row pairs that hold a peak are transformed along x, from
 // where the peaks' values are taken without a field.  The passes run on the
 // side stream beside the next filters' rocFFT kernels, which leave most of
@@ -717,8 +717,10 @@ static int bank_transform(pp_ctx *ctx, Bank &K, const double *Rf, int f)
     const SpecGeo &g = K.G.g;
     const int n = g.n, half = n / 2;
     K.B.gauss = K.tables + (size_t)f * (half + 1);
-    // exp(-(c dk R)^2 / 8) < 1e-20: below every Float32 rounding of the result
-    const double c = sqrt(8.0 * 46.0) / fabs(K.dk * Rf[f]);
+    // exp(-(c dk R)^2 / 8) < 1e-12: with the growth of k^2 and of the number of
+    // modes out to there (30 and 10 times those at the window's edge) 3e-10 of
+    // the field, far below its Float32 rounding
+    const double c = sqrt(8.0 * 27.64) / fabs(K.dk * Rf[f]);
     K.B.cut = c < half ? (int)c + 1 : half;
     K.B.plain = Rf[f] == 0.0;
     const int rows = std::min(n, 2 * K.B.cut + 1), bins = std::min(K.B.cut, g.nk - 1) + 1;
