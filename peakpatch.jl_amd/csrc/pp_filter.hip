@@ -59,15 +59,28 @@ __device__ __forceinline__ double window_value(int wsmooth, double k, double fkR
     return 3.0 * (s - fkR * c) / (fkR * fkR * fkR);
 }
 
-__global__ void __launch_bounds__(256) k_window(const float2 *__restrict__ in, WinSel a, WinSel b, int n, int nk,
-                                                double dk, double Rf, float scale)
+// a filter's window multiplication: gx x gz workgroups
+struct WinJob {
+    const float2 *in;
+    WinSel a, b;
+    int n, nk;
+    double dk, Rf;
+    float scale;
+    int gx, gz;
+};
+
+__device__ __forceinline__ void window_block(const WinJob &J, int bx, int hz)
 {
 #pragma clang fp contract(off)
+    const float2 *__restrict__ in = J.in;
+    const WinSel &a = J.a, &b = J.b;
+    const int n = J.n, nk = J.nk;
+    const double dk = J.dk, Rf = J.Rf;
+    const float scale = J.scale;
     const int half = n / 2;
-    const int idx = blockIdx.x * 256 + threadIdx.x;
+    const int idx = bx * 256 + threadIdx.x;
     const int hy = idx / nk;
     const int ix = idx - hy * nk;
-    const int hz = blockIdx.y;
     if (hy > half) return;
     const int iy2 = hy == 0 ? 0 : n - hy, iz2 = hz == 0 ? 0 : n - hz;
     const int ny = iy2 == hy ? 1 : 2, nz = iz2 == hz ? 1 : 2;
@@ -111,18 +124,25 @@ __global__ void __launch_bounds__(256) k_window(const float2 *__restrict__ in, W
     }
 }
 
-static int launch_window2(pp_ctx *ctx, const void *in, void *out_a, int ws_a, const FftLayout *lay_a, void *out_b,
-                          int ws_b, int n, double boxsize, double Rf, float scale)
+__global__ void __launch_bounds__(256) k_window(WinJob J) { window_block(J, blockIdx.x, blockIdx.y); }
+
+static int window_job(const void *in, void *out_a, int ws_a, const FftLayout *lay_a, void *out_b, int ws_b, int n,
+                      double boxsize, double Rf, float scale, WinJob *J)
 {
     const int nk = n / 2 + 1, half = n / 2;
     const long long per = (long long)nk * (half + 1);
     PP_ARG(per < (1ll << 31) && half + 1 <= 65535, "mesh %d too large for the window grid", n);
-    const double dk = 2.0 * M_PI / boxsize;
-    dim3 grid((unsigned)((per + 255) / 256), (unsigned)(half + 1));
     const size_t plane = (size_t)nk * n;
-    WinSel a{(float2 *)out_a, ws_a, lay_a ? lay_a->pitch : nk, lay_a ? lay_a->plane : plane};
-    WinSel b{(float2 *)out_b, out_b ? ws_b : -1, nk, plane};
-    hipLaunchKernelGGL(k_window, grid, dim3(256), 0, ctx->stream, (const float2 *)in, a, b, n, nk, dk, Rf, scale);
+    *J = WinJob{(const float2 *)in,
+                {(float2 *)out_a, ws_a, lay_a ? lay_a->pitch : nk, lay_a ? lay_a->plane : plane},
+                {(float2 *)out_b, out_b ? ws_b : -1, nk, plane},
+                n, nk, 2.0 * M_PI / boxsize, Rf, scale, (int)((per + 255) / 256), half + 1};
+    return PP_OK;
+}
+
+static int launch_window(pp_ctx *ctx, const WinJob &J)
+{
+    hipLaunchKernelGGL(k_window, dim3(J.gx, J.gz), dim3(256), 0, ctx->stream, J);
     PP_HIP(hipGetLastError());
     return PP_OK;
 }
@@ -130,7 +150,9 @@ static int launch_window2(pp_ctx *ctx, const void *in, void *out_a, int ws_a, co
 static int launch_window(pp_ctx *ctx, const void *in, void *out, int n, double boxsize, double Rf,
                          int wsmooth, float scale)
 {
-    return launch_window2(ctx, in, out, wsmooth, nullptr, nullptr, -1, n, boxsize, Rf, scale);
+    WinJob J;
+    PP_CHECK(window_job(in, out, wsmooth, nullptr, nullptr, -1, n, boxsize, Rf, scale, &J));
+    return launch_window(ctx, J);
 }
 
 // ------------------------------------------------------------- stencil
@@ -358,14 +380,21 @@ __global__ void __launch_bounds__(256) k_peak_sums(const int *__restrict__ count
 // sums for each workgroup.  The filter's first slot is base[parity]; the last
 // workgroup leaves the next one in the other word (counters[0] itself would
 // need every workgroup to have read it: a device-wide fence by each took 0.2
-// ms at 512^3).
+// ms at 512^3).  With WIN the workgroups from nemit on multiply the next
+// filter's window, which needs nothing of this one's peaks.
+template <bool WIN>
 __global__ void __launch_bounds__(256) k_peak_emit(const float *__restrict__ d, int8_t *__restrict__ mask,
                                                    StencilGeom g, StencilTiles tl, const uint64_t *__restrict__ bits,
                                                    const int *__restrict__ before, int per,
                                                    long long *__restrict__ base, int parity,
                                                    long long *__restrict__ counters, long long max_peaks, int filt,
-                                                   PeakOut o, long long *__restrict__ range)
+                                                   PeakOut o, long long *__restrict__ range, int nemit, WinJob J)
 {
+    if (WIN && (int)blockIdx.x >= nemit) {
+        const int b = blockIdx.x - nemit, z = b / J.gx;
+        window_block(J, b - z * J.gx, z);
+        return;
+    }
     __shared__ int wsum[4];
     int sum = 0, total;
     for (long long q = threadIdx.x, e = (long long)blockIdx.x * per; q < e; q += 256) sum += before[q];
@@ -399,7 +428,7 @@ __global__ void __launch_bounds__(256) k_peak_emit(const float *__restrict__ d, 
             }
         }
     }
-    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
+    if ((int)blockIdx.x == nemit - 1 && threadIdx.x == 0) {
         const long long kept = first < max_peaks ? first : max_peaks;  // first: all of the filter's peaks
         base[parity ^ 1] = b0 + kept;
         counters[0] = b0 + kept;
@@ -470,16 +499,18 @@ static int stencil_clear(pp_ctx *ctx, const StencilScratch &s, long long *d_coun
 }
 
 // Stencil over one field, the step-th of a call; peaks appended after
-// counters[0].
+// counters[0].  The last launch also does the window of `next`: one launch less
+// a filter, which takes ten filters at 128^3, bound by the host, from 0.90 to
+// 0.84 ms and costs nothing at 512^3.
 static int run_stencil(pp_ctx *ctx, const float *d_field, int8_t *d_mask, const StencilGeom &g,
                        float fcrit, long long max_peaks, int step, const PeakOut &o, long long *d_counters,
-                       const StencilScratch &s, long long *range = nullptr)
+                       const StencilScratch &s, long long *range = nullptr, const WinJob *next = nullptr)
 {
     PP_ARG(g.nwords < (1ll << 31), "inner cube too large for the stencil");
     if (g.nwords == 0) {
         hipLaunchKernelGGL(k_stencil_none, dim3(1), dim3(1), 0, ctx->stream, d_counters, range);
         PP_HIP(hipGetLastError());
-        return PP_OK;
+        return next ? launch_window(ctx, *next) : PP_OK;
     }
     StencilTiles tl;
     tl.nbx = g.words;
@@ -507,9 +538,13 @@ static int run_stencil(pp_ctx *ctx, const float *d_field, int8_t *d_mask, const 
                            ncounts, tl.per, blocks, s.sums);
         PP_HIP(hipGetLastError());
     }
-    hipLaunchKernelGGL(k_peak_emit, dim3(blocks), dim3(256), 0, ctx->stream, d_field, d_mask, g, tl,
-                       (const uint64_t *)s.bits, (const int *)(sums ? s.sums : s.counts), sums ? 1 : tl.per, s.base,
-                       step & 1, d_counters, max_peaks, step, o, range);
+    auto emit = [&](auto kern, long long more) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)(blocks + more)), dim3(256), 0, ctx->stream, d_field, d_mask, g, tl,
+                           (const uint64_t *)s.bits, (const int *)(sums ? s.sums : s.counts), sums ? 1 : tl.per, s.base,
+                           step & 1, d_counters, max_peaks, step, o, range, blocks, next ? *next : WinJob{});
+    };
+    if (next) emit(k_peak_emit<true>, (long long)next->gx * next->gz);
+    else emit(k_peak_emit<false>, 0);
     PP_HIP(hipGetLastError());
     return PP_OK;
 }
@@ -1003,18 +1038,27 @@ int pp_find_peaks(pp_ctx *ctx, const float *delta, int on_device, int n, double 
     const float inv = (float)(1.0 / ((double)n * n * n));
     Bank K;
     if (lines && nfilt > 0) PP_CHECK(bank_start(ctx, ctx->d_k0.ptr, n, nbuff, n - nbuff, boxsize, Rf, nfilt, K));
+    // one read of delta_k gives a filter's spectrum and, with want_lapd and no
+    // line transform, the wsmooth = 3 spectrum sampled at the filter's new
+    // peaks; without the latter it is formed beside the filter before's peaks
+    const bool two = want_lapd && !lines;
+    auto window = [&](int f, WinJob *J) {
+        return window_job(ctx->d_k0.ptr, ctx->d_k1.ptr, wsmooth, &lay, two ? ctx->d_k2.ptr : nullptr, PP_WINDOW_K2GAUSS,
+                          n, boxsize, Rf[f], inv, J);
+    };
     for (int f = 0; f < nfilt; f++) {
         if (lines) PP_CHECK(bank_transform(ctx, K, Rf, f));
-        // one read of delta_k gives the filter's spectrum and, with want_lapd
-        // and no line transform, the wsmooth = 3 spectrum sampled at the
-        // filter's new peaks
-        PP_CHECK(launch_window2(ctx, ctx->d_k0.ptr, ctx->d_k1.ptr, wsmooth, &lay,
-                                want_lapd && !lines ? ctx->d_k2.ptr : nullptr, PP_WINDOW_K2GAUSS, n, boxsize, Rf[f],
-                                inv));
+        WinJob J;
+        if (f == 0 || two) {
+            PP_CHECK(window(f, &J));
+            PP_CHECK(launch_window(ctx, J));
+        }
+        const bool ahead = !two && f + 1 < nfilt;
+        if (ahead) PP_CHECK(window(f + 1, &J));
         void *ib[1] = {ctx->d_k1.ptr}, *ob[1] = {ctx->d_field_a.ptr};
         PP_FFT(rocfft_execute(lay.c2r, ib, ob, ctx->fftp->info));
         PP_CHECK(run_stencil(ctx, ctx->d_field_a.as<float>(), d_mask, g, fcrit[f], max_peaks_per_filter, f,
-                             o, d_counters, S, lines ? K.ranges + 2 * f : nullptr));
+                             o, d_counters, S, lines ? K.ranges + 2 * f : nullptr, ahead ? &J : nullptr));
         if (lines) {
             PP_CHECK(bank_sample(ctx, K, f, o, d_lapd));
         } else if (want_lapd) {
