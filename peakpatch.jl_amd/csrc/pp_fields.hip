@@ -8,13 +8,17 @@
 // displacements_2lpt (src/InitialConditions/LPT.jl:21-191);
 // _compute_laplacian (src/Pipeline.jl:35-51).
 //
-// Design: rocFFT for the transforms (the context's cached plans); every
-// k-space step is one pass over the half spectrum that evaluates its Float64
-// factor per mode and rounds the product into Float32 once, as the
-// reference's Float64 factor times its ComplexF32 array does.  The 1/n^3 of
-// the normalised inverse transforms is folded into that factor (an exact
-// power of two for power-of-two n).  The 2LPT source is accumulated in real
-// space in the reference's order, so only the diagonal potentials and the
+// Design: line transforms in LDS (pp_fft.h) where the mesh has them: the noise
+// is drawn in the x pass, the transfer functions sit between the forward and
+// the inverse transform of the z pass, several outputs share a pass, and the
+// 2LPT source is formed in the pass that brings its potentials to real space.
+// Other meshes (a prime factor above 7) go through rocFFT (the context's
+// cached plans) and one pass over the half spectrum per k-space step, which
+// evaluates its Float64 factor per mode and rounds the product into Float32
+// once, as the reference's Float64 factor times its ComplexF32 array does; the
+// 1/n^3 of the normalised inverse transforms is folded into that factor (an
+// exact power of two for power-of-two n), and the source is accumulated in
+// real space in the reference's order, so only the diagonal potentials and the
 // running sum are held at once.
 #include <cmath>
 #include <vector>

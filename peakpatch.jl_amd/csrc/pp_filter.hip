@@ -13,12 +13,14 @@
 //    into the same pass (a power of two for power-of-two n, so bit-identical
 //    to scaling after the transform).
 //  * stencil: the inner cube is linearised k-outer / j / i-inner, exactly the
-//    CPU loop order; pass 1 counts candidates per 256-cell block (wave ballot),
-//    an exclusive scan turns counts into offsets, pass 2 recomputes the
-//    predicate and writes each peak at offset + rank.  The output order is
-//    therefore the CPU order, deterministic, with no atomics.  The cap of
-//    max_peaks per filter (PeakFind.jl:70-72) drops the tail of that order and
-//    masks only the kept peaks, as the CPU early return does.
+//    CPU loop order; pass 1 tests the cells into a bit mask (wave ballots) and
+//    counts them by tile and plane, pass 2 writes each peak at the sum of the
+//    counts before it.  The output order is therefore the CPU order,
+//    deterministic, with no atomics.  The cap of max_peaks per filter
+//    (PeakFind.jl:70-72) drops the tail of that order and masks only the kept
+//    peaks, as the CPU early return does.
+//  * the k^2 field at the peaks: line transforms (pp_fft.h) as far as the
+//    peaks need them, on a second stream.
 #include <hipcub/hipcub.hpp>
 
 #include <cmath>
