@@ -75,7 +75,7 @@ class TileConfig:
 
 
 CONFIGS = {
-    # BASELINE configs[0..3]
+    # the benchmark's tiles, smallest first
     "c1": TileConfig("c1", 128, 75.0, 10, 1.5, 8.0, ilpt=1, ioutshear=0, z_out=0.0),
     "c2": TileConfig("c2", 256, 250.0, 20, 1.0, 15.0, ilpt=2, ioutshear=1, z_out=0.5),
     "c3": TileConfig("c3", 512, 600.0, 25, 1.0, 30.0, ilpt=2, ioutshear=1, ievol=1, z_max=4.6,
