@@ -214,6 +214,10 @@ __global__ void __launch_bounds__(256) k_residual_pad(float *__restrict__ R, Til
             double g1 = 0, g2 = 0;
 #pragma unroll
             for (int h = 0; h < 2; h++) {
+                if (x + h >= T.n) {  // odd n: the pair's second cell is padding
+                    out2[h] = 0.f;
+                    continue;
+                }
                 const int gx = wrap1(T.i0 + x + h, T.N);
                 const long long idx0 = gx + rowb;  // idx - 1
                 const long long pr = idx0 >> 1;
@@ -934,8 +938,7 @@ int pp_split_tile_fields(pp_ctx *ctx, const pp_coarse *c, int it, int jt, int kt
     T.k0 = (kt - 1) * c->nsub - G.nbuff;
     T.inv_b3 = (float)(1.0 / sqrt(pow((double)c->block, 3)));
     T.seed = G.seed;
-    // odd n: k_residual_pad's layout (pairs of cells) reaches one cell past the
-    // tile, so its fields are not those of the line transforms
+    // the line passes pair rows of even length
     if (n % 2 == 0 && line_supported(n) && G.M <= kLineCoarse) return split_tile_lines(ctx, c, T, f);
     const long long n3 = (long long)n * n * n;
     // 1. residual -> padded buffer R; base spectrum in place
