@@ -564,13 +564,14 @@ static int stencil_start(pp_ctx *ctx, const StencilGeom &g, long long *d_counter
 // only.  Its inverse transform (rocFFT: 1.46 ms at 512^3, after half of
 // k_window's 0.31 ms) is done on line transforms (pp_fft.h) instead, as far as
 // the peaks need it: the window goes into the z pass, planes and rows outside
-// the inner cube are not written, modes whose Gaussian is below 1e-12 are not
+// the inner cube are not written, modes whose window is zero in Float32 are not
 // read, and only the row pairs that hold a peak are transformed along x, from
 // where the peaks' values are taken without a field.  The passes run on the
 // side stream beside the next filters' rocFFT kernels, which leave most of
 // HBM's bandwidth free; only the last waits for its filter's stencil.
-// pp_smooth_field with wsmooth = 3 takes the same passes over the whole grid,
-// so both give the same bits.
+// pp_smooth_field with wsmooth = 3 takes the same passes over the whole grid
+// and every mode, so both give the same bits (the peaks' spectrum is finite: a
+// field with other modes has no peaks).
 struct BankGeo {
     int n, lo, hi;      // planes [lo, hi)
     int ylo, yhi;       // rows [ylo, yhi): the inner ones and their partners in row pairs
@@ -748,17 +749,28 @@ static int bank_join(pp_ctx *ctx)
     return PP_OK;
 }
 
+// The largest |i| on an axis at which k^2 exp(-(k R)^2 / 8), k = dk i, may still
+// be other than zero in Float32.  With u = (k R)^2 / 8 the window is
+// (8 / R^2) u exp(-u), which falls beyond u = 1 and rounds to zero from 2^-150
+// on: u - ln u > ln(8 / R^2) + 150 ln 2, solved by iteration, with a per cent
+// of the window to spare.
+static int window_reach(double dk, double R, int half)
+{
+    if (!(fabs(R) > 0.0)) return half;
+    const double L = log(8.0) - 2.0 * log(fabs(R)) + 150.0 * M_LN2;
+    double u = 1000.0;
+    for (int q = 0; q < 100; q++) u = std::max(1.0, L + log(u));
+    const double c = sqrt(8.0 * (u + 0.01)) / (dk * fabs(R));
+    return c < half ? (int)c + 1 : half;
+}
+
 // filter f's spectrum along z and y (needs no peaks)
-static int bank_transform(pp_ctx *ctx, Bank &K, const double *Rf, int f)
+static int bank_transform(pp_ctx *ctx, Bank &K, const double *Rf, int f, bool every_mode)
 {
     const SpecGeo &g = K.G.g;
     const int n = g.n, half = n / 2;
     K.B.gauss = K.tables + (size_t)f * (half + 1);
-    // exp(-(c dk R)^2 / 8) < 1e-12: with the growth of k^2 and of the number of
-    // modes out to there (30 and 10 times those at the window's edge) 3e-10 of
-    // the field, far below its Float32 rounding
-    const double c = sqrt(8.0 * 27.64) / fabs(K.dk * Rf[f]);
-    K.B.cut = c < half ? (int)c + 1 : half;
+    K.B.cut = every_mode ? half : window_reach(K.dk, Rf[f], half);
     K.B.plain = Rf[f] == 0.0;
     const int rows = std::min(n, 2 * K.B.cut + 1), bins = std::min(K.B.cut, g.nk - 1) + 1;
     if (K.B.hi <= K.B.lo) return PP_OK;
@@ -932,7 +944,7 @@ int pp_smooth_field(pp_ctx *ctx, const void *delta_k, float *out, int on_device,
     if (wsmooth == PP_WINDOW_K2GAUSS && line_supported(n)) {
         Bank K;
         PP_CHECK(bank_start(ctx, src, n, 0, n, boxsize, &Rf, 1, K));
-        PP_CHECK(bank_transform(ctx, K, &Rf, 0));
+        PP_CHECK(bank_transform(ctx, K, &Rf, 0, true));
         XArgs X{};
         X.top = K.B.cut;
         X.add(K.T, dst, 0, false, 1.f);
@@ -1049,7 +1061,7 @@ int pp_find_peaks(pp_ctx *ctx, const float *delta, int on_device, int n, double 
                           n, boxsize, Rf[f], inv, J);
     };
     for (int f = 0; f < nfilt; f++) {
-        if (lines) PP_CHECK(bank_transform(ctx, K, Rf, f));
+        if (lines) PP_CHECK(bank_transform(ctx, K, Rf, f, false));
         WinJob J;
         if (f == 0 || two) {
             PP_CHECK(window(f, &J));
