@@ -577,17 +577,18 @@ struct BankGeo {
     int ylo, yhi;       // rows [ylo, yhi): the inner ones and their partners in row pairs
     int cut;            // modes |i| > cut on any axis are left out
     int plain;          // radius 0: no window
-    float mult2, scale; // k^2 = mult2 |i|^2
-    const float *gauss; // exp(-(k Rf)^2 / 8) by index, n / 2 + 1
+    double mult2;       // k^2 = mult2 |i|^2
+    float scale;
+    const double *gauss; // exp(-(k Rf)^2 / 8) by index, n / 2 + 1
 };
 
-// exp(-(i dk R)^2 / 8) of every filter, Float64 rounded once
-__global__ void k_gauss_table(const double *__restrict__ Rf, int nfilt, int count, double dk, float *__restrict__ out)
+// exp(-(i dk R)^2 / 8) of every filter
+__global__ void k_gauss_table(const double *__restrict__ Rf, int nfilt, int count, double dk, double *__restrict__ out)
 {
     for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < nfilt * count; t += gridDim.x * blockDim.x) {
         const int f = t / count, i = t - f * count;
         const double x = (double)i * dk * Rf[f] / 2.0;
-        out[t] = (float)exp(-(x * x) / 2.0);
+        out[t] = exp(-(x * x) / 2.0);
     }
 }
 
@@ -615,7 +616,7 @@ __global__ void __launch_bounds__(1024) k_bank_z(SpecGeo g, LineFft P, ColGrid C
     const int fy = iy < (n + 1) / 2 ? iy : iy - n, ay = abs(fy), kx = min(t.kx, g.nk - 1), ixy = kx * kx + fy * fy;
     const ColAddr<M != kLineAny> at(lds, t.l, C.logl);
     const LineZ src(g, in, iy, t.kx);
-    const float gxy = B.gauss[kx] * B.gauss[ay] * B.scale;
+    const double gxy = B.gauss[kx] * B.gauss[ay] * B.mult2;
     float2 X[kLineEpt];
 #pragma unroll
     for (int q = 0; q < kLineEpt; q++) {
@@ -624,8 +625,9 @@ __global__ void __launch_bounds__(1024) k_bank_z(SpecGeo g, LineFft P, ColGrid C
         if (az <= B.cut) {
             const float2 v = *src.at(e);
             const int i2 = ixy + fz * fz;
-            const float f = i2 == 0 || B.plain ? B.scale : gxy * B.gauss[az] * ((float)i2 * B.mult2);  // k = 0: unscaled
-            X[q] = make_float2(v.x * f, v.y * f);
+            // the window in Float64, rounded once, as window_value's; k = 0: none
+            const float f = i2 == 0 || B.plain ? 1.f : (float)(gxy * B.gauss[az] * (double)i2);
+            X[q] = make_float2(v.x * f * B.scale, v.y * f * B.scale);
         }
     }
     line_run<1, M, false, false>(at, P, t.jj, X);
@@ -700,7 +702,7 @@ struct Bank {
     GridPlan G;
     BankGeo B{};
     float2 *R = nullptr, *T = nullptr;
-    float *tables = nullptr;
+    double *tables = nullptr;
     long long *ranges = nullptr;
     double dk = 0;
 };
@@ -718,17 +720,17 @@ static int bank_start(pp_ctx *ctx, const void *spec, int n, int lo, int hi, doub
     PP_CHECK(ctx->d_spec.grow(2 * arr * sizeof(float2)));
     K.R = ctx->d_spec.as<float2>();
     K.T = K.R + arr;
-    PP_CHECK(ctx->d_misc.grow((size_t)nfilt * (3 * sizeof(double) + count * sizeof(float))));
+    PP_CHECK(ctx->d_misc.grow((size_t)nfilt * (3 + count) * sizeof(double)));
     double *d_Rf = ctx->d_misc.as<double>();
     K.ranges = (long long *)(d_Rf + nfilt);
-    K.tables = (float *)(K.ranges + 2 * nfilt);
+    K.tables = (double *)(K.ranges + 2 * nfilt);
     K.dk = 2.0 * M_PI / boxsize;
     K.B.n = n;
     K.B.lo = lo;
     K.B.hi = hi;
     K.B.ylo = std::max(0, lo - 1);
     K.B.yhi = std::min(n, hi + 1);
-    K.B.mult2 = (float)(K.dk * K.dk);
+    K.B.mult2 = K.dk * K.dk;
     K.B.scale = (float)(1.0 / ((double)n * n * n));
     PP_HIP(hipEventRecord(ctx->ev_bank, ctx->stream));
     PP_HIP(hipStreamWaitEvent(ctx->side, ctx->ev_bank, 0));
