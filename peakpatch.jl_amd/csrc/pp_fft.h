@@ -23,8 +23,10 @@
 //   butterflies read them.  Vector instructions are the second bound beside
 //   HBM (a radix-8 stage takes 14 per element, a pass has room for about a
 //   hundred), so addresses advance by scalar strides and the kernels' own
-//   factors are Float32 wherever their error stays below the transform's.
+//   Float64 factors are pairs of Float32 numbers (Two), wave numbers whole.
 #pragma once
+
+#include <cmath>
 
 #include "pp_common.h"
 
@@ -108,6 +110,36 @@ __device__ __forceinline__ float2 fsub(float2 a, float2 b)
 __device__ __forceinline__ float2 faxpy(float s, float2 b, float2 a)
 {
     return make_float2(__builtin_fmaf(s, b.x, a.x), __builtin_fmaf(s, b.y, a.y));
+}
+// A Float64 factor as the sum of two Float32 numbers, right to 2^-48: a complex
+// value times it takes two instructions a component more than Float32's two and
+// is rounded once, as the product in Float64 is (which takes conversions both
+// ways besides).
+struct Two {
+    float h, l;
+};
+inline Two two(double v)
+{
+    const float h = (float)v;
+    return Two{h, std::isfinite(h) ? (float)(v - (double)h) : 0.f};
+}
+__device__ __forceinline__ float2 ftimes(Two f, float2 x)
+{
+    PP_NO_CONTRACT
+    return make_float2(__builtin_fmaf(f.h, x.x, f.l * x.x), __builtin_fmaf(f.h, x.y, f.l * x.y));
+}
+// times a whole number
+__device__ __forceinline__ Two ftimes(Two f, float k)
+{
+    PP_NO_CONTRACT
+    const float p = f.h * k;
+    return Two{p, __builtin_fmaf(f.l, k, __builtin_fmaf(f.h, k, -p))};
+}
+// 1 / d of a whole number 0 < d < 2^24
+__device__ __forceinline__ Two finverse(float d)
+{
+    const float r = __builtin_amdgcn_rcpf(d), h = __builtin_fmaf(__builtin_fmaf(-d, r, 1.f), r, r);
+    return Two{h, __builtin_fmaf(-d, h, 1.f) * h};
 }
 // times -i (forward) or +i (inverse)
 template <int SIGN> __device__ __forceinline__ float2 rot(float2 a)

@@ -7,14 +7,15 @@
 
 namespace pp {
 
-// Transfer of one output of the z pass, times scale: X; X k^2 (with k and the
-// product as _compute_laplacian forms them, or from the integer wave
-// numbers); X / k^2, kz X / k^2, kz^2 X / k^2 (0 at k = 0).  |k|^2 is mult^2
-// times an integer, exact in Float32, so these factors carry one or two
-// Float32 roundings, and the amplitude comes from a table over that integer.  The
-// factors of kx and ky that a displacement or potential takes besides are
-// constant along z and follow in the y and x passes, so three z-inverses
-// serve the nine spectra of both orders.
+// Transfer of one output of the z pass, i the whole wave numbers (k = mult i):
+// X; X k^2 with k and the product as _compute_laplacian forms them, in Float32;
+// X |i|^2; X / |i|^2, iz X / |i|^2, iz^2 X / |i|^2 (0 at k = 0).  The factors of
+// ix and iy that a displacement or potential takes besides are constant along z
+// and follow in the y and x passes, so three z-inverses serve the nine spectra
+// of both orders.  Wave numbers and their squares are exact in Float32, the
+// amplitude (from a table over |i|^2), 1 / |i|^2 and the field's constant (mult
+// and the normalisation, in the x pass) are pairs (Two): a pass rounds a mode
+// once, as a Float64 factor does, and no unit of length overflows on the way.
 enum ZKind { Z_X = 0, Z_K2F, Z_K2, Z_INV, Z_INV_Z, Z_INV_ZZ };
 
 struct ZArgs {
@@ -24,17 +25,8 @@ struct ZArgs {
         float2 *p;
         int kind, nyq;  // nyq: the Nyquist planes are zeroed
     } out[7];
-    float mult, scale;  // k of an index
-    float inv, k2;      // scale / mult^2, scale mult^2
-    const float *amp;   // amplitude by integer |k|^2, or null
-    float dkf;
-    void set(double m, double sc)
-    {
-        mult = (float)m;
-        scale = (float)sc;
-        inv = (float)(sc / (m * m));
-        k2 = (float)(sc * (m * m));
-    }
+    const Two *amp;    // amplitude by |i|^2, or null
+    float dkf, scale;  // Z_K2F's k of an index and normalisation
     void add(float2 *p, int kind, int nyq) { out[nout++] = Out{p, kind, nyq}; }
 };
 
@@ -42,9 +34,8 @@ struct YArgs {
     int narr;
     struct Arr {
         const float2 *in;
-        float2 *out[3];  // times 1, ky, ky^2; null: not wanted
+        float2 *out[3];  // times 1, iy, iy^2; null: not wanted
     } arr[7];
-    float mult;
     void add(const float2 *in, float2 *o0, float2 *o1, float2 *o2) { arr[narr++] = Arr{in, {o0, o1, o2}}; }
 };
 
@@ -53,21 +44,20 @@ struct XArgs {
     struct Op {
         const float2 *in;
         float *out;
-        int pow;    // power of kx
-        bool imag;  // the factor is i f kx^pow, else f kx^pow
-        float f;
+        int pow;    // power of ix
+        bool imag;  // the factor is i f ix^pow, else f ix^pow
+        Two f;
     } op[5];
-    float mult;
     int top = 1 << 30;  // bins above it are zero and not read
-    void add(const float2 *in, float *out, int pow, bool imag, float f) { op[nop++] = Op{in, out, pow, imag, f}; }
+    void add(const float2 *in, float *out, int pow, bool imag, double f) { op[nop++] = Op{in, out, pow, imag, two(f)}; }
 };
 
 struct SrcArgs {
     const float2 *in[6];  // potentials 11 22 33 12 13 23
     int pow[6];
     const float *delta;
+    Two f;  // the potentials' constant
     float2 *out;
-    float mult;
 };
 
 // The rows of a P(k) table (device, npk log k then npk log P) and, for rows
@@ -81,18 +71,18 @@ inline size_t pk_log_doubles(int npk) { return 4 * (size_t)npk + 2; }
 // there (on the host they took as long as a 128^3 tile's kernels).
 int pk_log_device(pp_ctx *ctx, const pp_pk_table *pk, double *buf, PkLog *out);
 
-// sqrt(P(k) dk^3 n^3) at k^2 = mult^2 i for i = 0 .. 3 imax^2 (0 at i = 0), in
-// Float64 rounded once.  A mode's amplitude in the kernels was the bigger part
-// of their Float64 work: the table holds a few hundred thousand values for
-// the up to 10^9 modes of a grid.
+// sqrt(P(k) dk^3 n^3) / n^3 at k^2 = mult^2 i for i = 0 .. 3 imax^2 (0 at i = 0).
+// A mode's amplitude in the kernels was the bigger part of their Float64 work:
+// the table holds a few hundred thousand values for the up to 10^9 modes of a
+// grid.
 inline long long amp_count(int imax) { return 3ll * imax * imax + 1; }
-int amp_table(pp_ctx *ctx, const PkLog &T, double mult, double dk3, double n3, long long count, float *out);
+int amp_table(pp_ctx *ctx, const PkLog &T, double mult, double dk3, double n3, long long count, Two *out);
 
-// the line of a row pair from an x-spectrum times f kx^pow or i f kx^pow; bins
+// the line of a row pair from an x-spectrum times f ix^pow or i f ix^pow; bins
 // above top are zero
 __device__ __forceinline__ void load_row_pair(const RowAddr &at, const LineFft &P, const SpecGeo &g,
                                               const float2 *in, long long r, bool two, int jj, int pow, bool imag,
-                                              float f, float mult, int top)
+                                              Two f, int top)
 {
     const long long z = r / g.n, z2 = (r + 1) / g.n;
     const float2 *a = in + g.row((int)z, (int)(r - z * g.n)), *b = in + g.row((int)z2, (int)(r + 1 - z2 * g.n));
@@ -107,10 +97,10 @@ __device__ __forceinline__ void load_row_pair(const RowAddr &at, const LineFft &
     for (int q = 0; q < kRowBins; q++) {
         const int k = jj + q * P.tj;
         if (k >= g.nk) break;
-        const float kx = (float)k * mult, c = pow == 0 ? f : pow == 1 ? f * kx : f * kx * kx;
-        const float2 u = va[q], v = vb[q];
-        join_rows(at, g.n, k, imag ? make_float2(-c * u.y, c * u.x) : make_float2(c * u.x, c * u.y),
-                  imag ? make_float2(-c * v.y, c * v.x) : make_float2(c * v.x, c * v.y));
+        const float ix = (float)k;
+        const Two c = pow == 0 ? f : ftimes(f, pow == 1 ? ix : ix * ix);
+        const float2 u = ftimes(c, va[q]), v = ftimes(c, vb[q]);
+        join_rows(at, g.n, k, imag ? make_float2(-u.y, u.x) : u, imag ? make_float2(-v.y, v.x) : v);
     }
 }
 
@@ -131,7 +121,6 @@ int rows_inv(const GridPlan &G, const XArgs &X);
 int rows_src(const GridPlan &G, const SrcArgs &S);
 void src_inputs(SrcArgs &S, const float2 *a, const float2 *a1, const float2 *a2, const float2 *b, const float2 *b1,
                 const float2 *c);
-int second_order(const GridPlan &G, float2 *const s[3], double mult, double scale,
-                 float *const out[3]);
+int second_order(const GridPlan &G, float2 *const s[3], double mult, double scale, float *const out[3]);
 
 }  // namespace pp

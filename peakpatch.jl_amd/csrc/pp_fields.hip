@@ -222,16 +222,12 @@ __global__ void __launch_bounds__(1024) k_cols_z(SpecGeo g, LineFft P, ColGrid C
     line_run<-1, M, false, false>(at, P, t.jj, X);
     const int kx = min(t.kx, g.nk - 1), fy = iy < (n + 1) / 2 ? iy : iy - n, ixy = kx * kx + fy * fy;
     const bool nyq_xy = kx == g.nk - 1 || iy == half;
-    float ik[kLineEpt];  // scale / k^2
+    Two ik[kLineEpt];  // 1 / |i|^2
 #pragma unroll
     for (int q = 0; q < kLineEpt; q++) {
         const int e = min(t.jj + q * P.tj, n - 1), fz = e < (n + 1) / 2 ? e : e - n, i2 = ixy + fz * fz;
-        if (A.amp) {
-            const float a = A.amp[i2];
-            X[q] = make_float2(X[q].x * a, X[q].y * a);
-        }
-        const float d = (float)i2, r = __builtin_amdgcn_rcpf(d);
-        ik[q] = i2 == 0 ? 0.f : A.inv * __builtin_fmaf(__builtin_fmaf(-d, r, 1.f), r, r);
+        if (A.amp) X[q] = ftimes(A.amp[i2], X[q]);
+        ik[q] = i2 == 0 ? Two{0.f, 0.f} : finverse((float)i2);
     }
     for (int o = 0; o < A.nout; o++) {
         const int kind = A.out[o].kind, nyq = A.out[o].nyq;
@@ -241,22 +237,23 @@ __global__ void __launch_bounds__(1024) k_cols_z(SpecGeo g, LineFft P, ColGrid C
 #pragma unroll
         for (int q = 0; q < kLineEpt; q++) {
             const int e = jj + q * P.tj, fz = e < (n + 1) / 2 ? e : e - n;
-            float f;
             if (kind == Z_X) {
-                f = A.scale;
+                x[q] = X[q];
             } else if (kind == Z_K2F) {
-                // k and the product in Float32, both normalisations (_compute_laplacian)
+                // k and the product in Float32 (_compute_laplacian); the spectrum
+                // holds the first of the two normalisations
                 const float fx = (float)kx * A.dkf, fyf = (float)(iy <= half ? iy : iy - n) * A.dkf,
                             fzf = (float)(e <= half ? e : e - n) * A.dkf;
-                f = (fx * fx + fyf * fyf + fzf * fzf) * A.scale * A.scale;
+                const float f = (fx * fx + fyf * fyf + fzf * fzf) * A.scale;
+                x[q] = make_float2(X[q].x * f, X[q].y * f);
             } else if (kind == Z_K2) {
-                f = A.k2 * (float)(ixy + fz * fz);
+                const float f = (float)(ixy + fz * fz);
+                x[q] = make_float2(X[q].x * f, X[q].y * f);
             } else {
-                const float kz = (float)fz * A.mult;
-                f = kind == Z_INV ? ik[q] : kind == Z_INV_Z ? ik[q] * kz : ik[q] * kz * kz;
+                const float iz = (float)fz;
+                x[q] = ftimes(kind == Z_INV ? ik[q] : ftimes(ik[q], kind == Z_INV_Z ? iz : iz * iz), X[q]);
             }
-            if (nyq && (nyq_xy || e == half)) f = 0.f;
-            x[q] = make_float2(X[q].x * f, X[q].y * f);
+            if (nyq && (nyq_xy || e == half)) x[q] = make_float2(0.f, 0.f);
         }
         line_run<1, M, false, false>(at, P, jj, x);
         line_store(P, jj, x, LineZ(g, A.out[o].p, iy, t.kx));
@@ -264,13 +261,16 @@ __global__ void __launch_bounds__(1024) k_cols_z(SpecGeo g, LineFft P, ColGrid C
 }
 
 __global__ void __launch_bounds__(256) k_amp_table(PkLog T, double mult2, double dk3, double n3, long long count,
-                                                   float *__restrict__ out)
+                                                   Two *__restrict__ out)
 {
 #pragma clang fp contract(off)
     const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
     if (i >= count) return;
     const double k2 = (double)i * mult2;
-    out[i] = i == 0 ? 0.f : (float)sqrt(pk_eval(T.lk, T.lp, T.np, sqrt(k2), T.even[0], T.even[1]) * dk3 * n3);
+    const double a =
+        i == 0 ? 0.0 : sqrt(pk_eval(T.lk, T.lp, T.np, sqrt(k2), T.even[0], T.even[1]) * dk3 * n3) * (1.0 / n3);
+    const float h = (float)a;
+    out[i] = Two{h, isfinite(h) ? (float)(a - (double)h) : 0.f};
 }
 
 // logarithms of k and P (one block) and whether log k is evenly spaced, to
@@ -296,7 +296,7 @@ __global__ void __launch_bounds__(1024) k_pk_log(const double *__restrict__ k, c
     }
 }
 
-// y-inverse of the arrays of Y, each times the powers of ky asked for:
+// y-inverse of the arrays of Y, each times the powers of iy asked for:
 // z planes, grid y the arrays; an output may be its input
 template <int M>
 __global__ void __launch_bounds__(1024, M == kLineReg ? 8 : 4) k_cols_y_inv(SpecGeo g, LineFft P, ColGrid C, YArgs Y)
@@ -310,7 +310,7 @@ __global__ void __launch_bounds__(1024, M == kLineReg ? 8 : 4) k_cols_y_inv(Spec
     float2 X[kLineEpt];
     line_load(P, t.jj, X, LineY(g, R.in, t.plane, 0, 1, t.kx));
     for (int o = 0; o < 3; o++) {
-        float2 *w = R.out[o];  // ky^o
+        float2 *w = R.out[o];  // iy^o
         if (!w) continue;
         int jj = t.jj;
         asm volatile("" : "+v"(jj));
@@ -318,7 +318,7 @@ __global__ void __launch_bounds__(1024, M == kLineReg ? 8 : 4) k_cols_y_inv(Spec
 #pragma unroll
         for (int q = 0; q < kLineEpt; q++) {
             const int e = jj + q * P.tj;
-            const float ky = (float)(e < (n + 1) / 2 ? e : e - n) * Y.mult, f = o == 0 ? 1.f : o == 1 ? ky : ky * ky;
+            const float iy = (float)(e < (n + 1) / 2 ? e : e - n), f = o == 0 ? 1.f : o == 1 ? iy : iy * iy;
             x[q] = make_float2(X[q].x * f, X[q].y * f);
         }
         line_run<1, M, false, false>(at, P, jj, x);
@@ -336,7 +336,7 @@ __global__ void __launch_bounds__(512) k_rows_inv(SpecGeo g, LineFft P, XArgs X)
     const RowAddr at(lds + line * row_pitch(n));
     const bool two = r + 1 < rows;
     const XArgs::Op &O = X.op[blockIdx.y];
-    if (r < rows) load_row_pair(at, P, g, O.in, r, two, jj, O.pow, O.imag, O.f, X.mult, X.top);
+    if (r < rows) load_row_pair(at, P, g, O.in, r, two, jj, O.pow, O.imag, O.f, X.top);
     __syncthreads();
     float2 x[kLineEpt];
     line_run<1, M, true, false>(at, P, jj, x);
@@ -382,7 +382,7 @@ __global__ void __launch_bounds__(512) k_rows_src(SpecGeo g, LineFft P, SrcArgs 
         int j2 = jj;
         asm volatile("" : "+v"(j2));
         __syncthreads();
-        if (live) load_row_pair(at, P, g, S.in[v], r, two, j2, S.pow[v], false, 1.f, S.mult, g.nk);
+        if (live) load_row_pair(at, P, g, S.in[v], r, two, j2, S.pow[v], false, S.f, g.nk);
         __syncthreads();
         float2 x[kLineEpt];
         line_run<1, M, true, false>(at, P, j2, x);
@@ -480,7 +480,7 @@ int rows_src(const GridPlan &G, const SrcArgs &S)
     return PP_OK;
 }
 
-int amp_table(pp_ctx *ctx, const PkLog &T, double mult, double dk3, double n3, long long count, float *out)
+int amp_table(pp_ctx *ctx, const PkLog &T, double mult, double dk3, double n3, long long count, Two *out)
 {
     hipLaunchKernelGGL(k_amp_table, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, ctx->stream, T, mult * mult,
                        dk3, n3, count, out);
@@ -501,8 +501,8 @@ int pk_log_device(pp_ctx *ctx, const pp_pk_table *pk, double *buf, PkLog *out)
     return PP_OK;
 }
 
-// The six potentials' arrays: y-inverses of X / k^2, kz X / k^2, kz^2 X / k^2
-// times powers of ky, in the order 11 22 33 12 13 23 with their powers of kx
+// The six potentials' arrays: y-inverses of X / |i|^2, iz X / |i|^2, iz^2 X / |i|^2
+// times powers of iy, in the order 11 22 33 12 13 23 with their powers of ix
 void src_inputs(SrcArgs &S, const float2 *a, const float2 *a1, const float2 *a2, const float2 *b, const float2 *b1,
                 const float2 *c)
 {
@@ -521,20 +521,17 @@ int second_order(const GridPlan &G, float2 *const s[3], double mult, double scal
     PP_CHECK(cols_y_fwd(G, s[0]));
     ZArgs Z{};
     Z.in = s[0];
-    Z.set(mult, scale);
     Z.add(s[0], Z_INV, 1);
     Z.add(s[1], Z_INV_Z, 1);
     PP_CHECK(cols_z(G, Z));
     YArgs Y{};
-    Y.mult = (float)mult;
     Y.add(s[0], s[0], s[2], nullptr);
     Y.add(s[1], s[1], nullptr, nullptr);
     PP_CHECK(cols_y_inv(G, Y));
     XArgs X{};
-    X.mult = (float)mult;
-    X.add(s[0], out[0], 1, true, -1.f);
-    X.add(s[2], out[1], 0, true, -1.f);
-    X.add(s[1], out[2], 0, true, -1.f);
+    X.add(s[0], out[0], 1, true, -scale / mult);
+    X.add(s[2], out[1], 0, true, -scale / mult);
+    X.add(s[1], out[2], 0, true, -scale / mult);
     return rows_inv(G, X);
 }
 
@@ -547,7 +544,7 @@ static int make_tile_lines(pp_ctx *ctx, int n, double boxsize, uint64_t seed, co
     GridPlan G;
     PP_CHECK(grid_plan(ctx, n, &G));
     const size_t arr = G.g.size(n);  // complex values of one array
-    // delta / source, A', B', ky A', L, and with 2LPT A, B, C, ky A, ky^2 A, ky B
+    // delta / source, A', B', iy A', L, and with 2LPT A, B, C, iy A, iy^2 A, iy B
     const int narr = 4 + (f->lapd ? 1 : 0) + (lpt2 ? 6 : 0);
     PP_CHECK(ctx->d_spec.grow(arr * narr * sizeof(float2)));
     float2 *s[11];
@@ -557,17 +554,17 @@ static int make_tile_lines(pp_ctx *ctx, int n, double boxsize, uint64_t seed, co
     PP_CHECK(cols_y_fwd(G, s[0]));
     const double dk = 2.0 * M_PI / boxsize, mult = ((double)n * dk) / (double)n, n3 = (double)n * n * n;
     const long long count = amp_count(n / 2);
-    PP_CHECK(ctx->d_misc.grow(pk_log_doubles(pk->npk) * sizeof(double) + count * sizeof(float)));
+    PP_CHECK(ctx->d_misc.grow(pk_log_doubles(pk->npk) * sizeof(double) + count * sizeof(Two)));
     double *d_pk = ctx->d_misc.as<double>();
-    float *amp = (float *)(d_pk + pk_log_doubles(pk->npk));
+    Two *amp = (Two *)(d_pk + pk_log_doubles(pk->npk));
     PkLog T;
     PP_CHECK(pk_log_device(ctx, pk, d_pk, &T));
     PP_CHECK(amp_table(ctx, T, mult, dk * dk * dk, n3, count, amp));
     ZArgs Z{};
     Z.in = s[0];
-    Z.set(mult, 1.0 / n3);
     Z.amp = amp;
     Z.dkf = (float)dk;
+    Z.scale = (float)(1.0 / n3);
     Z.add(s[0], Z_X, 0);
     Z.add(s[1], Z_INV, 1);
     Z.add(s[2], Z_INV_Z, 1);
@@ -579,7 +576,6 @@ static int make_tile_lines(pp_ctx *ctx, int n, double boxsize, uint64_t seed, co
     }
     PP_CHECK(cols_z(G, Z));
     YArgs Y{};
-    Y.mult = (float)mult;
     Y.add(s[0], s[0], nullptr, nullptr);
     Y.add(s[1], s[1], s[3], nullptr);
     Y.add(s[2], s[2], nullptr, nullptr);
@@ -591,16 +587,15 @@ static int make_tile_lines(pp_ctx *ctx, int n, double boxsize, uint64_t seed, co
     }
     PP_CHECK(cols_y_inv(G, Y));
     XArgs X{};
-    X.mult = (float)mult;
-    X.add(s[0], f->delta, 0, false, 1.f);
-    X.add(s[1], f->etax, 1, true, 1.f);
-    X.add(s[3], f->etay, 0, true, 1.f);
-    X.add(s[2], f->etaz, 0, true, 1.f);
-    if (L) X.add(L, f->lapd, 0, false, 1.f);
+    X.add(s[0], f->delta, 0, false, 1.0);
+    X.add(s[1], f->etax, 1, true, 1.0 / mult);
+    X.add(s[3], f->etay, 0, true, 1.0 / mult);
+    X.add(s[2], f->etaz, 0, true, 1.0 / mult);
+    if (L) X.add(L, f->lapd, 0, false, 1.0);
     PP_CHECK(rows_inv(G, X));
     if (lpt2) {
         SrcArgs S{};
-        S.mult = (float)mult;
+        S.f = two(1.0);
         S.out = s[0];
         src_inputs(S, W[0], W[3], W[4], W[1], W[5], W[2]);
         PP_CHECK(rows_src(G, S));

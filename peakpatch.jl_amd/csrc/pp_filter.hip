@@ -686,7 +686,7 @@ __global__ void __launch_bounds__(512) k_bank_rows(SpecGeo g, LineFft P, BankGeo
     const bool has = lo < hi && row(lo) <= r + 1;
     if (!__syncthreads_or(has)) return;
     const RowAddr at(lds + line * row_pitch(n));
-    if (has) load_row_pair(at, P, g, s, r, true, jj, 0, false, 1.f, 0.f, B.cut);
+    if (has) load_row_pair(at, P, g, s, r, true, jj, 0, false, Two{1.f, 0.f}, B.cut);
     __syncthreads();
     float2 x[kLineEpt];
     line_run<1, M, true, true>(at, P, jj, x);
@@ -949,7 +949,7 @@ int pp_smooth_field(pp_ctx *ctx, const void *delta_k, float *out, int on_device,
         PP_CHECK(bank_transform(ctx, K, &Rf, 0, true));
         XArgs X{};
         X.top = K.B.cut;
-        X.add(K.T, dst, 0, false, 1.f);
+        X.add(K.T, dst, 0, false, 1.0);
         PP_CHECK(rows_inv(K.G, X));
         PP_CHECK(bank_join(ctx));
         if (!on_device) PP_HIP(hipMemcpyAsync(out, dst, rb, hipMemcpyDeviceToHost, ctx->stream));

@@ -337,9 +337,10 @@ __global__ void __launch_bounds__(256) k_src_sub(float *__restrict__ src, const 
 //   y[j], j < n = IFFT_n(X[2 m])[j] + w^-j IFFT_n(X[2 m + 1])[j].
 // A spectrum holds n z planes (real space along z) of 2 n rows.  The z pass
 // transforms forward, applies the transfer and transforms back while a
-// column is in LDS, so the (2 n)^3 spectrum never exists in memory; ky A goes to
+// column is in LDS, so the (2 n)^3 spectrum never exists in memory; iy A goes to
 // the upper half of A's rows, which the cut leaves free.  delta, psi_x, psi_y
-// and psi_z come from the three arrays X, X / k^2 and kz X / k^2.  Traffic at
+// and psi_z come from the three arrays X, X / |i|^2 and iz X / |i|^2 (whole wave
+// numbers i and factors in pairs, as in pp_fields.h).  Traffic at
 // n = 512: 30 GB in place of 170.
 constexpr int kLineCoarse = 512;  // coarse cells a side whose rows fit LDS beside a line
 struct PadGeo {
@@ -458,9 +459,8 @@ __global__ void __launch_bounds__(1024) k_pad_cols_y_fwd(PadGeo G, LineFft P, Co
 
 struct PadZ {
     const float2 *in;
-    float2 *out[3];    // X, X / k^2, kz X / k^2
-    const float *amp;  // by integer |k|^2
-    float mult, scale, inv;
+    float2 *out[3];  // X, X / |i|^2, iz X / |i|^2
+    const Two *amp;  // by |i|^2
 };
 
 // z-forward, transfer, z-inverse
@@ -483,8 +483,7 @@ __global__ void __launch_bounds__(1024) k_pad_cols_z(PadGeo G, LineFft P, ColGri
 #pragma unroll
             for (int q = 0; q < kLineEpt; q++) {
                 const int e = 2 * min(jj0 + q * P.tj, n - 1) + h, fz = e < n ? e : e - 2 * n;
-                const float a = A.amp[ixy + fz * fz];
-                X[h][q] = make_float2(X[h][q].x * a, X[h][q].y * a);
+                X[h][q] = ftimes(A.amp[ixy + fz * fz], X[h][q]);
             }
         }
     }
@@ -498,13 +497,12 @@ __global__ void __launch_bounds__(1024) k_pad_cols_z(PadGeo G, LineFft P, ColGri
 #pragma unroll
             for (int q = 0; q < kLineEpt; q++) {
                 const int e = jj + q * P.tj, k = 2 * e + h, fz = k < n ? k : k - 2 * n, i2 = ixy + fz * fz;
-                float f = A.scale;
+                x[q] = X[h][q];
                 if (o > 0) {
-                    const float d = (float)i2, r = __builtin_amdgcn_rcpf(d);
-                    f = i2 == 0 ? 0.f : A.inv * __builtin_fmaf(__builtin_fmaf(-d, r, 1.f), r, r);
-                    if (o == 2) f = f * ((float)fz * A.mult);
+                    Two f = i2 == 0 ? Two{0.f, 0.f} : finverse((float)i2);
+                    if (o == 2) f = ftimes(f, (float)fz);
+                    x[q] = ftimes(f, x[q]);
                 }
-                x[q] = make_float2(X[h][q].x * f, X[h][q].y * f);
             }
             pad_inverse<M, false>(at, P, jj, x, y, h);
         }
@@ -514,8 +512,7 @@ __global__ void __launch_bounds__(1024) k_pad_cols_z(PadGeo G, LineFft P, ColGri
 
 struct PadY {
     float2 *s[3];
-    int nvar[3];  // 1, or 2: times ky too, to rows n .. 2 n - 1
-    float mult;
+    int nvar[3];  // 1, or 2: times iy too, to rows n .. 2 n - 1
 };
 
 // y-inverse, in place: 2 n rows in, n (per power of ky) out
@@ -542,7 +539,7 @@ __global__ void __launch_bounds__(1024) k_pad_cols_y_inv(PadGeo G, LineFft P, Co
 #pragma unroll
             for (int q = 0; q < kLineEpt; q++) {
                 const int e = jj + q * P.tj, k = 2 * e + h;
-                const float f = o == 0 ? 1.f : (float)(k < n ? k : k - 2 * n) * A.mult;
+                const float f = o == 0 ? 1.f : (float)(k < n ? k : k - 2 * n);
                 x[q] = make_float2(X[h][q].x * f, X[h][q].y * f);
             }
             pad_inverse<M, false>(at, P, jj, x, y, h);
@@ -556,11 +553,11 @@ struct PadX {
     struct Op {
         const float2 *in;
         int row0;       // first row of the plane
-        int imag, pow;  // factor 1, i or i kx
+        int imag, pow;  // factor f, i f or i f ix
+        Two f;
         const float *coarse;
         float *out;
     } op[4];
-    float mult;
 };
 
 // Coarse row of tile row (y, z): the sum over the 4 x 4 taps along y and z,
@@ -621,10 +618,9 @@ __global__ void __launch_bounds__(512) k_pad_rows_inv(PadGeo G, LineFft P, TileG
             for (int q = 0; q < kRowBins; q++) {
                 const int m = j2 + q * P.tj, k = 2 * m + h;
                 if (k > n) break;
-                const float c = O.pow ? (float)k * A.mult : 1.f;
-                const float2 p = va[q], s = vb[q];
-                const float2 f1 = O.imag ? make_float2(-c * p.y, c * p.x) : make_float2(c * p.x, c * p.y),
-                             f2 = O.imag ? make_float2(-c * s.y, c * s.x) : make_float2(c * s.x, c * s.y);
+                const Two c = O.pow ? ftimes(O.f, (float)k) : O.f;
+                const float2 p = ftimes(c, va[q]), s = ftimes(c, vb[q]);
+                const float2 f1 = O.imag ? make_float2(-p.y, p.x) : p, f2 = O.imag ? make_float2(-s.y, s.x) : s;
                 const int mc = h ? n - 1 - m : (m == 0 ? 0 : n - m);
                 if (k == 0 || k == n) {  // real bins (mc = m)
                     at(m) = make_float2(f1.x, f2.x);
@@ -678,7 +674,7 @@ static int split_tile_lines(pp_ctx *ctx, const pp_coarse *c, const TileGeo &T, p
     // Stream ordered and returned when the tile's fields are written, so a
     // context does not keep them between tiles
     const size_t pad = Q.g.size(n), arr = D.g.size(n);
-    const int narr = 1 + (f->lapd ? 1 : 0) + (lpt2 ? 6 : 0);  // source or delta, then A .. ky B; L last
+    const int narr = 1 + (f->lapd ? 1 : 0) + (lpt2 ? 6 : 0);  // source or delta, then A .. iy B; L last
     const size_t need = std::max(3 * pad, (size_t)narr * arr) * sizeof(float2);
     void *arena = nullptr;
     hipError_t ea = hipMallocAsync(&arena, need, ctx->stream);
@@ -692,8 +688,8 @@ static int split_tile_lines(pp_ctx *ctx, const pp_coarse *c, const TileGeo &T, p
         ~Release() { (void)hipFreeAsync(p, s); }
     } release{ctx->stream, arena};
     const long long count = amp_count(n);
-    PP_CHECK(ctx->d_misc.grow(count * sizeof(float)));
-    float *amp = ctx->d_misc.as<float>();
+    PP_CHECK(ctx->d_misc.grow(count * sizeof(Two)));
+    Two *amp = ctx->d_misc.as<Two>();
     const int n2 = 2 * n;
     const double dx = (double)G.nmesh * G.alatt / n, dki = 2.0 * M_PI / (n2 * dx), mi = ((double)n2 * dki) / (double)n2;
     const double pad3 = (double)n2 * n2 * n2;
@@ -707,17 +703,16 @@ static int split_tile_lines(pp_ctx *ctx, const pp_coarse *c, const TileGeo &T, p
     PP_LINE_LAUNCH(D.row, k_pad_rows_noise, rgrid, rblock, D.rs.lds, ctx->stream, Q, D.row, T, c->noise.as<float>(),
                    s[0]);
     PP_LINE_LAUNCH(D.col, k_pad_cols_y_fwd, gy, cblock, D.cs.lds, ctx->stream, Q, D.col, cy, s[0]);
-    PadZ Z{s[0], {s[0], s[1], s[2]}, amp, (float)mi, (float)(1.0 / pad3), (float)(1.0 / pad3 / (mi * mi))};
+    PadZ Z{s[0], {s[0], s[1], s[2]}, amp};
     PP_LINE_LAUNCH(D.col, k_pad_cols_z, gz, cblock, D.cs.lds, ctx->stream, Q, D.col, cz, Z);
-    PadY Y{{s[0], s[1], s[2]}, {1, 2, 1}, (float)mi};
+    PadY Y{{s[0], s[1], s[2]}, {1, 2, 1}};
     PP_LINE_LAUNCH(D.col, k_pad_cols_y_inv, dim3(gy.x, 3), cblock, D.cs.lds, ctx->stream, Q, D.col, cy, Y);
     PadX X{};
-    X.mult = (float)mi;
     const float *psi = c->psi.as<float>();
-    X.op[0] = PadX::Op{s[0], 0, 0, 0, c->delta.as<float>(), f->delta};
-    X.op[1] = PadX::Op{s[1], 0, 1, 1, psi, f->etax};
-    X.op[2] = PadX::Op{s[1], n, 1, 0, psi + M3, f->etay};
-    X.op[3] = PadX::Op{s[2], 0, 1, 0, psi + 2 * M3, f->etaz};
+    X.op[0] = PadX::Op{s[0], 0, 0, 0, two(1.0), c->delta.as<float>(), f->delta};
+    X.op[1] = PadX::Op{s[1], 0, 1, 1, two(1.0 / mi), psi, f->etax};
+    X.op[2] = PadX::Op{s[1], n, 1, 0, two(1.0 / mi), psi + M3, f->etay};
+    X.op[3] = PadX::Op{s[2], 0, 1, 0, two(1.0 / mi), psi + 2 * M3, f->etaz};
     const size_t rlds = D.rs.lds + (size_t)D.rs.nl * 2 * M * sizeof(float);
     PP_LINE_LAUNCH(D.row, k_pad_rows_inv, dim3(rgrid.x, 4), rblock, rlds, ctx->stream, Q, D.row, T, X);
     if (!lpt2 && !f->lapd) {
@@ -733,9 +728,7 @@ static int split_tile_lines(pp_ctx *ctx, const pp_coarse *c, const TileGeo &T, p
     PP_CHECK(cols_y_fwd(D, t[0]));
     ZArgs Z2{};
     Z2.in = t[0];
-    Z2.set(mt, 1.0 / (double)n3);
     YArgs Y2{};
-    Y2.mult = (float)mt;
     if (L) {
         Z2.add(L, Z_K2, 1);
         Y2.add(L, L, nullptr, nullptr);
@@ -752,15 +745,14 @@ static int split_tile_lines(pp_ctx *ctx, const pp_coarse *c, const TileGeo &T, p
     PP_CHECK(cols_y_inv(D, Y2));
     if (L) {
         XArgs X2{};
-        X2.mult = (float)mt;
-        X2.add(L, f->lapd, 0, false, 1.f);
+        X2.add(L, f->lapd, 0, false, mt * mt / (double)n3);
         PP_CHECK(rows_inv(D, X2));
     }
     if (lpt2) {
         float2 *src = t[6];
         SrcArgs S{};
         S.delta = f->delta;
-        S.mult = (float)mt;
+        S.f = two(1.0 / (double)n3);
         S.out = src;
         src_inputs(S, t[0], t[3], t[4], t[1], t[5], t[2]);
         PP_CHECK(rows_src(D, S));
