@@ -141,6 +141,12 @@ __device__ __forceinline__ Two finverse(float d)
     const float r = __builtin_amdgcn_rcpf(d), h = __builtin_fmaf(__builtin_fmaf(-d, r, 1.f), r, r);
     return Two{h, __builtin_fmaf(-d, h, 1.f) * h};
 }
+// a + s b with a constant s to 48 bits
+__device__ __forceinline__ float2 faxpy2(double s, float2 b, float2 a)
+{
+    const float h = (float)s, l = (float)(s - (double)h);
+    return faxpy(h, b, l == 0.f ? a : faxpy(l, b, a));
+}
 // times -i (forward) or +i (inverse)
 template <int SIGN> __device__ __forceinline__ float2 rot(float2 a)
 {
@@ -175,35 +181,43 @@ template <int R, int SIGN> __device__ __forceinline__ void butterfly(float2 *v)
         v[3] = faxpy(h, o3, e[3]);
         v[7] = faxpy(-h, o3, e[3]);
     } else {
-        // odd prime: the sums and differences of conjugate inputs
-        constexpr float C3[1] = {-0.5f}, S3[1] = {0.86602540378443865f};
-        constexpr float C5[2] = {0.30901699437494742f, -0.80901699437494742f},
-                        S5[2] = {0.95105651629515357f, 0.58778525229247313f};
-        constexpr float C7[3] = {0.62348980185873353f, -0.22252093395631440f, -0.90096886790241913f},
-                        S7[3] = {0.78183148246802981f, 0.97492791218182361f, 0.43388373911755812f};
-        const float *C = R == 3 ? C3 : R == 5 ? C5 : C7, *S = R == 3 ? S3 : R == 5 ? S5 : S7;
+        // odd prime: the sums p and differences m of conjugate inputs; outputs
+        // k and R - k are x0 + sum C p plus or minus i sum S m, as one chain of
+        // fma each.  The constants are pairs: in Float32 alone they are half of
+        // what such a stage is off (3e-8 of 5e-8), and the same in every mode.
+        constexpr double C3[1] = {-0.5}, S3[1] = {0.86602540378443864676};
+        constexpr double C5[2] = {0.30901699437494742410, -0.80901699437494742410},
+                         S5[2] = {0.95105651629515357212, 0.58778525229247312917};
+        constexpr double C7[3] = {0.62348980185873353053, -0.22252093395631440429, -0.90096886790241912624},
+                         S7[3] = {0.78183148246802980871, 0.97492791218182360702, 0.43388373911755812048};
+        const double *C = R == 3 ? C3 : R == 5 ? C5 : C7, *S = R == 3 ? S3 : R == 5 ? S5 : S7;
         constexpr int H = R / 2;
         float2 p[H], m[H], x0 = v[0], sum = v[0];
 #pragma unroll
         for (int q = 0; q < H; q++) {
             p[q] = fadd(v[q + 1], v[R - 1 - q]);
-            m[q] = fsub(v[q + 1], v[R - 1 - q]);
+            m[q] = rot<SIGN>(fsub(v[q + 1], v[R - 1 - q]));
             sum = fadd(sum, p[q]);
         }
         v[0] = sum;
 #pragma unroll
         for (int k = 1; k <= H; k++) {
-            float2 a = x0, b = make_float2(0.f, 0.f);
+            float2 a = x0;
 #pragma unroll
             for (int q = 0; q < H; q++) {
                 const int t = (k * (q + 1)) % R, u = t <= H ? t : R - t;
-                const float s = t <= H ? S[u - 1] : -S[u - 1];
-                a = faxpy(C[u - 1], p[q], a);
-                b = faxpy(s, m[q], b);
+                a = faxpy2(C[u - 1], p[q], a);
             }
-            b = rot<SIGN>(b);
-            v[k] = fadd(a, b);
-            v[R - k] = fsub(a, b);
+            float2 b = a;
+#pragma unroll
+            for (int q = H - 1; q >= 0; q--) {
+                const int t = (k * (q + 1)) % R, u = t <= H ? t : R - t;
+                const double s = t <= H ? S[u - 1] : -S[u - 1];
+                a = faxpy2(s, m[q], a);
+                b = faxpy2(-s, m[q], b);
+            }
+            v[k] = a;
+            v[R - k] = b;
         }
     }
 }
