@@ -645,7 +645,8 @@ __global__ void __launch_bounds__(512) k_pad_rows_inv(PadGeo G, LineFft P, TileG
         // the base cell and fraction of (g + 1/2) / b + 1/2 (cr_coord), in integers
         const unsigned num = 2u * (unsigned)wrap1(T.i0 + e, T.N) + 1u + (unsigned)T.b, i = num / b2;
         float w[4];
-        cr_weights((float)(num - i * b2) * ib2, w);
+        const float rem = (float)(num - i * b2), t0 = rem * ib2;
+        cr_weights(__builtin_fmaf(__builtin_fmaf(-t0, (float)b2, rem), ib2, t0), w);  // rem / b2, rounded once
         float c1 = 0.f, c2 = 0.f;
 #pragma unroll
         for (int t = 0; t < 4; t++) {
