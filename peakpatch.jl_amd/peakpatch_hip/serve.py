@@ -87,11 +87,14 @@ def tile_config(req: TileRequest, template: TileConfig = SERVE_TEMPLATE) -> Tile
 
 
 def footprint_bytes(n: int) -> int:
-    """Device bytes one tile holds at its peak: the 9 Float32 fields, their
-    spectrum and the synthesis temporaries (~24 B/cell), filter scratch and
-    mask (~9 B/cell), the transposed delta, profiles and results
-    (~30 B/cell at ~1.5e-2 peaks/cell), plus fixed tables and plans."""
-    return int(n) ** 3 * 100 + (256 << 20)
+    """Device bytes a slot holds at the peak of a periodic tile: the 8 Float32
+    fields and the mask (33 B/cell), the synthesis' 11 padded spectra (44 to
+    50), which the context keeps, the filter bank's spectra, field and mask
+    (13), the gathered fields' interleaved copies (40), profiles, walk table
+    and results (30 to 50 at ~1.5e-2 peaks/cell), the caller's copies of peaks
+    and records, plus fixed tables and plans.  Measured, two tiles in a row:
+    176, 181, 188, 196, 179 and 178 B/cell at 128, 192, 256, 320, 512, 768."""
+    return int(n) ** 3 * 200 + (256 << 20)
 
 
 def poisson_stream(ntiles: int, rate: float, seed: int = 0, nmesh=SERVE_NMESH, weights=None,

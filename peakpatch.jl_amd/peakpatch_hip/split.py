@@ -131,12 +131,20 @@ def make_split_tile(ctx, coarse: CoarseField, it: int, jt: int, kt: int, ilpt: i
 
 
 def footprint_bytes(n: int) -> int:
-    """Device bytes a split tile of nmesh n holds at its peak: two padded
-    (2n)^3 spectra (64 n^3 B each), the eight output fields (32 n^3), the
-    tile-periodic spectra and real scratch (16 n^3), then the peak finder's
-    and the shell analysis' working set (~60 n^3 at ~1.5e-2 peaks per cell),
-    plus fixed tables and plans."""
-    return int(n) ** 3 * 172 + (512 << 20)
+    """Device bytes a slot holds at the peak of a split tile of nmesh n: what
+    it keeps from tile to tile (fields, filter bank, gathered fields, profiles,
+    walk table, results: 140 to 160 n^3 B at ~1.5e-2 peaks per cell) and the
+    convolution's working set, three spectra of half the padded grid (48 to
+    53 n^3) on line transforms, two whole ones (128 n^3) on rocFFT (odd n or a
+    prime factor above 7), plus fixed tables and plans.  Measured, two tiles in
+    a row: 181, 190, 189, 209, 203 and 208 B/cell at 128, 192, 256, 320, 512,
+    768; on rocFFT up to 253."""
+    m = int(n)
+    for p in (2, 3, 5, 7):
+        while m % p == 0:
+            m //= p
+    lines = m == 1 and n % 2 == 0 and 16 <= n <= 1024
+    return int(n) ** 3 * (220 if lines else 290) + (512 << 20)
 
 
 def tiles(geom: SplitGeom):
