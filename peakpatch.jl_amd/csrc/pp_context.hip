@@ -27,6 +27,7 @@ int DevBuf::grow(size_t need)
     size_t b = need < 256 ? 256 : need;
     hipError_t e = hipMalloc(&ptr, b);
     if (e != hipSuccess) {
+        (void)hipGetLastError();  // reported here, not again by the next launch's check
         ptr = nullptr;
         set_error("hipMalloc(%zu bytes) failed: %s", b, hipGetErrorString(e));
         return e == hipErrorOutOfMemory ? PP_ERR_OOM : PP_ERR_HIP;
