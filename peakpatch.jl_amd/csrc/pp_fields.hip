@@ -631,7 +631,10 @@ extern "C" int pp_make_tile_fields(pp_ctx *ctx, int n, double boxsize, uint64_t 
         PP_ARG(q == 0 || pk->k[q] > pk->k[q - 1], "P(k) table k not increasing at row %d", q);
     }
     PP_CHECK(ensure_device(ctx));
-    if (lines_for(n)) return make_tile_lines(ctx, n, boxsize, seed, pk, f);
+    if (lines_for(n)) {
+        const int rc = make_tile_lines(ctx, n, boxsize, seed, pk, f);
+        if (rc != PP_ERR_OOM) return rc;  // 44 to 50 B a cell are not there: rocFFT's route takes 24
+    }
     PP_CHECK(fft_prepare(ctx, n));
     const int nk = n / 2 + 1;
     const long long total = (long long)nk * n * n;

@@ -936,7 +936,6 @@ int pp_smooth_field(pp_ctx *ctx, const void *delta_k, float *out, int on_device,
     PP_CHECK(ensure_device(ctx));
     PP_CHECK(fft_prepare(ctx, n));
     size_t rb = (size_t)n * n * n * sizeof(float), cb = (size_t)(n / 2 + 1) * n * n * sizeof(float2);
-    PP_CHECK(ctx->d_k1.grow(cb));
     const void *src = delta_k;
     if (!on_device) {
         PP_CHECK(ctx->d_k0.grow(cb));
@@ -962,6 +961,7 @@ int pp_smooth_field(pp_ctx *ctx, const void *delta_k, float *out, int on_device,
         PP_HIP(hipStreamSynchronize(ctx->stream));
         return PP_OK;
     }
+    PP_CHECK(ctx->d_k1.grow(cb));
     PP_CHECK(launch_window(ctx, src, ctx->d_k1.ptr, n, boxsize, Rf, wsmooth, inv));
     void *ib[1] = {ctx->d_k1.ptr}, *ob[1] = {dst};
     PP_FFT(rocfft_execute(ctx->fftp->c2r, ib, ob, ctx->fftp->info));

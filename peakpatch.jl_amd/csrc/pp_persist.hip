@@ -1687,7 +1687,9 @@ static int run_persistent_impl(pp_ctx *ctx, GatherFields G, ShellRun &S, PostCon
             PP_HIP(hipStreamSynchronize(ctx->stream));
             nrec_w = last[0] + last[1];
         }
-        PP_CHECK(ctx->d_walk.grow((size_t)std::max<int64_t>(nrec_w, 1) * sizeof(WalkRec)));
+        const int rc = ctx->d_walk.grow((size_t)std::max<int64_t>(nrec_w, 1) * sizeof(WalkRec));
+        if (rc == PP_ERR_OOM) return PP_OK;  // the posts form the steps themselves
+        PP_CHECK(rc);
         d_wtab = ctx->d_walk.as<WalkRec>();
         // classes: consecutive runs of the lane-post order (m descending)
         WalkClasses K{};

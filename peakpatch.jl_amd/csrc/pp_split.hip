@@ -680,6 +680,7 @@ static int split_tile_lines(pp_ctx *ctx, const pp_coarse *c, const TileGeo &T, p
     void *arena = nullptr;
     hipError_t ea = hipMallocAsync(&arena, need, ctx->stream);
     if (ea != hipSuccess) {
+        (void)hipGetLastError();
         set_error("hipMallocAsync of %zu B: %s", need, hipGetErrorString(ea));
         return ea == hipErrorOutOfMemory ? PP_ERR_OOM : PP_ERR_HIP;
     }

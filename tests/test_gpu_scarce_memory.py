@@ -1,0 +1,92 @@
+"""Calls with little device memory left: what is faster with more work space
+goes on without it.  The rest of the memory is held by a tensor that no kernel
+touches; each call's own needs are well within what is left."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from peakpatch_hip import SHELL_PERSISTENT, Context, collapse
+from test_gpu_shell import FIELDS, bump_field
+
+pytestmark = pytest.mark.gpu
+
+
+def _hold(leave):
+    import torch
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    return torch.empty(torch.cuda.mem_get_info()[0] - leave, dtype=torch.uint8, device="cuda")
+
+
+def test_tile_fields():
+    """512^3: 6.4 GB of spectra on the line transforms, 3.2 GB on rocFFT."""
+    import torch
+    from peakpatch_hip import _lib as L
+    from peakpatch_hip import synth
+    n, box = 512, 600.0
+    k, P = synth.pk_table()
+    tab = L.PkTable(len(k), k.ctypes.data, P.ctypes.data)
+    f = [torch.empty((n, n, n), device="cuda") for _ in range(8)]
+    out = L.TileFields(*(a.data_ptr() for a in f))
+
+    def run(ctx):
+        ctx._call(lambda: ctx.lib.pp_make_tile_fields(ctx.h, n, box, 5, C.byref(tab), C.byref(out)), True)
+        return [a.cpu().numpy() for a in f]
+
+    with Context(0) as ctx:
+        want = run(ctx)
+    with Context(0) as ctx:
+        ctx.rfft(np.zeros((n, n, n), np.float32))  # rocFFT's plans
+        held = _hold(4500 << 20)
+        try:
+            got = run(ctx)
+        finally:
+            del held
+            torch.cuda.empty_cache()
+    for a, b in zip(got, want):
+        assert np.abs(a - b).max() <= 2e-5 * np.abs(b).max()
+
+
+def test_shell_analysis():
+    """240 k peaks, whose walk table takes 0.5 GB or more."""
+    import torch
+    n, p, times = 64, 400, 600
+    d, eta, eta2, lap = bump_field(n, 5)
+    ct = collapse.sinusoidal_table()
+    rng = np.random.default_rng(2)
+    c = np.argsort(d[6:-6, 6:-6, 6:-6].ravel())[-4 * p::4]
+    k, j, i = (q + 6 for q in np.unravel_index(c, (n - 12,) * 3))
+    Rf = rng.uniform(5.0, 6.0, p)
+    pk = dict(i=i.astype(np.int32), j=j.astype(np.int32), k=k.astype(np.int32), Rf=Rf,
+              ir2min=np.floor((1.75 * Rf) ** 2).astype(np.int64), ZZon=rng.uniform(0.3, 0.8, p))
+    pk = {q: np.tile(v, times) for q, v in pk.items()}
+
+    def run(ctx):
+        r = ctx.analyse_peaks(d, eta, pk["i"], pk["j"], pk["k"], pk["Rf"], pk["ir2min"], pk["ZZon"], 0.7, 1.0,
+                              eta2=eta2, lapd=lap, nbuff=2, kernel=SHELL_PERSISTENT)
+        return r
+
+    with Context(0) as ctx:
+        ctx.upload_collapse_table(ct.table, *ct.bounds)
+        ctx.build_shell_tables(14)
+        default = ctx.tunables()
+        want = run(ctx)
+        assert int(want["nshells"].astype(np.int64).sum()) * 64 > 600 << 20
+        ctx.lib.pp_ctx_release_scratch(ctx.h)
+        ctx.tunables(post_width=2)  # the same buffers without a walk table
+        run(ctx)
+        ctx.tunables(**default)
+        held = _hold(400 << 20)
+        try:
+            got = run(ctx)
+        finally:
+            del held
+            torch.cuda.empty_cache()
+    ok = want["status"] == 0
+    assert ok.sum() > 1000
+    np.testing.assert_array_equal(got["status"], want["status"])
+    np.testing.assert_array_equal(got["nshells"], want["nshells"])
+    for q in FIELDS:
+        a, b = got[q][ok], want[q][ok]
+        assert np.all(np.abs(a - b) <= 1e-11 * np.abs(b).max()), q
