@@ -16,15 +16,15 @@ def test_a_refused_call_leaves_no_error_behind():
         want = ctx.rfft(d)
         ctx.fill_noise(8, 1)
         ctx.synchronize()
+        big = torch.zeros((640, 640, 640), device="cuda")
         torch.cuda.synchronize()
         torch.cuda.empty_cache()
         held = torch.empty(torch.cuda.mem_get_info()[0] - (400 << 20), dtype=torch.uint8, device="cuda")
         try:
-            big = np.broadcast_to(np.float32(0), (512, 512, 512))
-            with pytest.raises(PPError, match="OOM"):
-                ctx.find_peaks_field(np.ascontiguousarray(big), np.zeros(big.shape, np.int8), 2, 1.0)
+            with pytest.raises(PPError, match="OOM"):  # three arrays of 1 GB
+                ctx.find_peaks(big, 640.0, [2.0], [1.0], nbuff=2)
             ctx.fill_noise(8, 1)
             np.testing.assert_array_equal(ctx.rfft(d), want)
         finally:
-            del held
+            del held, big
             torch.cuda.empty_cache()
