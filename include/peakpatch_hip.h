@@ -300,15 +300,21 @@ int pp_autotune_shell(pp_ctx *ctx, const pp_fields *fields, const pp_peak_batch 
  *       are gathered cell by cell, floor(64 / m) per wave; 0 disables that
  *       path; at most 64),
  *   [1] shells per LDS chunk of the wave gather (8..1024),
- *   [2] shell count above which a peak's Float64 post runs on a whole wave,
+ *   [2] shell count above which a peak's Float64 post runs on a whole wave, or
+ *       PP_TUNE_AUTO (a new context's): none, unless the batch is too small,
  *   [3] cap on resident gather waves per CU,
- *   [4] lanes per peak of the Float64 post below [2] (1, 2, 4, 8 or 16),
+ *   [4] lanes per peak of the Float64 post below [2] (1, 2, 4, 8 or 16), or
+ *       PP_TUNE_AUTO (a new context's): 1, or as many as fill idle lanes of a
+ *       small batch,
  *   [5] with one lane per peak: virialisation walks longer than this many
  *       shells are re-run one wave per peak (0: no limit).
  * set (may be NULL): new values, entries <= 0 keep the current one except
  * [0] and [5], where 0 is a value and < 0 keeps; get (may be NULL): the
  * values in force.  They change speed only: results do not depend on them
- * beyond the last bits of the Float64 sums. */
+ * beyond the last bits of the Float64 sums.  Under PP_TUNE_AUTO those bits
+ * follow the number of peaks in the batch; with [2] and [4] set only Sbar,
+ * Sbar2 and d2F do, whose waves per peak always follow it. */
+#define PP_TUNE_AUTO (1 << 30)
 #define PP_NTUNABLES 6
 int pp_shell_tunables(pp_ctx *ctx, const int32_t *set, int32_t *get);
 

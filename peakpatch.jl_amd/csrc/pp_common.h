@@ -153,12 +153,12 @@ struct pp_ctx {
     // finalised shells (several peaks per wave), shells per LDS chunk of the
     // wave gather, the shell count above which a peak's Float64 post runs on
     // a whole wave, the cap on gather waves per CU, and the lanes per peak of
-    // the post below that count
+    // the post below that count (1, 2, 4, 8, 16)
     int tiny_m = 16;
     int chunk_shells = 64;
-    int coop_m = 1 << 20;
+    int coop_m = PP_TUNE_AUTO;
     int gather_waves_cu = 16;
-    int post_width = 1;  // lanes per peak of the post below coop_m (1, 4, 8, 16)
+    int post_width = PP_TUNE_AUTO;
     int lane_walk = 0;   // lane post: walks longer than this go to the wave post (0: no limit)
     // events: [0,1] whole call, [2..13] persistent-form stage boundaries
     static constexpr int NEV = 15;

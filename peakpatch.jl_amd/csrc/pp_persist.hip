@@ -1493,12 +1493,14 @@ static int run_persistent_impl(pp_ctx *ctx, GatherFields G, ShellRun &S, PostCon
     // One lane per peak wins at every batch measured once the walk table feeds
     // it (wave post for m > 64 against none, whole call: 1.95 M peaks of a
     // 512^3 tile 21.6 -> 15.5 ms, 180 k of 256^3 4.55 -> 3.36, 9 k large ones
-    // 5.44 -> 4.24, 2 k of 128^3 2.08 -> 2.03), so coop_m starts above every m.
-    // A class too small for the table (cross_order below) would leave its
-    // largest peaks to single lanes: those go to the wave post.
+    // 5.44 -> 4.24, 2 k of 128^3 2.08 -> 2.03), so coop_m left alone is above
+    // every m.  A class too small for the table (cross_order below) would leave
+    // its largest peaks to single lanes: those go to the wave post then.
+    const bool auto_width = ctx->post_width == PP_TUNE_AUTO;
+    int width = auto_width ? 1 : std::max(ctx->post_width, 1);
     int coop_m = std::max(ctx->coop_m, 1);
-    if (ctx->post_width <= 1 && small_lo - std::min(small_lo, cnt_gt(coop_m)) <= kLaneTableMin)
-        coop_m = std::min(coop_m, 64);
+    if (coop_m == PP_TUNE_AUTO && width == 1 && small_lo - std::min(small_lo, cnt_gt(coop_m)) <= kLaneTableMin)
+        coop_m = 64;
     const int64_t coop_end = std::min(small_lo, cnt_gt(coop_m));
     // waves per peak in the gather and the finish pass
     int waves = 8;
@@ -1650,7 +1652,7 @@ static int run_persistent_impl(pp_ctx *ctx, GatherFields G, ShellRun &S, PostCon
     for (int x = small_m + 1; x <= cmax && x < nb; x++) wrec_max += (int64_t)hist[x] * x;
     auto cross_order = [&]() -> int {
         const int64_t nl = cross_hi - cross_lo;
-        if (ctx->post_width > 1 || nl <= kLaneTableMin) return PP_OK;
+        if (nl <= kLaneTableMin) return PP_OK;
         // crossings and offsets apart from the records, whose number is only
         // bounded here
         PP_CHECK(ctx->d_cross.grow(al((size_t)nl * 8) * 2));
@@ -1835,10 +1837,9 @@ static int run_persistent_impl(pp_ctx *ctx, GatherFields G, ShellRun &S, PostCon
     // 5. posts: the wave post runs on the side stream (before the small
     // peaks' work), beside the lane post on the main stream
     PP_HIP(hipEventRecord(ctx->ev[5], ctx->stream));
-    if (ctx->post_width <= 1) PP_CHECK(walk_table());
+    PP_CHECK(walk_table());
     // one lane per peak, or groups of lanes as far as that only fills idle SIMDs
-    int width = std::max(ctx->post_width, 1);
-    if (d_wtab && ctx->lane_walk == 0)
+    if (auto_width && d_wtab && ctx->lane_walk == 0)
         while (width < kGroupPost && (small_lo - coop_end) * width * 2 <= (int64_t)ctx->num_cu * kGroupPostLanesCU) width *= 2;
     if (width == 1) {
         PP_CHECK(post_lane(coop_end, small_lo, false));

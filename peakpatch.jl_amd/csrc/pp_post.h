@@ -416,8 +416,9 @@ __device__ __forceinline__ int tab_crossing(const PV &P)
 }
 
 // Ebar of a walk step: the peak's walk-table record for mp when it was formed
-// on the same band (identical to kernel_strain's, which computed it), else
-// kernel_strain itself.  The wave post has no table.
+// on the same band (kernel_strain's on one lane: the same bits for W = 1, a
+// sum grouped otherwise for the rest), else kernel_strain itself.  The wave
+// post has no table.
 template <int W, class PV>
 __device__ __forceinline__ Strain walk_strain(const PV &P, const PostConst &C, int mp, int mlow, int mupp)
 {

@@ -160,12 +160,14 @@ class Context:
     def synchronize(self):
         L.check(self.lib.pp_ctx_synchronize(self.h))
 
+    TUNE_AUTO = 1 << 30
     TUNABLES = ("small_m", "chunk_shells", "coop_m", "gather_waves_cu", "post_width", "lane_walk")
 
     def tunables(self, **kw):
         """Get (and with keywords, set) the persistent form's launch
         parameters: small_m, chunk_shells, coop_m, gather_waves_cu, post_width,
-        lane_walk."""
+        lane_walk.  A new context's coop_m and post_width are TUNE_AUTO, which
+        fits them to each batch; values that were set hold for every batch."""
         unknown = set(kw) - set(self.TUNABLES)
         if unknown:
             raise ValueError(f"unknown tunables {sorted(unknown)}")
