@@ -437,7 +437,10 @@ int pp_pack_halos(pp_ctx *ctx, const pp_results *res, const pp_halo_inputs *in, 
  * r_new = ((4/3 pi r^3 - dV) / (4/3 pi))^(1/3), halos left without volume
  * removed).  keep[i] = 1 for the halos of the merged catalogue, whose RTHL
  * becomes new_rthl[i] (0 for removed halos); *nkept counts them.  keep and
- * new_rthl are device arrays when on_device, else host. */
+ * new_rthl are device arrays when on_device, else host.  A halo with a NaN
+ * coordinate or radius is kept as it is and neither excludes nor overlaps
+ * another; infinite ones, and 2^31 overlapping pairs or more, are refused
+ * (PP_ERR_ARG, keep and new_rthl untouched). */
 int pp_merge_halos(pp_ctx *ctx, int64_t n, const float *x, const float *y, const float *z, const float *rthl,
                    int on_device, int8_t *keep, float *new_rthl, int64_t *nkept);
 

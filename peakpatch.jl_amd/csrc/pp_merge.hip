@@ -349,13 +349,16 @@ __global__ void __launch_bounds__(256, 6) k_pairs(MergeCells C, MergeGeo G, doub
 }
 
 // reduced radii: deficit = caps as the larger member + caps as the smaller
+// (nothing for a number of pairs that is refused)
 __global__ void __launch_bounds__(256) k_finalize(MergeCells C, const int32_t *__restrict__ state,
+                                                  const unsigned long long *__restrict__ npair,
                                                   const double *__restrict__ caps,
                                                   const unsigned long long *__restrict__ frac,
                                                   int8_t *__restrict__ keep, float *__restrict__ new_r,
                                                   unsigned long long *__restrict__ nkept)
 {
 #pragma clang fp contract(off)
+    if (*npair >> 31) return;
     unsigned long long kept = 0;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < C.n; i += (int64_t)gridDim.x * 256) {
         const int32_t o = C.id[i];
@@ -571,16 +574,17 @@ extern "C" int pp_merge_halos(pp_ctx *ctx, int64_t n, const float *x, const floa
     // pass 2: caps of overlapping survivors, then the radii they leave
     hipLaunchKernelGGL(k_pairs, dim3(grid_n(ctx, n * kPairLanes)), dim3(256), 0, s, C, G, caps, frac, d_num);
     hipLaunchKernelGGL(k_finalize, dim3(std::min(grid_n(ctx, n), ctx->num_cu * 4)), dim3(256), 0, s, C, (const int32_t *)state,
-                       (const double *)caps, (const unsigned long long *)frac, d_keep, d_nr, d_num + 1);
+                       (const unsigned long long *)d_num, (const double *)caps, (const unsigned long long *)frac, d_keep, d_nr, d_num + 1);
     PP_HIP(hipGetLastError());
-    if (!on_device) {
-        PP_HIP(hipMemcpyAsync(keep, d_keep, n, hipMemcpyDeviceToHost, s));
-        PP_HIP(hipMemcpyAsync(new_rthl, d_nr, n * 4, hipMemcpyDeviceToHost, s));
-    }
     unsigned long long num[2];
     PP_HIP(hipMemcpyAsync(num, d_num, sizeof(num), hipMemcpyDeviceToHost, s));
     PP_HIP(hipStreamSynchronize(s));
     PP_ARG(num[0] < (1ull << 31), "too many overlapping pairs (%llu)", num[0]);
+    if (!on_device) {
+        PP_HIP(hipMemcpyAsync(keep, d_keep, n, hipMemcpyDeviceToHost, s));
+        PP_HIP(hipMemcpyAsync(new_rthl, d_nr, n * 4, hipMemcpyDeviceToHost, s));
+        PP_HIP(hipStreamSynchronize(s));
+    }
     *nkept = (int64_t)num[1];
     return PP_OK;
 }
