@@ -33,19 +33,20 @@ __device__ __forceinline__ uint64_t rotl64(uint64_t x, int r)
 }
 
 // -2 ln(x / 2^53) for a whole x in [1, 2^53].  x = 2^e m with m in
-// [1/sqrt 2, sqrt 2), ln m = 2 atanh(s), s = (m - 1) / (m + 1): the series in
-// s^2 as its polynomial through seven Chebyshev nodes on [0, (3 - 2 sqrt 2)^2]
-// (5e-18 of the whole); the quotient by the hardware's reciprocal, one Newton
-// step and the remainder.
+// [sqrt(1/2), sqrt 2): a fraction 1.f from sqrt 2 on (by its leading 20 bits) is
+// halved.  ln m = 2 atanh(s), s = (m - 1) / (m + 1): the series in s^2 as its
+// polynomial through seven Chebyshev nodes on [0, (3 - 2 sqrt 2)^2] (5e-18 of
+// the whole); the quotient by the hardware's reciprocal, one Newton step and
+// the remainder.
 __device__ __forceinline__ double noise_neg2log(double x)
 {
     constexpr double A[7] = {0.33333333333333348,  0.19999999999949722,  0.14285714313001635, 0.11111105565129939,
                              0.090914447278374735, 0.076658553091053863, 0.073082927124443114};
     const uint64_t bits = (uint64_t)__double_as_longlong(x);
-    const uint32_t hi = (uint32_t)(bits >> 32) + (0x3ff00000u - 0x3fe6a09eu);  // the exponent steps at sqrt 2
-    const int n = 53 + 1023 - (int)(hi >> 20);
-    const double m =
-        __longlong_as_double((long long)((uint64_t)((hi & 0xfffffu) + 0x3fe6a09eu) << 32 | (uint32_t)bits));
+    const uint32_t hi = (uint32_t)(bits >> 32), frac = hi & 0xfffffu;
+    const uint32_t over = frac >= 434334u ? 1u : 0u;  // (sqrt 2 - 1) 2^20 = 434334.4
+    const int n = 53 + 1023 - (int)(hi >> 20) - (int)over;
+    const double m = __longlong_as_double((long long)((uint64_t)(frac + ((1023u - over) << 20)) << 32 | (uint32_t)bits));
     const double f = m - 1.0, d = m + 1.0;
     double r = __builtin_amdgcn_rcp(d);
     r = fma(fma(-d, r, 1.0), r, r);
