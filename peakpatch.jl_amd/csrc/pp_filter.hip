@@ -21,8 +21,6 @@
 //    peaks, as the CPU early return does.
 //  * the k^2 field at the peaks: line transforms (pp_fft.h) as far as the
 //    peaks need them, on a second stream.
-#include <hipcub/hipcub.hpp>
-
 #include <cmath>
 #include <mutex>
 
@@ -805,13 +803,16 @@ static int bank_sample(pp_ctx *ctx, Bank &K, int f, const PeakOut &o, float *d_l
 }
 
 // ------------------------------------------- peak finding without allocation
-// pp_find_peaks_field_noalloc keeps its counters and the stencil's bit mask,
-// offsets and scan storage in `scratch`, a file-scope array every device the
+// pp_find_peaks_field_noalloc keeps its counters and the stencil's bit mask and
+// counts in `scratch`, a file-scope array every device the
 // library runs on holds until the process ends.  Host code never passes the
 // array's name to a kernel: it passes the device address hipGetSymbolAddress
 // gives for the current device, taken once per device when a context is
 // created there (noalloc_scratch_init).
 static __device__ __align__(256) unsigned char scratch[PP_NOALLOC_SCRATCH_BYTES];
+// Row words of the inner cube it is for, the bound callers know (12 bytes a
+// word and 17 KB of sums; 64 words less than fit).
+constexpr long long kNoallocWords = 8387136;
 
 constexpr int kMaxDevices = 64;
 static std::mutex g_scratch_mu;
@@ -1113,16 +1114,10 @@ int pp_find_peaks_field_noalloc(pp_ctx *ctx, const float *delta_s, int8_t *mask,
     PP_CHECK(ensure_device(ctx));
     if (max_peaks <= 0) max_peaks = 2000000;
     const StencilGeom g = stencil_geom(n1, n2, n3, nbuff);
-    // the bound callers know: 12 bytes a word and the storage of a scan over
-    // them, more than the bit mask and the runs now take
-    hipcub::CountingInputIterator<int> it(0);
-    size_t tmp = 0;
-    PP_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, it, (int *)nullptr, (int)std::max(1ll, g.nwords)));
-    const size_t need = std::max(align256((size_t)g.nwords * 8) + align256((size_t)g.nwords * 4) + align256(tmp),
-                                 stencil_scratch_bytes(g)) + 256;
-    PP_ARG(need <= (size_t)PP_NOALLOC_SCRATCH_BYTES,
-           "inner cube %dx%dx%d needs %zu B of scratch, more than the %zu B this entry point has; use "
-           "pp_find_peaks_field", g.in1, g.in2, g.in3, need, (size_t)PP_NOALLOC_SCRATCH_BYTES);
+    const size_t need = stencil_scratch_bytes(g) + 256;
+    PP_ARG(g.nwords <= kNoallocWords && need <= (size_t)PP_NOALLOC_SCRATCH_BYTES,
+           "inner cube %dx%dx%d has %lld words, more than the %lld the scratch of this entry point is for; use "
+           "pp_find_peaks_field", g.in1, g.in2, g.in3, g.nwords, kNoallocWords);
     char *base = (char *)noalloc_scratch(ctx->device);
     if (!base) {
         set_error("no scratch address for device %d (context creation records it)", ctx->device);
