@@ -190,6 +190,47 @@ bool line_supported(int n)
     return n == 1;
 }
 
+// Roots of unity in Float32 that keep the amplitude on average.  Rounded to the
+// nearest, the few distinct roots of a length (cos 45, cos 30 degrees and their
+// like, both rounded down) shorten every mode by 4 to 6e-8 a transform there and
+// back and axis, a quarter of the whole rounding error and the same in every
+// cell.  Where a table's roots are shorter or longer than 1 in the sum, those
+// components that lose least by it (the ones near half a unit) are rounded the
+// other way until they are not: 1.54 -> 1.47e-7 rms at 480, 1.43 -> 1.37 at 512,
+// 5 to 25 times less of it common to all modes.
+static void append_roots(std::vector<float2> &t, const std::vector<double> &turn)  // exp(-i pi turn)
+{
+    struct Other {
+        double cost, gain;  // added to the squared error; to the table's sum of lengths
+        float *at, to;
+    };
+    const size_t first = t.size();
+    t.resize(first + turn.size());
+    std::vector<Other> other;
+    double sum = 0.0;
+    for (size_t q = 0; q < turn.size(); q++) {
+        const double c[2] = {cos(M_PI * turn[q]), -sin(M_PI * turn[q])};
+        float2 &v = t[first + q];
+        float *const f[2] = {&v.x, &v.y};
+        for (int a = 0; a < 2; a++) {
+            *f[a] = (float)c[a];
+            const double d = (double)*f[a] - c[a];
+            if (d == 0.0 || fabs(c[a]) < 1e-6) continue;
+            const float to = nextafterf(*f[a], d < 0.0 ? 2.f : -2.f);
+            const double e = (double)to - c[a];
+            sum += c[a] * d;
+            other.push_back({e * e - d * d, c[a] * (e - d), f[a], to});
+        }
+    }
+    std::stable_sort(other.begin(), other.end(),
+                     [](const Other &a, const Other &b) { return a.cost * fabs(b.gain) < b.cost * fabs(a.gain); });
+    for (const Other &o : other)
+        if (fabs(sum + o.gain) < fabs(sum)) {
+            sum += o.gain;
+            *o.at = o.to;
+        }
+}
+
 int line_plan(pp_ctx *ctx, int n, LineFft *out)
 {
     PP_ARG(line_supported(n), "line length %d has no line transform", n);
@@ -232,11 +273,9 @@ int line_plan(pp_ctx *ctx, int n, LineFft *out)
         f.mode = !reg ? kLineAny : seven ? kLineReg7 : kLineReg;
         PP_ARG(rad.size() <= 8, "line length %d takes %zu stages", n, rad.size());
         std::vector<float2> t;
-        auto root = [&](double num, double den) {  // exp(-i pi num / den)
-            const double a = M_PI * num / den;
-            t.push_back(make_float2((float)cos(a), (float)-sin(a)));
-        };
-        for (int k = 0; k < n; k++) root(k, n);
+        std::vector<double> turn;
+        for (int k = 0; k < n; k++) turn.push_back((double)k / n);
+        append_roots(t, turn);
         int ns = 1;
         for (size_t q = 0; q < rad.size(); q++) {
             const int R = rad[q];
@@ -247,9 +286,12 @@ int line_plan(pp_ctx *ctx, int n, LineFft *out)
             f.magic[q] = (1u << 22) / (unsigned)ns + 1;
             while (t.size() % 2) t.push_back(float2{});  // 16-byte aligned tables
             f.two[q] = (int)t.size() - n;
-            if (q > 0)
+            if (q > 0) {
+                turn.clear();
                 for (int k = 0; k < ns; k++)
-                    for (int r = 0; r < R; r++) root(2.0 * k * r, (double)ns * R);
+                    for (int r = 0; r < R; r++) turn.push_back(2.0 * k * r / ((double)ns * R));
+                append_roots(t, turn);
+            }
             ns *= R;
         }
         f.nst = (int)rad.size();

@@ -19,8 +19,8 @@
 //   radices are chosen at run time, so one kernel serves every length up to
 //   kLineMax with no larger prime factor).  A stage reads its inputs into
 //   registers, then writes them back in place, so one buffer is enough.
-//   Twiddles come from a table rounded from Float64, laid out as the
-//   butterflies read them.  Vector instructions are the second bound beside
+//   Twiddles come from a table rounded from Float64 (append_roots), laid out as
+//   the butterflies read them.  Vector instructions are the second bound beside
 //   HBM (a radix-8 stage takes 14 per element, a pass has room for about a
 //   hundred), so addresses advance by scalar strides and the kernels' own
 //   Float64 factors are pairs of Float32 numbers (Two), wave numbers whole.

@@ -103,7 +103,7 @@ __device__ __forceinline__ void noise_sincos(double x, double &c, double &s)
 // the two Float64 normals of counter pair `pair`
 //
 // Every kernel that draws them is bound by the issue of these instructions,
-// 223 of them (505 with the general log, cos and sin, whose ranges, signs and
+// 229 of them (505 with the general log, cos and sin, whose ranges, signs and
 // special values a uniform of 53 bits does not need).  Against 113 bits over
 // 10^7 pairs the normals are right to 3.6e-16 of their radius (1.2e-16 rms),
 // where the angle 2 pi u, rounded before its cosine is taken, left 7.3e-16
