@@ -608,10 +608,10 @@ static int make_tile_lines(pp_ctx *ctx, int n, double boxsize, uint64_t seed, co
 }
 
 // Meshes on line transforms.  Odd multiples of 15 stay with rocFFT, which
-// rounds less in them (the density's rms error at 45, 75, 135, 225, 405: 1.84,
-// 2.04, 2.12, 2.25, 2.40e-7 against 2.04, 2.21, 2.39, 2.51, 2.71 on the lines);
-// at the other lengths measured the lines have 0.76 to 1.05 of rocFFT's, all
-// fields together 0.52 to 0.88.
+// rounds less in them (the density's rms error at 45, 75, 135, 225, 375: 1.85,
+// 2.05, 2.12, 2.26, 2.58e-7 against 2.04, 2.22, 2.38, 2.53, 2.67 on the lines);
+// at the 73 other lengths measured between 16 and 512 no field's error on the
+// lines is larger than 0.97 of rocFFT's, all fields together 0.48 to 0.78.
 static bool lines_for(int n) { return line_supported(n) && (n % 2 == 0 || n % 15 != 0); }
 
 }  // namespace pp

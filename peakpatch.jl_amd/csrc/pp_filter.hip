@@ -571,9 +571,9 @@ static int stencil_start(pp_ctx *ctx, const StencilGeom &g, long long *d_counter
 // and every mode, so both give the same bits (the peaks' spectrum is finite: a
 // field with other modes has no peaks).
 // Odd meshes stay with rocFFT, which rounds less in them (rms error at 25, 45,
-// 81, 125, 135: 1.28, 1.22, 1.44, 1.43, 1.39e-7 against 1.36, 1.54, 1.66, 1.69,
-// 1.78 on the lines; even ones, 64, 120, 128: 1.71, 1.73, 1.88 against 1.49,
-// 1.66, 1.68).
+// 81, 125, 135: 1.28, 1.22, 1.44, 1.43, 1.39e-7 against 1.37, 1.55, 1.66, 1.70,
+// 1.78 on the lines; even ones, 64, 120, 128: 1.71, 1.73, 1.88 against 1.42,
+// 1.66, 1.56).
 static bool bank_lines(int n) { return n % 2 == 0 && line_supported(n); }
 
 struct BankGeo {
